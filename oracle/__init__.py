@@ -26,9 +26,9 @@ _I64 = ctypes.c_int64
 
 
 def build(with_ref: bool = True) -> None:
-    """Builds liboracle.so, and oracle/_ref when the reference tree exists."""
+    """Builds liboracle.so, and oracle/_ref when the reference tree holds its sources."""
     subprocess.run(["make", "-s", "-C", str(HERE)], check=True)
-    if with_ref and REFERENCE_TREE.exists():
+    if with_ref and (REFERENCE_TREE / "src" / "Library").is_dir():
         subprocess.run(["make", "-s", "-j8", "-C", str(HERE / "ref"), f"REF={REFERENCE_TREE}"], check=True)
 
 
