@@ -53,6 +53,19 @@ rise_hip_status trace_host(const WideBVH& bvh, int64_t n_tris, int32_t bvh_sourc
 
 }  // namespace
 
+namespace {
+
+// The slots of a node that hold a child (a nonzero meta byte).
+unsigned occupied_slots(const uint4& w1)
+{
+    unsigned m = 0;
+    for (int s = 0; s < 8; ++s)
+        if (byte_of(s < 4 ? w1.z : w1.w, s & 3)) m |= 1u << s;
+    return m;
+}
+
+}  // namespace
+
 extern "C" rise_hip_status rise_hip_debug_node_accept_host(const void* node, const float ray[6], double best,
                                                            uint32_t* accept)
 {
@@ -62,7 +75,7 @@ extern "C" rise_hip_status rise_hip_debug_node_accept_host(const void* node, con
     std::memcpy(w, node, sizeof(w));
     RayState r;
     init_ray(r, ray[0], ray[1], ray[2], ray[3], ray[4], ray[5]);
-    *accept = node_accept_mask(r, w[0], w[1], w[2], w[3], w[4], box_limit(r, best));
+    *accept = node_accept_mask(r, w[0], w[2], w[3], w[4], box_limit(r, best)) & occupied_slots(w[1]);
     return RISE_HIP_OK;
 }
 
@@ -228,7 +241,7 @@ extern "C" rise_hip_status rise_hip_debug_node_accept_obj_host(const void* node,
     const double ow[3] = {ray[0], ray[1], ray[2]}, dw[3] = {ray[3], ray[4], ray[5]};
     ObjRayT<kArithIeee> q;
     init_obj_ray(q, ow, dw, to_object);
-    *accept = node_accept_mask(q, w[0], w[1], w[2], w[3], w[4], box_limit(q, best));
+    *accept = node_accept_mask(q, w[0], w[2], w[3], w[4], box_limit(q, best)) & occupied_slots(w[1]);
     return RISE_HIP_OK;
 }
 

@@ -17,6 +17,11 @@ namespace {
 
 constexpr int kObjBlock = 128;
 
+// Idle lanes at which a wave takes new rays.
+#ifndef RISE_REFILL_OBJ
+#define RISE_REFILL_OBJ 20
+#endif
+
 __device__ inline void load_ray6(const float* __restrict__ rays, int64_t n, int64_t i, float ray[6])
 {
 #pragma unroll
@@ -58,8 +63,8 @@ static_assert(sizeof(ObjectHit) <= sizeof(rise_hip_hit) && alignof(ObjectHit) <=
               "an ObjectHit must fit in a hit record's slot");
 
 // Persistent: the grid is sized to the resident waves, each lane's first ray
-// is assigned statically and later ones are fetched wave-wide (refill) as
-// lanes finish.  REC: stage the ObjectHit in hits[ray] for object_records;
+// is assigned statically and later ones are fetched wave-wide (ItemFetch) as
+// lanes finish; a query that has ended is written out when its wave fetches.  REC: stage the ObjectHit in hits[ray] for object_records;
 // else write prim_id and t (float world range).
 template <int A, bool REC, int STACK>
 __global__ __launch_bounds__(kObjBlock) void closest_objects(ObjectSceneView sc, const float* __restrict__ rays,
@@ -71,20 +76,14 @@ __global__ __launch_bounds__(kObjBlock) void closest_objects(ObjectSceneView sc,
     __shared__ uint2 lds[STACK > 0 ? kObjLds * kObjBlock : 1];
     auto st = make_stack<STACK>(lds);
     ObjClosestQuery<A> Q;
-    long long ray = -1;  // -1 idle, -2 exhausted
-    const int64_t grid_threads = (int64_t)gridDim.x * blockDim.x;
-    for (bool first_pass = true;; first_pass = false) {
-        const long long got = first_pass ? first_item(n) : refill(ray == -1, ray >= 0, next, n, grid_threads);
-        if (ray == -1 && got != -1) {
-            ray = got;
-            if (ray >= 0) {
-                float r6[6];
-                load_ray6(rays, n, ray, r6);
-                objects_closest_begin(sc, r6, faces, st, Q);
-            }
-        }
-        if (__ballot(ray >= 0) == 0ull && __ballot(ray == -1) == 0ull) break;
-        if (ray >= 0 && !objects_closest_step(sc, st, Q)) {
+    ItemFetch fetch(next, n);
+    long long ray = -1;
+    bool busy = false;
+    for (;;) {
+        if (busy) busy = objects_closest_step(sc, st, Q);
+        const unsigned long long bm = __ballot(busy);
+        if (bm != 0ull && !(fetch.more && __popcll(bm) <= 64 - RISE_REFILL_OBJ)) continue;
+        if (!busy && ray >= 0) {
             if (REC) {
                 *reinterpret_cast<ObjectHit*>(hits + ray) = Q.h;
             } else {
@@ -92,6 +91,18 @@ __global__ __launch_bounds__(kObjBlock) void closest_objects(ObjectSceneView sc,
                 t_out[ray] = Q.h.prim_id >= 0 ? (float)Q.h.range : INFINITY;
             }
             ray = -1;
+        }
+        if (fetch.more) {
+            const long long got = fetch.take(busy);
+            if (got >= 0) {
+                float r6[6];
+                load_ray6(rays, n, got, r6);
+                objects_closest_begin(sc, r6, faces, st, Q);
+                ray = got;
+                busy = true;
+            }
+        } else if (bm == 0ull) {
+            break;
         }
     }
 }
@@ -119,22 +130,28 @@ __global__ __launch_bounds__(kObjBlock) void any_objects(ObjectSceneView sc, con
     __shared__ uint2 lds[STACK > 0 ? kObjLds * kObjBlock : 1];
     auto st = make_stack<STACK>(lds);
     ObjAnyQuery<A> Q;
+    ItemFetch fetch(next, n);
     long long ray = -1;
-    const int64_t grid_threads = (int64_t)gridDim.x * blockDim.x;
-    for (bool first_pass = true;; first_pass = false) {
-        const long long got = first_pass ? first_item(n) : refill(ray == -1, ray >= 0, next, n, grid_threads);
-        if (ray == -1 && got != -1) {
-            ray = got;
-            if (ray >= 0) {
-                float r6[6];
-                load_ray6(rays, n, ray, r6);
-                objects_any_begin(sc, r6, tmax ? (double)tmax[ray] : kRiseInfinity, faces, st, Q);
-            }
-        }
-        if (__ballot(ray >= 0) == 0ull && __ballot(ray == -1) == 0ull) break;
-        if (ray >= 0 && !objects_any_step(sc, st, Q)) {
+    bool busy = false;
+    for (;;) {
+        if (busy) busy = objects_any_step(sc, st, Q);
+        const unsigned long long bm = __ballot(busy);
+        if (bm != 0ull && !(fetch.more && __popcll(bm) <= 64 - RISE_REFILL_OBJ)) continue;
+        if (!busy && ray >= 0) {
             occluded[ray] = Q.hit ? 1 : 0;
             ray = -1;
+        }
+        if (fetch.more) {
+            const long long got = fetch.take(busy);
+            if (got >= 0) {
+                float r6[6];
+                load_ray6(rays, n, got, r6);
+                objects_any_begin(sc, r6, tmax ? (double)tmax[got] : kRiseInfinity, faces, st, Q);
+                ray = got;
+                busy = true;
+            }
+        } else if (bm == 0ull) {
+            break;
         }
     }
 }

@@ -119,19 +119,16 @@ struct ObjLdsStack {
 // The top-level walk's state: the node group being tested and the leaves of
 // the last node tested.
 struct TopWalk {
-    unsigned gbase, ghits, gimask;
-    unsigned tbase, tmask;
+    NodeGroup g;
+    LeafWalk leaves;
     float tlim;  // box limit along the scaled world direction
 };
 
 template <int A>
 RISE_HD inline void top_begin(const RayStateT<A>& r, float tlim, TopWalk& w)
 {
-    w.gbase = 0;
-    w.ghits = 1u << (0u ^ r.oinv);  // the root, in slot 0 of a virtual group
-    w.gimask = 1u;
-    w.tbase = 0;
-    w.tmask = 0;
+    w.g = root_group(r);
+    w.leaves = LeafWalk{0u, 0u, 0u, 0u};
     w.tlim = tlim;
 }
 
@@ -144,28 +141,13 @@ template <int A, class Stack>
 RISE_HD inline int top_step(const RayStateT<A>& r, const NodeSlot* __restrict__ nodes,
                             const Tri48* __restrict__ leaves, Stack& st, TopWalk& w)
 {
-    if (w.tmask) {
-        const unsigned j = __builtin_ctz(w.tmask);
-        w.tmask &= w.tmask - 1u;
-        return (int)float_to_bits(leaves[w.tbase + j].v0[3]);
+    if (w.leaves.slots) {
+        unsigned leaf;
+        return next_triangle(w.leaves, leaf) ? (int)float_to_bits(leaves[leaf].v0[3]) : -1;
     }
-    if (w.ghits) {
-        const unsigned k = __builtin_ctz(w.ghits);
-        w.ghits &= w.ghits - 1u;
-        const unsigned slot = k ^ r.oinv;
-        const unsigned ni = w.gbase + __builtin_popcount(w.gimask & ((1u << slot) - 1u));
-        if (w.ghits) st.push(make_uint2(w.gbase, w.ghits | (w.gimask << 8)));
-        unsigned cb, im;
-        w.ghits = test_node(r, nodes, ni, w.tlim, cb, im, w.tbase, w.tmask);
-        w.gbase = cb;
-        w.gimask = im;
-        return -1;
-    }
-    if (st.empty()) return -2;
-    const uint2 g = st.pop();
-    w.gbase = g.x;
-    w.ghits = g.y & 0xffu;
-    w.gimask = (g.y >> 8) & 0xffu;
+    if (!next_group(st, w.g)) return -2;
+    unsigned nn = 0;
+    visit_node<false>(r, nodes, st, w.g, w.tlim, w.leaves, nn);
     return -1;
 }
 

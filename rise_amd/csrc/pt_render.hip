@@ -376,42 +376,26 @@ __global__ __launch_bounds__(BLOCK) void k_extend(const ReqInfo* __restrict__ re
         }
         return;
     }
-    unsigned long long* next = S.fetch + depth;
-    RayState r;
-    ClosestState s;
+    auto st = make_stack<STACK>(lds, BLOCK);
     const NodeSlot* nodes = nullptr;
     const Tri48* tris = nullptr;
     unsigned slot = 0, nn = 0, nt = 0;  // slot: lane * cap + path slot of the current item
-    long long item = -1;  // -1 idle, -2 exhausted
-    const int64_t grid_threads = (int64_t)gridDim.x * blockDim.x;
-    for (bool first_pass = true;; first_pass = false) {
-        // The first item of every thread is assigned statically; later ones come from the counter.
-        const long long got = first_pass ? first_item(n) : refill(item == -1, item >= 0, next, n, grid_threads);
-        if (item == -1 && got != -1) {
-            item = got;
-            if (item >= 0) {
-                const unsigned code = q[item];
-                slot = (code & 3u) * (unsigned)S.cap + (code >> 2);
-                const ReqInfo& R = reqs[S.req[code >> 2]];
-                nodes = R.sc.nodes;
-                tris = R.sc.tris;
-                init_ray(r, S.ox[slot], S.oy[slot], S.oz[slot], S.dx[slot], S.dy[slot], S.dz[slot]);
-                closest_begin(r, s);
-                lst.sp = 0;
-                pst.sp = 0;
-            }
-        }
-        if (__ballot(item >= 0) == 0ull && __ballot(item == -1) == 0ull) break;
-        if (item >= 0) {
-            const bool more = STACK > 0 ? closest_step<false>(r, nodes, tris, lst, s, nn, nt)
-                                        : closest_step<false>(r, nodes, tris, pst, s, nn, nt);
-            if (!more) {
-                S.hit_leaf[slot] = s.best_id >= 0 ? s.best_leaf : 0xffffffffu;
-                S.hit_t[slot] = s.best_id >= 0 ? (float)s.best_t : 0.0f;
-                item = -1;
-            }
-        }
-    }
+    persist_closest<false, false, false, RayState>(
+        st, n, S.fetch + depth, nn, nt, nodes, tris, nullptr,
+        [&](int64_t item, RayState& r, ClosestState& s) {
+            const unsigned code = q[item];
+            slot = (code & 3u) * (unsigned)S.cap + (code >> 2);
+            const ReqInfo& R = reqs[S.req[code >> 2]];
+            nodes = R.sc.nodes;
+            tris = R.sc.tris;
+            init_ray(r, S.ox[slot], S.oy[slot], S.oz[slot], S.dx[slot], S.dy[slot], S.dz[slot]);
+            closest_begin(r, s);
+            return true;
+        },
+        [&](int64_t, const RayState&, const ClosestState& s) {
+            S.hit_leaf[slot] = s.best_id >= 0 ? s.best_leaf : 0xffffffffu;
+            S.hit_t[slot] = s.best_id >= 0 ? (float)s.best_t : 0.0f;
+        });
 }
 
 // ---- materials at one wavelength ------------------------------------------------
@@ -1535,47 +1519,28 @@ __global__ __launch_bounds__(BLOCK, kConnectWaves) void k_connect(const ReqInfo*
         }
         return;
     }
-    unsigned long long* next = S.fetch + (kMaxPathDepth + 1) + depth;
-    RayState r;
-    AnyState s;
+    auto st = make_stack<STACK>(lds, BLOCK);
     const NodeSlot* nodes = nullptr;
     const Tri48* tris = nullptr;
     bool media = false;
     unsigned nn = 0, nt = 0;
-    long long item = -1;
-    const int64_t grid_threads = (int64_t)gridDim.x * blockDim.x;
-    for (bool first_pass = true;; first_pass = false) {
-        // The first item of every thread is assigned statically; later ones come from the counter.
-        const long long got = first_pass ? first_item(n) : refill(item == -1, item >= 0, next, n, grid_threads);
-        if (item == -1 && got != -1) {
-            item = got;
-            if (item >= 0 && S.sinfo && (S.sinfo[item] & kShadowInScatter)) {
-                item = -1;  // no occlusion test; the walk adds it
-            } else if (item >= 0) {
-                const unsigned slot = (S.sslot[item] & kRecSlotMask) >> 2;
-                const ReqInfo& R = reqs[S.req[slot]];
-                nodes = R.sc.nodes;
-                tris = R.sc.tris;
-                media = R.sc.has_media;
-                init_ray(r, S.sox[item], S.soy[item], S.soz[item], S.sdx[item], S.sdy[item], S.sdz[item]);
-                any_begin(r, scale_how_far(r, (double)(S.stmax[item] - 0.001f)), s);
-                lst.sp = 0;
-                pst.sp = 0;
-            }
-        }
-        if (__ballot(item >= 0) == 0ull && __ballot(item == -1) == 0ull) break;
-        if (item >= 0) {
-            const bool more = STACK > 0 ? any_step<false>(r, nodes, tris, lst, s, nn, nt)
-                                        : any_step<false>(r, nodes, tris, pst, s, nn, nt);
-            if (!more) {
-                if (!s.hit) {
-                    if (media) S.svis[item] = 1u;
-                    else add_shadow(S, S.sslot[item], S.sval[item], 1.0f);
-                }
-                item = -1;
-            }
-        }
-    }
+    persist_any<false, false, false, RayState>(
+        st, n, S.fetch + (kMaxPathDepth + 1) + depth, nn, nt, nodes, tris, nullptr,
+        [&](int64_t item, RayState& r, AnyState& s) {
+            if (S.sinfo && (S.sinfo[item] & kShadowInScatter)) return false;  // no occlusion test; the walk adds it
+            const ReqInfo& R = reqs[S.req[(S.sslot[item] & kRecSlotMask) >> 2]];
+            nodes = R.sc.nodes;
+            tris = R.sc.tris;
+            media = R.sc.has_media;
+            init_ray(r, S.sox[item], S.soy[item], S.soz[item], S.sdx[item], S.sdy[item], S.sdz[item]);
+            any_begin(r, scale_how_far(r, (double)(S.stmax[item] - 0.001f)), s);
+            return true;
+        },
+        [&](int64_t item, const AnyState& s) {
+            if (s.hit) return;
+            if (media) S.svis[item] = 1u;
+            else add_shadow(S, S.sslot[item], S.sval[item], 1.0f);
+        });
 }
 
 // Kernel tables over the traversal variants: stack (LDS 8, LDS 16, private),

@@ -113,9 +113,9 @@ struct RayStateT {
     float fx, fy, fz;      // (float)dn: the filter's direction (BVH.h:1212-1225)
     float ix, iy, iz;      // slab inverses 1/(d 2^k) (kInvClamp for tiny components)
     unsigned oinv;         // (~octant) & 7
+    float inv_len;         // 1 / (|d| 2^k): t along the scaled direction = distance * inv_len
     double ov;             // Normalize's 1/|d|
     double len_d;          // |d| in double
-    double len_s;          // |d| 2^k: t along the scaled direction = distance / len_s
 };
 using RayState = RayStateT<kArithIeee>;
 
@@ -177,7 +177,7 @@ RISE_HD inline void init_ray(RayStateT<A>& r, float ox, float oy, float oz, floa
     const double mag = sqrt(dot3<A>(d[0], d[0], d[1], d[1], d[2], d[2]));
     r.ov = mag > 0.0 ? 1.0 / mag : 1.0;
     r.len_d = mag;
-    r.len_s = mag > 0.0 ? ldexp(mag, sh) : 1.0;
+    r.inv_len = mag > 0.0 ? (float)ldexp(r.ov, -sh) : 1.0f;
     r.fx = (float)dn0(r);
     r.fy = (float)dn1(r);
     r.fz = (float)dn2(r);
@@ -225,7 +225,7 @@ struct ObjRayT {
     unsigned oinv;     // (~octant of (float)dn') & 7
     double o[3];       // o'
     double dn[3];      // dn'
-    double len_s;      // |(float)dn'| 2^k: t along the scaled direction = distance / len_s
+    float inv_len;     // 1 / (|(float)dn'| 2^k): t along the scaled direction = distance * inv_len
     double mag;        // |dl|
     double factor;     // |dl|, or 1 when |dl| <= NEARZERO
 };
@@ -271,7 +271,7 @@ RISE_HD inline void init_obj_ray(ObjRayT<A>& r, const double ow[3], const double
     r.oinv = (~oct) & 7u;
     const double f[3] = {r.fx, r.fy, r.fz};
     const double lf = sqrt(f[0] * f[0] + f[1] * f[1] + f[2] * f[2]);
-    r.len_s = lf > 0.0 ? ldexp(lf, sh) : 1.0;
+    r.inv_len = lf > 0.0 ? (float)(1.0 / ldexp(lf, sh)) : 1.0f;
     r.ex = (float)(fabs(r.o[0] - (double)r.ox) * fabs((double)r.ix) * (1.0 + 0x1p-20));
     r.ey = (float)(fabs(r.o[1] - (double)r.oy) * fabs((double)r.iy) * (1.0 + 0x1p-20));
     r.ez = (float)(fabs(r.o[2] - (double)r.oz) * fabs((double)r.iz) * (1.0 + 0x1p-20));
@@ -443,13 +443,16 @@ RISE_HD inline unsigned byte_of(unsigned w, int k) { return (w >> (8 * k)) & 0xf
 // 2.0001 * 2^-24 |b| besides its relative error (2.0001 * 2^-24 |t|): the
 // near plane subtracts, the far plane adds, 2^-21 |b| + 2^-100 (which also
 // covers flushed subnormals), leaving only the relative error for
-// RISE_SLAB_PAD.  Should b or s be too large for q s + b to stay finite
+// RISE_SLAB_PAD.  That factor is folded into the far planes, sf = s PAD and
+// bf = (b + slack) PAD, so no slot multiplies by it: rounding the two apart
+// adds at most 2^-24 (|t| + 2 |b|), inside the slack's 2^-21 |b| and the
+// factor's 2^-19 |t|.  Should b or s be too large for q s + b to stay finite
 // (|b| < 2^126 and |s| < 2^119 keep 255 |s| + |b| (1 + 2^-21) below 2^128),
 // the axis constrains nothing (s = 0, planes at -inf / +inf): still
 // conservative.  With the 2^80 inverse of a zero direction component that
 // happens only for nodes 2^46 away or 2^39 wide.
 struct SlabAxis {
-    float s, bn, bf;
+    float s, sf, bn, bf;
 };
 
 RISE_HD inline SlabAxis slab_axis(float p, int e, float o, float inv)
@@ -457,8 +460,9 @@ RISE_HD inline SlabAxis slab_axis(float p, int e, float o, float inv)
     const float b = (p - o) * inv;
     const float s = ldexpf(inv, e);
     const float slack = fmaf(fabsf(b), 0x1p-21f, 0x1p-100f);
-    if (fabsf(b) < 0x1p126f && fabsf(s) < 0x1p119f) return SlabAxis{s, b - slack, b + slack};
-    return SlabAxis{0.0f, -INFINITY, INFINITY};
+    if (fabsf(b) < 0x1p126f && fabsf(s) < 0x1p119f)
+        return SlabAxis{s, s * RISE_SLAB_PAD, b - slack, (b + slack) * RISE_SLAB_PAD};
+    return SlabAxis{0.0f, 0.0f, -INFINITY, INFINITY};
 }
 
 // slab_axis for an origin known only to within `extra / |inv|` of o: the
@@ -469,18 +473,21 @@ RISE_HD inline SlabAxis slab_axis_widened(float p, int e, float o, float inv, fl
     const float b = (p - o) * inv;
     const float s = ldexpf(inv, e);
     const float slack = fmaf(fabsf(b), 0x1p-21f, 0x1p-100f) + extra * (1.0f + 0x1p-22f);
-    if (fabsf(b) < 0x1p126f && fabsf(s) < 0x1p119f && extra < 0x1p125f) return SlabAxis{s, b - slack, b + slack};
-    return SlabAxis{0.0f, -INFINITY, INFINITY};
+    if (fabsf(b) < 0x1p126f && fabsf(s) < 0x1p119f && extra < 0x1p125f)
+        return SlabAxis{s, s * RISE_SLAB_PAD, b - slack, (b + slack) * RISE_SLAB_PAD};
+    return SlabAxis{0.0f, 0.0f, -INFINITY, INFINITY};
 }
 
 // The eight child boxes of one node against the axes' plane distances: bit s
-// of the result set when slot s is occupied and its box meets [0, tmax]
-// (conservatively).  The quantized planes are split by the sign of the
-// inverse into near and far words per axis, so each slot costs six byte
-// conversions, six FMAs and the interval reductions.
+// of the result set when slot s's box meets [0, tmax] (conservatively).  The
+// quantized planes are split by the sign of the inverse into near and far
+// words per axis, so each slot costs six byte conversions, six FMAs, the
+// interval reductions, one comparison and one add-with-carry that appends its
+// bit.  An empty slot's box is inverted (low 255, high 0), so it is met only
+// where an axis constrains nothing; the leaf walk skips it (count 0).
+// `pad_limit` is tmax times RISE_SLAB_PAD (box_limit), as the far planes are.
 RISE_HD inline unsigned accept_slots(const SlabAxis& ax, const SlabAxis& ay, const SlabAxis& az, bool nx, bool ny,
-                                     bool nz, const uint4& w1, const uint4& w2, const uint4& w3, const uint4& w4,
-                                     float tmax)
+                                     bool nz, const uint4& w2, const uint4& w3, const uint4& w4, float pad_limit)
 {
     // Low planes: qlox = w2.x|y, qloy = w2.z|w, qloz = w3.x|y; high planes:
     // qhix = w3.z|w, qhiy = w4.x|y, qhiz = w4.z|w (slots 0-3 | 4-7).  With a
@@ -493,84 +500,109 @@ RISE_HD inline unsigned accept_slots(const SlabAxis& ax, const SlabAxis& ay, con
     const unsigned fz0 = nz ? w3.x : w4.z, fz1 = nz ? w3.y : w4.w;
     unsigned acc = 0;
 #pragma unroll
-    for (int s = 0; s < 8; ++s) {
+    for (int s = 7; s >= 0; --s) {
         const int k = s & 3;
         const bool hi4 = s >= 4;
-        const unsigned meta = byte_of(s < 4 ? w1.z : w1.w, s & 3);
         const float tnx = fmaf((float)byte_of(hi4 ? nx1 : nx0, k), ax.s, ax.bn);
         const float tny = fmaf((float)byte_of(hi4 ? ny1 : ny0, k), ay.s, ay.bn);
         const float tnz = fmaf((float)byte_of(hi4 ? nz1 : nz0, k), az.s, az.bn);
-        const float tfx = fmaf((float)byte_of(hi4 ? fx1 : fx0, k), ax.s, ax.bf);
-        const float tfy = fmaf((float)byte_of(hi4 ? fy1 : fy0, k), ay.s, ay.bf);
-        const float tfz = fmaf((float)byte_of(hi4 ? fz1 : fz0, k), az.s, az.bf);
+        const float tfx = fmaf((float)byte_of(hi4 ? fx1 : fx0, k), ax.sf, ax.bf);
+        const float tfy = fmaf((float)byte_of(hi4 ? fy1 : fy0, k), ay.sf, ay.bf);
+        const float tfz = fmaf((float)byte_of(hi4 ? fz1 : fz0, k), az.sf, az.bf);
         const float tn = fmaxf(fmaxf(tnx, tny), fmaxf(tnz, 0.0f));
-        const float tf = fminf(fminf(tfx, tfy), fminf(tfz, tmax));
-        if ((meta != 0) && (tn <= tf * RISE_SLAB_PAD)) acc |= 1u << s;
+        const float tf = fminf(fminf(tfx, tfy), fminf(tfz, pad_limit));
+        acc = acc + acc + (tn <= tf ? 1u : 0u);
     }
     return acc;
 }
 
 template <int A>
-RISE_HD inline unsigned node_accept_mask(const RayStateT<A>& r, const uint4& w0, const uint4& w1, const uint4& w2,
-                                         const uint4& w3, const uint4& w4, float tmax)
+RISE_HD inline unsigned node_accept_mask(const RayStateT<A>& r, const uint4& w0, const uint4& w2, const uint4& w3,
+                                         const uint4& w4, float pad_limit)
 {
     const SlabAxis ax = slab_axis(bits_to_float(w0.x), (int)(signed char)(w0.w & 0xff), r.ox, r.ix);
     const SlabAxis ay = slab_axis(bits_to_float(w0.y), (int)(signed char)((w0.w >> 8) & 0xff), r.oy, r.iy);
     const SlabAxis az = slab_axis(bits_to_float(w0.z), (int)(signed char)((w0.w >> 16) & 0xff), r.oz, r.iz);
-    return accept_slots(ax, ay, az, r.ix < 0.0f, r.iy < 0.0f, r.iz < 0.0f, w1, w2, w3, w4, tmax);
+    return accept_slots(ax, ay, az, r.ix < 0.0f, r.iy < 0.0f, r.iz < 0.0f, w2, w3, w4, pad_limit);
 }
 
 // The same for an object-space ray: the float ray's planes widened by the
 // origin's rounding (ObjRayT).
 template <int A>
-RISE_HD inline unsigned node_accept_mask(const ObjRayT<A>& r, const uint4& w0, const uint4& w1, const uint4& w2,
-                                         const uint4& w3, const uint4& w4, float tmax)
+RISE_HD inline unsigned node_accept_mask(const ObjRayT<A>& r, const uint4& w0, const uint4& w2, const uint4& w3,
+                                         const uint4& w4, float pad_limit)
 {
     const SlabAxis ax = slab_axis_widened(bits_to_float(w0.x), (int)(signed char)(w0.w & 0xff), r.ox, r.ix, r.ex);
     const SlabAxis ay =
         slab_axis_widened(bits_to_float(w0.y), (int)(signed char)((w0.w >> 8) & 0xff), r.oy, r.iy, r.ey);
     const SlabAxis az =
         slab_axis_widened(bits_to_float(w0.z), (int)(signed char)((w0.w >> 16) & 0xff), r.oz, r.iz, r.ez);
-    return accept_slots(ax, ay, az, r.ix < 0.0f, r.iy < 0.0f, r.iz < 0.0f, w1, w2, w3, w4, tmax);
+    return accept_slots(ax, ay, az, r.ix < 0.0f, r.iy < 0.0f, r.iz < 0.0f, w2, w3, w4, pad_limit);
+}
+
+// Bit s of the 8-bit mask x moved to bit s ^ o (0 <= o < 8): the exchanges of
+// neighbouring bits, pairs and nibbles that the bits of o select.
+RISE_HD inline unsigned xor_permute8(unsigned x, unsigned o)
+{
+    const unsigned x1 = ((x & 0x55u) << 1) | ((x >> 1) & 0x55u);
+    x = (o & 1u) ? x1 : x;
+    const unsigned x2 = ((x & 0x33u) << 2) | ((x >> 2) & 0x33u);
+    x = (o & 2u) ? x2 : x;
+    const unsigned x4 = ((x & 0x0fu) << 4) | (x >> 4);
+    return (o & 4u) ? x4 : x;
+}
+
+// The triangles of a tested node's accepted leaf slots, walked one by one: the
+// slots still to do, the node's meta bytes (a leaf: count << 5 | offset) and
+// its triangle base.
+struct LeafWalk {
+    unsigned slots, m0, m1, base;
+};
+
+// The next triangle (leaf-order index) of w; false for an empty slot.  A
+// leaf of several triangles stays in the mask with its first one taken off
+// its meta byte (one fewer, the offset one further: 31 less).
+RISE_HD inline bool next_triangle(LeafWalk& w, unsigned& leaf)
+{
+    const unsigned s = __builtin_ctz(w.slots), sh = 8u * (s & 3u);
+    const unsigned meta = ((s & 4u) ? w.m1 : w.m0) >> sh;
+    const unsigned cnt = (meta >> 5) & 7u;
+    leaf = w.base + (meta & 31u);
+    if (cnt <= 1u) {
+        w.slots &= w.slots - 1u;
+    } else if (s & 4u) {
+        w.m1 -= 31u << sh;
+    } else {
+        w.m0 -= 31u << sh;
+    }
+    return cnt != 0u;
 }
 
 // Tests the eight children of one node.  Returns the permuted internal-hit
-// mask (bit k <-> slot k ^ oinv) and fills the node's leaf-triangle mask.
+// mask (bit k <-> slot k ^ oinv) and the walk over the accepted leaves.
 template <class R>
-RISE_HD inline unsigned test_node(const R& r, const NodeSlot* __restrict__ nodes, unsigned ni, float tmax,
-                                     unsigned& child_base, unsigned& imask, unsigned& tri_base, unsigned& tmask)
+RISE_HD inline unsigned test_node(const R& r, const NodeSlot* __restrict__ nodes, unsigned ni, float pad_limit,
+                                  unsigned& child_base, unsigned& imask, LeafWalk& w)
 {
     const uint4* p = reinterpret_cast<const uint4*>(nodes + ni);
     const uint4 w0 = p[0], w1 = p[1], w2 = p[2], w3 = p[3], w4 = p[4];
     imask = (w0.w >> 24) & 0xffu;
     child_base = w1.x;
-    tri_base = w1.y;
-    const unsigned acc = node_accept_mask(r, w0, w1, w2, w3, w4, tmax);
-    unsigned hits = 0;
-    tmask = 0;
-#pragma unroll
-    for (int s = 0; s < 8; ++s) {
-        if ((acc >> s) & 1u) {
-            if ((imask >> s) & 1u) {
-                hits |= 1u << (s ^ r.oinv);
-            } else {
-                const unsigned meta = byte_of(s < 4 ? w1.z : w1.w, s & 3);
-                const unsigned cnt = meta >> 5, off = meta & 31u;
-                tmask |= ((1u << cnt) - 1u) << off;
-            }
-        }
-    }
-    return hits;
+    const unsigned acc = node_accept_mask(r, w0, w2, w3, w4, pad_limit);
+    w = LeafWalk{acc & ~imask, w1.z, w1.w, w1.y};
+    return xor_permute8(acc & imask, r.oinv);
 }
 
 // Converts a best distance along dn into the float traversal parameter along
-// the scaled direction, widened (RISE_SLAB_PAD); kRiseInfinity maps to +inf.
+// the scaled direction, widened twice by RISE_SLAB_PAD: once for its own
+// rounding (the conversions here and inv_len are good to 2^-22), once because
+// it is compared with the far planes, which carry the factor (slab_axis);
+// kRiseInfinity maps to +inf.
 template <int A>
 RISE_HD inline float box_limit(const RayStateT<A>& r, double best)
 {
     if (!(best < kRiseInfinity)) return INFINITY;
-    const double s = best / r.len_s;
-    return (float)s * RISE_SLAB_PAD;
+    return (float)best * r.inv_len * (RISE_SLAB_PAD * RISE_SLAB_PAD);
 }
 
 // box_limit for an object-space ray: its slab test runs along the scaled
@@ -580,8 +612,7 @@ template <int A>
 RISE_HD inline float box_limit(const ObjRayT<A>& r, double best)
 {
     if (!(best < kRiseInfinity)) return INFINITY;
-    const double s = best / r.len_s;
-    return (float)s * RISE_SLAB_PAD;
+    return (float)best * r.inv_len * (RISE_SLAB_PAD * RISE_SLAB_PAD);
 }
 
 template <int STACK>
@@ -602,13 +633,80 @@ struct PrivStack {
     RISE_HD inline bool empty() const { return sp == 0; }
 };
 
-// Traversal state of one closest-hit query: the current node group (base,
-// 8-bit hit mask permuted by the ray octant, 8-bit internal mask), the best
-// certified hit and the box limit derived from it.
+// The node group a traversal stands at: base, 8-bit hit mask permuted by the
+// ray octant, 8-bit internal mask.
+struct NodeGroup {
+    unsigned base, hits, imask;
+};
+
+template <class R>
+RISE_HD inline NodeGroup root_group(const R& r)
+{
+    return NodeGroup{0u, 1u << (0u ^ r.oinv), 1u};  // the root, in slot 0 of a virtual group
+}
+
+// Visits the next node of the group (near-to-far by octant): pushes what is
+// left of the group, tests the node, and makes its accepted internal children
+// the group.  w receives its accepted leaves.
+template <bool COUNT, class Stack, class R>
+RISE_HD inline void visit_node(const R& r, const NodeSlot* __restrict__ nodes, Stack& st, NodeGroup& g,
+                               float pad_limit, LeafWalk& w, unsigned& n_nodes)
+{
+    const unsigned k = __builtin_ctz(g.hits);
+    g.hits &= g.hits - 1u;
+    const unsigned slot = k ^ r.oinv;
+    const unsigned ni = g.base + __builtin_popcount(g.imask & ((1u << slot) - 1u));
+    if (g.hits) st.push(make_uint2(g.base, g.hits | (g.imask << 8)));
+    if (COUNT) ++n_nodes;
+    unsigned cb, im;
+    g.hits = test_node(r, nodes, ni, pad_limit, cb, im, w);
+    g.base = cb;
+    g.imask = im;
+}
+
+// Pops the next group when this one is used up; false once none is left.
+template <class Stack>
+RISE_HD inline bool next_group(Stack& st, NodeGroup& g)
+{
+    if (g.hits) return true;
+    if (st.empty()) return false;
+    const uint2 e = st.pop();
+    g = NodeGroup{e.x, e.y & 0xffu, (e.y >> 8) & 0xffu};
+    return true;
+}
+
+// Face selection and the float pre-filter on one leaf triangle.  ANY: a
+// triangle that casts no shadow (bit 0 of v2.w) never passes
+// (ObjectManager.cpp:119-124).
+// CULL: apply the face selection `faces` (face_ok) before the filter.
+// F64: the triangles' double vertices are in tri64 (9 doubles per leaf
+// record, leaf order) and the certifier and face test use them.
+template <bool CULL, bool F64, bool ANY, class R>
+RISE_HD inline bool passes_filter(const R& r, const Tri48* __restrict__ tris, const double* __restrict__ tri64,
+                                  unsigned leaf, unsigned faces, float best)
+{
+    const float4* tp = reinterpret_cast<const float4*>(tris + leaf);
+    const float4 a = tp[0], b = tp[1], c = tp[2];
+    if (CULL && faces != 3u && !(float_to_bits(c.w) & kTriDoubleSided) &&
+        !(F64 ? face_ok64(r, tri64 + 9 * (size_t)leaf, faces) : face_ok(r, a, b, c, faces)))
+        return false;
+    return filter_float(r, a, b, c, best) && !(ANY && (float_to_bits(c.w) & 1));
+}
+
+// A candidate that the filter has passed is certified later (below): the
+// certifier is some hundred double operations that one lane in thirty needs
+// per step, so running it at once costs a whole wave those instructions at
+// nearly every step.
+constexpr unsigned kNoLeaf = 0xffffffffu;
+
+// Traversal state of one closest-hit query: the current node group, the best
+// certified hit, the box limit derived from it and the candidate awaiting the
+// certifier.
 struct ClosestState {
-    unsigned gbase, ghits, gimask;
+    NodeGroup g;
     unsigned best_leaf;
     int best_id;
+    unsigned pend;   // leaf-order index of the candidate, kNoLeaf: none
     float tlim;
     double best_t;
     unsigned faces;  // face selection (face_ok), read by the culling variant only
@@ -617,71 +715,87 @@ struct ClosestState {
 template <class R>
 RISE_HD inline void closest_begin(const R& r, ClosestState& s)
 {
-    s.gbase = 0;
-    s.ghits = 1u << (0u ^ r.oinv);  // the root, in slot 0 of a virtual group
-    s.gimask = 1u;
-    s.best_leaf = 0xffffffffu;
+    s.g = root_group(r);
+    s.best_leaf = kNoLeaf;
     s.best_id = -1;
+    s.pend = kNoLeaf;
     s.tlim = INFINITY;
     s.best_t = kRiseInfinity;
     s.faces = 3u;
 }
 
-// One traversal step: visit the next node of the current group (near-to-far
-// by octant) and certify the triangles of its leaf children; when the group
-// is used up, pop the next one.  Returns false once the traversal is over.
-// Closest hit: smallest t, exact ties to the lowest caller id (the
-// reference's strict-closer guard, ...Specializations.h:172, plus the tie rule).
-// CULL: apply the face selection in s.faces (face_ok) before the filter.
-// F64: the triangles' double vertices are in tri64 (9 doubles per leaf
-// record, leaf order) and the certifier and face test use them.
-template <bool COUNT, bool CULL = false, bool F64 = false, class Stack, class R>
-RISE_HD inline bool closest_step(const R& r, const NodeSlot* __restrict__ nodes,
-                                 const Tri48* __restrict__ tris, Stack& st, ClosestState& s, unsigned& n_nodes,
-                                 unsigned& n_tris, const double* __restrict__ tri64 = nullptr)
+// A copy of the ray's 1/|d| that the compiler takes for a new value, so that
+// the certifier's double direction is computed where it is needed and not
+// hoisted in front of the leaf loop, which every step passes.
+RISE_HD inline void keep_late(double& x)
 {
-    unsigned tmask = 0, tbase = 0;
-    if (s.ghits) {
-        const unsigned k = __builtin_ctz(s.ghits);
-        s.ghits &= s.ghits - 1u;
-        const unsigned slot = k ^ r.oinv;
-        const unsigned ni = s.gbase + __builtin_popcount(s.gimask & ((1u << slot) - 1u));
-        if (s.ghits) st.push(make_uint2(s.gbase, s.ghits | (s.gimask << 8)));
-        if (COUNT) ++n_nodes;
-        unsigned cb, im;
-        s.ghits = test_node(r, nodes, ni, s.tlim, cb, im, tbase, tmask);
-        s.gbase = cb;
-        s.gimask = im;
-    }
-    while (tmask) {
-        const unsigned j = __builtin_ctz(tmask);
-        tmask &= tmask - 1u;
-        const float4* tp = reinterpret_cast<const float4*>(tris + tbase + j);
-        const float4 a = tp[0], b = tp[1], c = tp[2];
-        if (COUNT) ++n_tris;
-        const double* v64 = F64 ? tri64 + 9 * (size_t)(tbase + j) : nullptr;
-        if (CULL && s.faces != 3u && !(float_to_bits(c.w) & kTriDoubleSided) &&
-            !(F64 ? face_ok64(r, v64, s.faces) : face_ok(r, a, b, c, s.faces)))
-            continue;
-        double tt;
-        if (filter_float(r, a, b, c, (float)s.best_t) && (F64 ? certify64(r, v64, tt) : certify(r, a, b, c, tt))) {
-            const int id = float_to_bits(a.w);
-            if (tt < s.best_t || (tt == s.best_t && id < s.best_id)) {
-                s.best_t = tt;
-                s.best_id = id;
-                s.best_leaf = tbase + j;
-                s.tlim = box_limit(r, s.best_t);
-            }
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" : "+v"(x));
+#else
+    (void)x;
+#endif
+}
+template <int A>
+RISE_HD inline RayStateT<A> late_ray(const RayStateT<A>& r)
+{
+    RayStateT<A> q = r;
+    keep_late(q.ov);
+    return q;
+}
+template <int A>
+RISE_HD inline const ObjRayT<A>& late_ray(const ObjRayT<A>& r) { return r; }
+
+// Certifies the awaiting candidate and keeps it if it is the closest so far:
+// smallest t, exact ties to the lowest caller id (the reference's
+// strict-closer guard, ...Specializations.h:172, plus the tie rule).
+template <bool F64, class R>
+RISE_HD inline void closest_commit(const R& r, const Tri48* __restrict__ tris, const double* __restrict__ tri64,
+                                   ClosestState& s)
+{
+    const float4* tp = reinterpret_cast<const float4*>(tris + s.pend);
+    const float4 a = tp[0], b = tp[1], c = tp[2];
+    double tt;
+    const auto& q = late_ray(r);
+    if (F64 ? certify64(q, tri64 + 9 * (size_t)s.pend, tt) : certify(q, a, b, c, tt)) {
+        const int id = float_to_bits(a.w);
+        if (tt < s.best_t || (tt == s.best_t && id < s.best_id)) {
+            s.best_t = tt;
+            s.best_id = id;
+            s.best_leaf = s.pend;
+            s.tlim = box_limit(r, s.best_t);
         }
     }
-    if (!s.ghits) {
-        if (st.empty()) return false;
-        const uint2 g = st.pop();
-        s.gbase = g.x;
-        s.ghits = g.y & 0xffu;
-        s.gimask = (g.y >> 8) & 0xffu;
+    s.pend = kNoLeaf;
+}
+
+// One traversal step: visit the next node and filter the triangles of its
+// leaf children; when the group is used up, pop the next one.  Returns false
+// once the traversal is over (a candidate may still be awaiting
+// closest_commit).  DEFER: a candidate waits for the caller's closest_commit,
+// or for the next candidate; else it is certified at once.  Waiting leaves the
+// box limit and the filter's range at the hit certified before, which visits
+// a few more nodes and changes no result: the certifier decides every hit.
+template <bool COUNT, bool CULL = false, bool F64 = false, bool DEFER = false, class Stack, class R>
+RISE_HD inline bool closest_step(const R& r, const NodeSlot* __restrict__ nodes, const Tri48* __restrict__ tris,
+                                 Stack& st, ClosestState& s, unsigned& n_nodes, unsigned& n_tris,
+                                 const double* __restrict__ tri64 = nullptr)
+{
+    LeafWalk w;
+    visit_node<COUNT>(r, nodes, st, s.g, s.tlim, w, n_nodes);
+    while (w.slots) {
+        unsigned leaf;
+        if (!next_triangle(w, leaf)) continue;
+        if (COUNT) ++n_tris;
+        if (!passes_filter<CULL, F64, false>(r, tris, tri64, leaf, s.faces, (float)s.best_t)) continue;
+        if (DEFER) {
+            if (s.pend != kNoLeaf) closest_commit<F64>(r, tris, tri64, s);
+            s.pend = leaf;
+        } else {
+            s.pend = leaf;
+            closest_commit<F64>(r, tris, tri64, s);
+        }
     }
-    return true;
+    return next_group(st, s.g);
 }
 
 // Closest-hit traversal.  Returns the caller id (-1 on miss), the best
@@ -701,10 +815,13 @@ RISE_HD inline int trace_closest(const R& r, const NodeSlot* __restrict__ nodes,
     return s.best_id;
 }
 
-// Any-hit state: the current group, the box limit and the result.
+// Any-hit state: the current group, the box limit, the candidate awaiting the
+// certifier and the result.
 struct AnyState {
-    unsigned gbase, ghits, gimask;
+    NodeGroup g;
     unsigned faces;  // face selection (face_ok), read by the culling variant only
+    unsigned pend;   // leaf-order index of the candidate, kNoLeaf: none
+    bool over;       // every node has been visited
     bool hit;
     float tlim;
     float fbest;  // (float)dHowFar2: the filter's range (BVH.h:1283)
@@ -714,64 +831,61 @@ struct AnyState {
 template <class R>
 RISE_HD inline void any_begin(const R& r, double how_far2, AnyState& s)
 {
-    s.gbase = 0;
-    s.ghits = 1u << (0u ^ r.oinv);
-    s.gimask = 1u;
+    s.g = root_group(r);
     s.faces = 3u;
+    s.pend = kNoLeaf;
+    s.over = false;
     s.hit = false;
     s.how_far2 = how_far2;
     s.fbest = (float)how_far2;
     s.tlim = box_limit(r, how_far2);
 }
 
-// One any-hit step; true iff some triangle certifies with
-// kNearZero < t < how_far2 (...Specializations.h:517-519) and casts shadows
-// (bit 0 of v2.w clear; ObjectManager.cpp:119-124).  Returns false once
-// the query is decided (a hit, or the tree exhausted).
-template <bool COUNT, bool CULL = false, bool F64 = false, class Stack, class R>
+// Certifies the awaiting candidate: the query is answered iff it certifies
+// with kNearZero < t < how_far2 (...Specializations.h:517-519).
+template <bool F64, class R>
+RISE_HD inline void any_commit(const R& r, const Tri48* __restrict__ tris, const double* __restrict__ tri64,
+                               AnyState& s)
+{
+    const float4* tp = reinterpret_cast<const float4*>(tris + s.pend);
+    const float4 a = tp[0], b = tp[1], c = tp[2];
+    double tt;
+    const auto& q = late_ray(r);
+    if ((F64 ? certify64(q, tri64 + 9 * (size_t)s.pend, tt) : certify(q, a, b, c, tt)) && tt > kNearZero &&
+        tt < s.how_far2)
+        s.hit = true;
+    s.pend = kNoLeaf;
+}
+
+// One any-hit step.  Returns false once the query is decided (s.hit, or the
+// tree exhausted: s.over) or, with DEFER, once a candidate awaits any_commit;
+// a query that it leaves undecided (neither s.hit nor s.over) goes on.  With
+// DEFER a second candidate of the same node is certified at once.
+template <bool COUNT, bool CULL = false, bool F64 = false, bool DEFER = false, class Stack, class R>
 RISE_HD inline bool any_step(const R& r, const NodeSlot* __restrict__ nodes, const Tri48* __restrict__ tris,
                              Stack& st, AnyState& s, unsigned& n_nodes, unsigned& n_tris,
                              const double* __restrict__ tri64 = nullptr)
 {
-    unsigned tmask = 0, tbase = 0;
-    if (s.ghits) {
-        const unsigned k = __builtin_ctz(s.ghits);
-        s.ghits &= s.ghits - 1u;
-        const unsigned slot = k ^ r.oinv;
-        const unsigned ni = s.gbase + __builtin_popcount(s.gimask & ((1u << slot) - 1u));
-        if (s.ghits) st.push(make_uint2(s.gbase, s.ghits | (s.gimask << 8)));
-        if (COUNT) ++n_nodes;
-        unsigned cb, im;
-        s.ghits = test_node(r, nodes, ni, s.tlim, cb, im, tbase, tmask);
-        s.gbase = cb;
-        s.gimask = im;
-    }
-    while (tmask) {
-        const unsigned j = __builtin_ctz(tmask);
-        tmask &= tmask - 1u;
-        const float4* tp = reinterpret_cast<const float4*>(tris + tbase + j);
-        const float4 a = tp[0], b = tp[1], c = tp[2];
+    LeafWalk w;
+    visit_node<COUNT>(r, nodes, st, s.g, s.tlim, w, n_nodes);
+    while (w.slots) {
+        unsigned leaf;
+        if (!next_triangle(w, leaf)) continue;
         if (COUNT) ++n_tris;
-        const double* v64 = F64 ? tri64 + 9 * (size_t)(tbase + j) : nullptr;
-        if (CULL && s.faces != 3u && !(float_to_bits(c.w) & kTriDoubleSided) &&
-            !(F64 ? face_ok64(r, v64, s.faces) : face_ok(r, a, b, c, s.faces)))
-            continue;
-        double tt;
-        if (filter_float(r, a, b, c, s.fbest) && (F64 ? certify64(r, v64, tt) : certify(r, a, b, c, tt)) &&
-            tt > kNearZero && tt < s.how_far2 &&
-            !(float_to_bits(c.w) & 1u)) {
-            s.hit = true;
-            return false;
+        if (!passes_filter<CULL, F64, true>(r, tris, tri64, leaf, s.faces, s.fbest)) continue;
+        const bool second = s.pend != kNoLeaf;
+        if (!DEFER || second) {
+            const unsigned first = s.pend;
+            s.pend = leaf;
+            any_commit<F64>(r, tris, tri64, s);
+            if (s.hit) return false;
+            if (DEFER) s.pend = first;
+        } else {
+            s.pend = leaf;
         }
     }
-    if (!s.ghits) {
-        if (st.empty()) return false;
-        const uint2 g = st.pop();
-        s.gbase = g.x;
-        s.ghits = g.y & 0xffu;
-        s.gimask = (g.y >> 8) & 0xffu;
-    }
-    return true;
+    s.over = !next_group(st, s.g);
+    return !s.over && s.pend == kNoLeaf;
 }
 
 template <bool COUNT, class Stack, class R>

@@ -20,9 +20,6 @@ static_assert(kArithIeee == RISE_HIP_ARITH_IEEE && kArithX86Fma == RISE_HIP_ARIT
 
 namespace {
 
-#ifndef RISE_PERSISTENT
-#define RISE_PERSISTENT 1
-#endif
 #ifndef RISE_TRACE_BLOCK
 #define RISE_TRACE_BLOCK 128
 #endif
@@ -39,6 +36,14 @@ __device__ inline void load_ray(const float* __restrict__ rays, int64_t n, int64
     dz = rays[5 * n + i];
 }
 
+template <int A>
+__device__ inline void init_ray_at(RayStateT<A>& r, const float* __restrict__ rays, int64_t n, int64_t i)
+{
+    float ox, oy, oz, dx, dy, dz;
+    load_ray(rays, n, i, ox, oy, oz, dx, dy, dz);
+    init_ray(r, ox, oy, oz, dx, dy, dz);
+}
+
 template <bool COUNT>
 __device__ inline void flush_counts(unsigned long long* counters, unsigned nn, unsigned nt)
 {
@@ -48,66 +53,7 @@ __device__ inline void flush_counts(unsigned long long* counters, unsigned nn, u
     }
 }
 
-// STACK: node-group entries per lane held in LDS; 0 selects a private array.
-template <bool COUNT, int STACK, int A>
-__global__ __launch_bounds__(kBlock) void closest_kernel(const NodeSlot* __restrict__ nodes,
-                                                         const Tri48* __restrict__ tris,
-                                                         const float* __restrict__ rays, int64_t n,
-                                                         int32_t* __restrict__ prim_id, float* __restrict__ t_out,
-                                                         unsigned long long* counters)
-{
-    __shared__ uint2 lds[STACK > 0 ? STACK * kBlock : 1];
-    const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    if (i >= n) return;
-    float ox, oy, oz, dx, dy, dz;
-    load_ray(rays, n, i, ox, oy, oz, dx, dy, dz);
-    RayStateT<A> r;
-    init_ray(r, ox, oy, oz, dx, dy, dz);
-    unsigned nn = 0, nt = 0;
-    double best;
-    unsigned leaf;
-    int id;
-    if (STACK > 0) {
-        LdsStack<STACK> st{lds + threadIdx.x, kBlock, 0};
-        id = trace_closest<COUNT>(r, nodes, tris, st, best, leaf, nn, nt);
-    } else {
-        PrivStack st;
-        st.sp = 0;
-        id = trace_closest<COUNT>(r, nodes, tris, st, best, leaf, nn, nt);
-    }
-    prim_id[i] = id;
-    t_out[i] = id >= 0 ? (float)world_range(r, best) : INFINITY;
-    flush_counts<COUNT>(counters, nn, nt);
-}
-
-template <bool COUNT, int STACK, int A>
-__global__ __launch_bounds__(kBlock) void any_kernel(const NodeSlot* __restrict__ nodes, const Tri48* __restrict__ tris,
-                                                     const float* __restrict__ rays,
-                                                     const float* __restrict__ tmax, int64_t n,
-                                                     uint8_t* __restrict__ occluded, unsigned long long* counters)
-{
-    __shared__ uint2 lds[STACK > 0 ? STACK * kBlock : 1];
-    const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    if (i >= n) return;
-    float ox, oy, oz, dx, dy, dz;
-    load_ray(rays, n, i, ox, oy, oz, dx, dy, dz);
-    RayStateT<A> r;
-    init_ray(r, ox, oy, oz, dx, dy, dz);
-    const double how_far = tmax ? (double)tmax[i] : kRiseInfinity;
-    const double how_far2 = scale_how_far(r, how_far);
-    unsigned nn = 0, nt = 0;
-    bool occ;
-    if (STACK > 0) {
-        LdsStack<STACK> st{lds + threadIdx.x, kBlock, 0};
-        occ = trace_any<COUNT>(r, nodes, tris, st, how_far2, nn, nt);
-    } else {
-        PrivStack st;
-        st.sp = 0;
-        occ = trace_any<COUNT>(r, nodes, tris, st, how_far2, nn, nt);
-    }
-    occluded[i] = occ ? 1 : 0;
-    flush_counts<COUNT>(counters, nn, nt);
-}
+// STACK (below): node-group entries per lane held in LDS; 0 selects a private array.
 
 inline unsigned grid_for(int64_t n) { return (unsigned)((n + kBlock - 1) / kBlock); }
 
@@ -122,39 +68,21 @@ __global__ __launch_bounds__(kBlock) void closest_persistent(const NodeSlot* __r
                                                              const double* __restrict__ tri64)
 {
     __shared__ uint2 lds[STACK > 0 ? STACK * kBlock : 1];
-    LdsStack<STACK> lst{lds + threadIdx.x, kBlock, 0};
-    PrivStack pst;
-    pst.sp = 0;
-    RayStateT<A> r;
-    ClosestState s;
-    long long ray = -1;  // -1 idle, -2 exhausted
+    auto st = make_stack<STACK>(lds, kBlock);
+    const NodeSlot* const np = nodes;
+    const Tri48* const tp = tris;
     unsigned nn = 0, nt = 0;
-    const int64_t grid_threads = (int64_t)gridDim.x * blockDim.x;
-    for (bool first_pass = true;; first_pass = false) {
-        // The first item of every thread is assigned statically; later ones come from the counter.
-        const long long got = first_pass ? first_item(n) : refill(ray == -1, ray >= 0, next, n, grid_threads);
-        if (ray == -1 && got != -1) {
-            ray = got;
-            if (ray >= 0) {
-                float ox, oy, oz, dx, dy, dz;
-                load_ray(rays, n, ray, ox, oy, oz, dx, dy, dz);
-                init_ray(r, ox, oy, oz, dx, dy, dz);
-                closest_begin(r, s);
-                lst.sp = 0;
-                pst.sp = 0;
-            }
-        }
-        if (__ballot(ray >= 0) == 0ull && __ballot(ray == -1) == 0ull) break;
-        if (ray >= 0) {
-            const bool more = STACK > 0 ? closest_step<COUNT, false, F64>(r, nodes, tris, lst, s, nn, nt, tri64)
-                                        : closest_step<COUNT, false, F64>(r, nodes, tris, pst, s, nn, nt, tri64);
-            if (!more) {
-                prim_id[ray] = s.best_id;
-                t_out[ray] = s.best_id >= 0 ? (float)world_range(r, s.best_t) : INFINITY;
-                ray = -1;
-            }
-        }
-    }
+    persist_closest<COUNT, false, F64, RayStateT<A>>(
+        st, n, next, nn, nt, np, tp, tri64,
+        [&](int64_t i, RayStateT<A>& r, ClosestState& s) {
+            init_ray_at(r, rays, n, i);
+            closest_begin(r, s);
+            return true;
+        },
+        [&](int64_t i, const RayStateT<A>& r, const ClosestState& s) {
+            prim_id[i] = s.best_id;
+            t_out[i] = s.best_id >= 0 ? (float)world_range(r, s.best_t) : INFINITY;
+        });
     flush_counts<COUNT>(counters, nn, nt);
 }
 
@@ -168,39 +96,18 @@ __global__ __launch_bounds__(kBlock) void any_persistent(const NodeSlot* __restr
                                                          const double* __restrict__ tri64)
 {
     __shared__ uint2 lds[STACK > 0 ? STACK * kBlock : 1];
-    LdsStack<STACK> lst{lds + threadIdx.x, kBlock, 0};
-    PrivStack pst;
-    pst.sp = 0;
-    RayStateT<A> r;
-    AnyState s;
-    long long ray = -1;
+    auto st = make_stack<STACK>(lds, kBlock);
+    const NodeSlot* const np = nodes;
+    const Tri48* const tp = tris;
     unsigned nn = 0, nt = 0;
-    const int64_t grid_threads = (int64_t)gridDim.x * blockDim.x;
-    for (bool first_pass = true;; first_pass = false) {
-        // The first item of every thread is assigned statically; later ones come from the counter.
-        const long long got = first_pass ? first_item(n) : refill(ray == -1, ray >= 0, next, n, grid_threads);
-        if (ray == -1 && got != -1) {
-            ray = got;
-            if (ray >= 0) {
-                float ox, oy, oz, dx, dy, dz;
-                load_ray(rays, n, ray, ox, oy, oz, dx, dy, dz);
-                init_ray(r, ox, oy, oz, dx, dy, dz);
-                const double how_far = tmax ? (double)tmax[ray] : kRiseInfinity;
-                any_begin(r, scale_how_far(r, how_far), s);
-                lst.sp = 0;
-                pst.sp = 0;
-            }
-        }
-        if (__ballot(ray >= 0) == 0ull && __ballot(ray == -1) == 0ull) break;
-        if (ray >= 0) {
-            const bool more = STACK > 0 ? any_step<COUNT, false, F64>(r, nodes, tris, lst, s, nn, nt, tri64)
-                                        : any_step<COUNT, false, F64>(r, nodes, tris, pst, s, nn, nt, tri64);
-            if (!more) {
-                occluded[ray] = s.hit ? 1 : 0;
-                ray = -1;
-            }
-        }
-    }
+    persist_any<COUNT, false, F64, RayStateT<A>>(
+        st, n, next, nn, nt, np, tp, tri64,
+        [&](int64_t i, RayStateT<A>& r, AnyState& s) {
+            init_ray_at(r, rays, n, i);
+            any_begin(r, scale_how_far(r, tmax ? (double)tmax[i] : kRiseInfinity), s);
+            return true;
+        },
+        [&](int64_t i, const AnyState& s) { occluded[i] = s.hit ? 1 : 0; });
     flush_counts<COUNT>(counters, nn, nt);
 }
 
@@ -226,9 +133,7 @@ __global__ __launch_bounds__(kBlock) void ex_records(const Tri48* __restrict__ t
     if (i >= n) return;
     const StagedHit sh = *reinterpret_cast<const StagedHit*>(hits + i);
     RayStateT<A> r;
-    float ox, oy, oz, dx, dy, dz;
-    load_ray(rays, n, i, ox, oy, oz, dx, dy, dz);
-    init_ray(r, ox, oy, oz, dx, dy, dz);
+    init_ray_at(r, rays, n, i);
     rise_hip_hit h;
     h.prim_id = sh.id;
     if (sh.id >= 0) {
@@ -269,38 +174,21 @@ __global__ __launch_bounds__(kBlock) void closest_ex_persistent(const NodeSlot* 
                                                                 const double* __restrict__ attr)
 {
     __shared__ uint2 lds[STACK > 0 ? STACK * kBlock : 1];
-    LdsStack<STACK> lst{lds + threadIdx.x, kBlock, 0};
-    PrivStack pst;
-    pst.sp = 0;
-    RayStateT<A> r;
-    ClosestState s;
-    long long ray = -1;
+    auto st = make_stack<STACK>(lds, kBlock);
+    const NodeSlot* const np = nodes;
+    const Tri48* const tp = tris;
     unsigned nn = 0, nt = 0;
-    const int64_t grid_threads = (int64_t)gridDim.x * blockDim.x;
-    for (bool first_pass = true;; first_pass = false) {
-        const long long got = first_pass ? first_item(n) : refill(ray == -1, ray >= 0, next, n, grid_threads);
-        if (ray == -1 && got != -1) {
-            ray = got;
-            if (ray >= 0) {
-                float ox, oy, oz, dx, dy, dz;
-                load_ray(rays, n, ray, ox, oy, oz, dx, dy, dz);
-                init_ray(r, ox, oy, oz, dx, dy, dz);
-                closest_begin(r, s);
-                s.faces = faces;
-                lst.sp = 0;
-                pst.sp = 0;
-            }
-        }
-        if (__ballot(ray >= 0) == 0ull && __ballot(ray == -1) == 0ull) break;
-        if (ray >= 0) {
-            const bool more = STACK > 0 ? closest_step<false, true, F64>(r, nodes, tris, lst, s, nn, nt, tri64)
-                                        : closest_step<false, true, F64>(r, nodes, tris, pst, s, nn, nt, tri64);
-            if (!more) {
-                *reinterpret_cast<StagedHit*>(hits + ray) = StagedHit{s.best_id, s.best_leaf, s.best_t};
-                ray = -1;
-            }
-        }
-    }
+    persist_closest<false, true, F64, RayStateT<A>>(
+        st, n, next, nn, nt, np, tp, tri64,
+        [&](int64_t i, RayStateT<A>& r, ClosestState& s) {
+            init_ray_at(r, rays, n, i);
+            closest_begin(r, s);
+            s.faces = faces;
+            return true;
+        },
+        [&](int64_t i, const RayStateT<A>&, const ClosestState& s) {
+            *reinterpret_cast<StagedHit*>(hits + i) = StagedHit{s.best_id, s.best_leaf, s.best_t};
+        });
 }
 
 // Any hit with the face selection of rise_hip_intersect_any_ex.
@@ -314,39 +202,19 @@ __global__ __launch_bounds__(kBlock) void any_ex_persistent(const NodeSlot* __re
                                                             const double* __restrict__ tri64)
 {
     __shared__ uint2 lds[STACK > 0 ? STACK * kBlock : 1];
-    LdsStack<STACK> lst{lds + threadIdx.x, kBlock, 0};
-    PrivStack pst;
-    pst.sp = 0;
-    RayStateT<A> r;
-    AnyState s;
-    long long ray = -1;
+    auto st = make_stack<STACK>(lds, kBlock);
+    const NodeSlot* const np = nodes;
+    const Tri48* const tp = tris;
     unsigned nn = 0, nt = 0;
-    const int64_t grid_threads = (int64_t)gridDim.x * blockDim.x;
-    for (bool first_pass = true;; first_pass = false) {
-        const long long got = first_pass ? first_item(n) : refill(ray == -1, ray >= 0, next, n, grid_threads);
-        if (ray == -1 && got != -1) {
-            ray = got;
-            if (ray >= 0) {
-                float ox, oy, oz, dx, dy, dz;
-                load_ray(rays, n, ray, ox, oy, oz, dx, dy, dz);
-                init_ray(r, ox, oy, oz, dx, dy, dz);
-                const double how_far = tmax ? (double)tmax[ray] : kRiseInfinity;
-                any_begin(r, scale_how_far(r, how_far), s);
-                s.faces = faces;
-                lst.sp = 0;
-                pst.sp = 0;
-            }
-        }
-        if (__ballot(ray >= 0) == 0ull && __ballot(ray == -1) == 0ull) break;
-        if (ray >= 0) {
-            const bool more = STACK > 0 ? any_step<false, true, F64>(r, nodes, tris, lst, s, nn, nt, tri64)
-                                        : any_step<false, true, F64>(r, nodes, tris, pst, s, nn, nt, tri64);
-            if (!more) {
-                occluded[ray] = s.hit ? 1 : 0;
-                ray = -1;
-            }
-        }
-    }
+    persist_any<false, true, F64, RayStateT<A>>(
+        st, n, next, nn, nt, np, tp, tri64,
+        [&](int64_t i, RayStateT<A>& r, AnyState& s) {
+            init_ray_at(r, rays, n, i);
+            any_begin(r, scale_how_far(r, tmax ? (double)tmax[i] : kRiseInfinity), s);
+            s.faces = faces;
+            return true;
+        },
+        [&](int64_t i, const AnyState& s) { occluded[i] = s.hit ? 1 : 0; });
 }
 
 __global__ void reset_counter(unsigned long long* c) { *c = 0ull; }
@@ -358,8 +226,8 @@ unsigned persistent_grid(K kernel, int64_t n)
     static int cus = 0;
     if (cus == 0) {
         int dev = 0;
-        hipGetDevice(&dev);
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+        (void)hipGetDevice(&dev);
+        (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
         if (cus <= 0) cus = 256;
     }
     int per_cu = 0;
@@ -379,8 +247,7 @@ hipError_t launch_closest(const TraceScene& s, const float* rays, int64_t n, int
 {
     if (n <= 0) return hipSuccess;
     const int need = s.depth - 1;
-    const dim3 grid(grid_for(n)), block(kBlock);
-#if RISE_PERSISTENT
+    const dim3 block(kBlock);
     hipLaunchKernelGGL(reset_counter, dim3(1), dim3(1), 0, stream, s.fetch_counter);
 #define RISE_LAUNCH_CLOSEST_F(C, S, A, F)                                                                   \
     hipLaunchKernelGGL((closest_persistent<C, S, A, F>), dim3(persistent_grid(closest_persistent<C, S, A, F>, n)), \
@@ -390,12 +257,6 @@ hipError_t launch_closest(const TraceScene& s, const float* rays, int64_t n, int
         if (s.tri64) RISE_LAUNCH_CLOSEST_F(C, S, A, true); \
         else RISE_LAUNCH_CLOSEST_F(C, S, A, false);     \
     } while (0)
-#else
-    if (s.tri64) return hipErrorNotSupported;  // the one-ray-per-thread kernels certify on floats only
-#define RISE_LAUNCH_CLOSEST(C, S, A)                                                                          \
-    hipLaunchKernelGGL((closest_kernel<C, S, A>), grid, block, 0, stream, s.nodes, s.tris, rays, n, prim_id, t, \
-                       counters)
-#endif
 #define RISE_LAUNCH_CLOSEST_A(C, S)                                             \
     do {                                                                         \
         if (s.arith == kArithX86Fma) RISE_LAUNCH_CLOSEST(C, S, kArithX86Fma);    \
@@ -421,8 +282,7 @@ hipError_t launch_any(const TraceScene& s, const float* rays, const float* tmax,
 {
     if (n <= 0) return hipSuccess;
     const int need = s.depth - 1;
-    const dim3 grid(grid_for(n)), block(kBlock);
-#if RISE_PERSISTENT
+    const dim3 block(kBlock);
     hipLaunchKernelGGL(reset_counter, dim3(1), dim3(1), 0, stream, s.fetch_counter);
 #define RISE_LAUNCH_ANY_F(C, S, A, F)                                                                        \
     hipLaunchKernelGGL((any_persistent<C, S, A, F>), dim3(persistent_grid(any_persistent<C, S, A, F>, n)), block, \
@@ -432,12 +292,6 @@ hipError_t launch_any(const TraceScene& s, const float* rays, const float* tmax,
         if (s.tri64) RISE_LAUNCH_ANY_F(C, S, A, true); \
         else RISE_LAUNCH_ANY_F(C, S, A, false);     \
     } while (0)
-#else
-    if (s.tri64) return hipErrorNotSupported;  // the one-ray-per-thread kernels certify on floats only
-#define RISE_LAUNCH_ANY(C, S, A)                                                                             \
-    hipLaunchKernelGGL((any_kernel<C, S, A>), grid, block, 0, stream, s.nodes, s.tris, rays, tmax, n, occluded, \
-                       counters)
-#endif
 #define RISE_LAUNCH_ANY_A(C, S)                                             \
     do {                                                                     \
         if (s.arith == kArithX86Fma) RISE_LAUNCH_ANY(C, S, kArithX86Fma);    \
