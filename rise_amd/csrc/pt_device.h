@@ -35,6 +35,12 @@ struct DevMaterial {
     int ior_spd;    // GGX conductor n / dielectric index (-1: the reference's defaults)
     int ext_spd;    // GGX conductor k / dielectric transmittance per unit length (-1: none)
     float alpha;    // GGX roughness
+    // GGX: first entry of the material's Fresnel averages in
+    // PtSceneView::ggx_favg, one per pair of (conductor n, k) values its step
+    // spectra take in air, n-major with favg_stride entries a row (-1: none).
+    int favg;
+    int favg_stride;
+    int pad[2];
 };
 
 struct DevObject {
@@ -100,6 +106,7 @@ struct PtSceneView {
     const DevMaterial* materials;
     const DevSpd* spds;
     const float* spd_amp;
+    const float* ggx_favg;  // Fresnel averages of the GGX materials (DevMaterial::favg)
     const DevLuminary* lums;
     const unsigned* lum_tris;   // leaf-order triangle indices
     const float* lum_cdf;       // area CDF per luminary
@@ -216,6 +223,18 @@ RISE_HD inline float sample_u(const SampleKey& k, unsigned dim)
     return sobol_f(index, dim, k.scramble);
 }
 
+// sample_u at dimensions 2 pair and 2 pair + 1, which share the shuffled index.
+RISE_HD inline void sample_pair(const SampleKey& k, unsigned pair, float& u0, float& u1)
+{
+    unsigned index = k.index;
+    if (k.mask) {
+        const unsigned pair_seed = hash_combine(k.scramble, 0x51ed270bu + pair);
+        index = (index & ~k.mask) | (owen_scramble(index, pair_seed) & k.mask);
+    }
+    u0 = sobol_f(index, 2u * pair, k.scramble);
+    u1 = sobol_f(index, 2u * pair + 1u, k.scramble);
+}
+
 // MortonCode::Part1By1 (Utilities/MortonCode.h).
 RISE_HD inline unsigned morton_part1by1(unsigned x)
 {
@@ -290,6 +309,15 @@ RISE_HD inline float power_heuristic(float pa, float pb)
     return a2 / (a2 + pb * pb);
 }
 
+// Bin of a step spectrum that holds nm, which lies in its range.
+RISE_HD inline int spd_bin(const DevSpd& d, float nm)
+{
+    int idx = (int)((nm - d.begin) * d.inv_delta);
+    if (idx >= d.n) idx = d.n - 1;
+    if (idx < 0) idx = 0;
+    return idx;
+}
+
 // SpectralPacket::ValueAtNM (Utilities/Color/SpectralPacket.h:285-297).
 RISE_HD inline float spd_value(const PtSceneView& s, int spd, float nm)
 {
@@ -303,10 +331,7 @@ RISE_HD inline float spd_value(const PtSceneView& s, int spd, float nm)
         const float x = (c[0] * t + c[1]) * t + c[2];
         return c[3] * (0.5f + x / (2.0f * sqrtf(1.0f + x * x)));
     }
-    int idx = (int)((nm - d.begin) * d.inv_delta);
-    if (idx >= d.n) idx = d.n - 1;
-    if (idx < 0) idx = 0;
-    return s.spd_amp[d.offset + idx];
+    return s.spd_amp[d.offset + spd_bin(d, nm)];
 }
 
 // Offsets a surface point along the geometric normal so a ray leaving it
@@ -382,12 +407,20 @@ RISE_HD inline float emitted(const PtSceneView& s, const DevMaterial& m, f3 out,
     return spd_value(s, m.emit_spd, nm) * kInvPi * m.emit_scale;
 }
 
-// SampledWavelengths::SampleEquidistant (SampledWavelengths.h:79-106).
+// SampledWavelengths::SampleEquidistant (SampledWavelengths.h:79-106), one
+// wavelength: the hero's offset plus w steps, wrapped once into the range
+// (below twice the range, so the subtraction is exact, as fmod's result is).
+RISE_HD inline float wavelength(float lambda0, float a, float b, int w)
+{
+    if (w == 0) return lambda0;
+    const float range = b - a, delta = range / (float)kHwss;
+    const float x = lambda0 - a + (float)w * delta;
+    return a + (x >= range ? x - range : x);
+}
+
 RISE_HD inline void wavelengths(float lambda0, float a, float b, float lam[kHwss])
 {
-    const float range = b - a, delta = range / (float)kHwss;
-    lam[0] = lambda0;
-    for (int i = 1; i < kHwss; ++i) lam[i] = a + fmodf(lambda0 - a + (float)i * delta, range);
+    for (int i = 0; i < kHwss; ++i) lam[i] = wavelength(lambda0, a, b, i);
 }
 
 }  // namespace rise_hip

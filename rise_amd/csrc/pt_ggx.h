@@ -238,6 +238,7 @@ RISE_HD inline float fresnel_conductor(float cos_i, float ni, float nt, float kt
 RISE_HD inline float fresnel_avg(const GgxTables& T, float ni, float nt, float kt)
 {
     float sum = 0.0f;
+#pragma unroll 1
     for (int i = 0; i < 21; ++i) sum += fresnel_conductor(T.gl_x[i], ni, nt, kt) * (2.0f * T.gl_x[i] * T.gl_w[i]);
     return sum;
 }
@@ -266,30 +267,51 @@ RISE_HD inline void ggx_facing(const Surf& h, Onb& b, f3& gn)
     gn = dot3(raw, h.dir) < 0.0f ? raw : -raw;
 }
 
-// GGXBRDF::valueNM (GGXBRDF.cpp:339-498), conductor Fresnel.
-RISE_HD inline float ggx_value(const GgxTables& T, const Surf& h, const GgxParams& g, f3 vin)
+// GGXBRDF::valueNM (GGXBRDF.cpp:339-498), conductor Fresnel, in two parts:
+// what depends on the directions alone, and the value at one wavelength.
+struct GgxDir {
+    bool ok;
+    bool ms;        // the multiscatter lobe counts
+    float sf;       // D G2 / (4 cos cos)
+    float shape;    // multiscatter lobe over its Fresnel factor
+    float cos_h;    // cosine of the Fresnel term
+    float eavg;
+};
+
+RISE_HD inline GgxDir ggx_dir(const GgxTables& T, const Surf& h, float alpha, f3 vin)
 {
+    GgxDir d{false, false, 0.0f, 0.0f, 0.0f, 0.0f};
     Onb b;
     f3 gn;
     ggx_facing(h, b, gn);
     const f3 n = b.w, v = norm3(vin), r = norm3(-h.dir);
     const float nr = dot3(n, r), nv = dot3(n, v);
-    if (nr < kNearZeroF || nv < kNearZeroF) return 0.0f;
-    if (dot3(v, gn) <= 0.0f || dot3(r, gn) <= 0.0f) return 0.0f;
-    const float a = fmaxf(g.alpha, 1e-4f);
+    if (nr < kNearZeroF || nv < kNearZeroF) return d;
+    if (dot3(v, gn) <= 0.0f || dot3(r, gn) <= 0.0f) return d;
+    const float a = fmaxf(alpha, 1e-4f);
     const f3 hv = norm3(v + r);
-    const float sf = ggx_d(a, to_local(b, hv)) * ggx_g2(a, to_local(b, v), to_local(b, r)) / (4.0f * nv * nr);
+    d.ok = true;
+    d.sf = ggx_d(a, to_local(b, hv)) * ggx_g2(a, to_local(b, v), to_local(b, r)) / (4.0f * nv * nr);
+    d.cos_h = dot3(h.dir, hv);
+    d.eavg = lookup_eavg(T, a);
+    if (1.0f - d.eavg > 1e-10f) {
+        d.ms = true;
+        d.shape = (1.0f - lookup_ess(T, nr, a)) * (1.0f - lookup_ess(T, nv, a)) /
+                  (3.14159265358979f * (1.0f - d.eavg));
+    }
+    return d;
+}
+
+// f_avg: the hemispherical Fresnel average at (g.amb, g.ior, g.ext).
+RISE_HD inline float ggx_value(const GgxDir& d, const GgxParams& g, float f_avg)
+{
+    if (!d.ok) return 0.0f;
     float spec = 0.0f;
-    if (sf > 0.0f) {
-        const float f = fresnel_conductor(dot3(h.dir, hv), g.amb, g.ior, g.ext);
-        if (f > 0.0f) spec = g.rs * f * sf;
+    if (d.sf > 0.0f) {
+        const float f = fresnel_conductor(d.cos_h, g.amb, g.ior, g.ext);
+        if (f > 0.0f) spec = g.rs * f * d.sf;
     }
-    const float eavg = lookup_eavg(T, a);
-    if (1.0f - eavg > 1e-10f) {
-        const float shape = (1.0f - lookup_ess(T, nr, a)) * (1.0f - lookup_ess(T, nv, a)) /
-                            (3.14159265358979f * (1.0f - eavg));
-        spec += ggx_fms(g.rs * fresnel_avg(T, g.amb, g.ior, g.ext), eavg) * shape;
-    }
+    if (d.ms) spec += ggx_fms(g.rs * f_avg, d.eavg) * d.shape;
     return g.rd * kInvPi + spec;
 }
 
@@ -321,8 +343,11 @@ struct ScatterOut {
 
 // GGXSPF::ScatterNM (GGXSPF.cpp:424-687), conductor Fresnel: lobe by u_lobe,
 // direction by (u1, u2).
+// f_avg() gives the Fresnel average at (g.amb, g.ior, g.ext), which only the
+// multiscatter lobe needs.
+template <class Favg>
 RISE_HD inline ScatterOut ggx_scatter(const GgxTables& T, const Surf& h, const GgxParams& g, float u_lobe, float u1,
-                                      float u2)
+                                      float u2, Favg f_avg)
 {
     ScatterOut out{false, mk3(0, 0, 0), 0.0f, 0.0f, 0};
     Onb b;
@@ -377,7 +402,7 @@ RISE_HD inline ScatterOut ggx_scatter(const GgxTables& T, const Surf& h, const G
             if (ct > 0.0f && dot3(wo, gn) > 0.0f) {
                 const float sp = a >= 1e-6f ? vndf_pdf(wi, wo, b, a) : 0.0f;
                 const float mp = ms_pdf(T, ct, a, z);
-                const float fms = ggx_fms(g.rs * fresnel_avg(T, g.amb, g.ior, g.ext), eavg);
+                const float fms = ggx_fms(g.rs * f_avg(), eavg);
                 const float f_ms = fms * (1.0f - lookup_ess(T, ct, a)) * (1.0f - ess_i) * kInvPi / (1.0f - eavg);
                 const float kray = mp > 1e-14f ? f_ms * ct / (mp * p_ms) : 0.0f;
                 if (kray > 0.0f) out = ScatterOut{true, wo, kray, mix(ct, sp, ct * kInvPi), 0};

@@ -27,6 +27,11 @@ struct rise_hip_pt_scene {
 void release_solo_batch(rise_hip_pt_scene* s);
 
 namespace rise_hip {
+// Fills one GGX material's Fresnel averages (DevMaterial::favg) on the null
+// stream: the offsets of its n and k amplitudes in amp (-1: no spectrum, the
+// default value) and their counts (pt_render.hip).
+hipError_t fill_ggx_favg(float* out, const float* amp, int ior_offset, int n_ior, int ext_offset, int n_ext);
+
 struct Bvh2Tree;
 // rise_hip_pt_scene_create_with_media with, optionally, a binary tree per
 // object (object_trees[o] over that object's triangles, NULL: built), as a

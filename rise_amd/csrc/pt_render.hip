@@ -101,13 +101,20 @@ __device__ inline bool xyz_from_nm(float nm, float& X, float& Y, float& Z)
 }
 
 // HosekWilkieSkyModel::SampleRadiance (Utilities/HosekWilkieSkyModel.cpp:
-// 172-256) times the map's scale: Perez-weighted xyY in direction d (unit),
-// turned into a radiance at nm by the colour-matching functions.
-__device__ inline float sky_radiance(const DevSky& k, f3 d, float nm)
+// 172-256) times the map's scale, in two parts: the Perez-weighted xyY in
+// direction d (unit) as XYZ, and the radiance at nm by the colour-matching
+// functions.
+struct SkyDir {
+    bool on;
+    float X, Y, Z;
+};
+
+__device__ inline SkyDir sky_dir(const DevSky& k, f3 d)
 {
-    if (!k.on || nm < 380.0f || nm > 780.0f) return 0.0f;
+    SkyDir s{false, 0.0f, 0.0f, 0.0f};
+    if (!k.on) return s;
     d = norm3(d);
-    if (d.y <= 0.0f) return 0.0f;
+    if (d.y <= 0.0f) return s;
     const float ds = fmaxf(-1.0f, fminf(1.0f, d.x * k.sun[0] + d.y * k.sun[1] + d.z * k.sun[2]));
     const float g = acosf(ds), cg = cosf(g);
     const float sc = fmaxf(1e-3f, d.y);
@@ -117,13 +124,17 @@ __device__ inline float sky_radiance(const DevSky& k, f3 d, float nm)
         v[c] = k.zen[c] * (1.0f + p[0] * expf(p[1] / sc)) * (1.0f + p[2] * expf(p[3] * g) + p[4] * cg * cg);
     }
     const float Y = v[0], x = v[1], y = v[2];
-    if (Y < 0.0f || y < 1e-6f) return 0.0f;
-    const float X = (x / y) * Y, Z = ((1.0f - x - y) / y) * Y;
+    if (Y < 0.0f || y < 1e-6f) return s;
+    return SkyDir{true, (x / y) * Y, Y, ((1.0f - x - y) / y) * Y};
+}
+
+__device__ inline float sky_radiance(const DevSky& k, const SkyDir& s, float nm)
+{
     float ox, oy, oz;
-    if (!xyz_from_nm(nm, ox, oy, oz)) return 0.0f;
+    if (!s.on || !xyz_from_nm(nm, ox, oy, oz)) return 0.0f;
     const float den = ox + oy + oz;
     if (den < 1e-9f) return 0.0f;
-    return (X * ox + Y * oy + Z * oz) / den * k.scale;
+    return (s.X * ox + s.Y * oy + s.Z * oz) / den * k.scale;
 }
 
 // One request: scene tables, render parameters, film accumulators, output.
@@ -227,11 +238,11 @@ struct BlockPush {
         __syncthreads();
         if (threadIdx.x < NB) {
             unsigned* c = b + threadIdx.x * (W + 1);
-            unsigned total = 0;
+            unsigned n[W], total = 0;
+            for (int w = 0; w < W; ++w) n[w] = c[w];  // all loads before the first store
             for (int w = 0; w < W; ++w) {
-                const unsigned n = c[w];
                 c[w] = total;
-                total += n;
+                total += n[w];
             }
             c[W] = total ? atomicAdd(counters[threadIdx.x], total) : 0u;
         }
@@ -243,6 +254,47 @@ struct BlockPush {
         unsigned* const cs[1] = {counter};
         return (*this)(cs, pred ? 0 : -1);
     }
+};
+
+// BlockPush for up to four entries of one queue per thread: thread i reserves
+// one entry for each bit of its mask with one pair of barriers and one atomic
+// for all of them, where four BlockPushes take four of each.  pos(k) is the
+// entry of bit k; the entries of one bit are contiguous over the workgroup.
+template <int BLOCK>
+struct BlockPush4 {
+    static constexpr int W = BLOCK / 64, N = 4 * W;
+    static_assert(N <= 64, "one wave scans the counts");
+    unsigned* lds;  // 2 * (N + 1) entries
+    int flip;
+    unsigned rank[4];
+    const unsigned* b;
+
+    __device__ inline void reserve(unsigned* counter, unsigned mask)
+    {
+        unsigned* c = lds + flip * (N + 1);
+        flip ^= 1;
+        b = c;
+        const unsigned wave = threadIdx.x >> 6;
+        for (int k = 0; k < 4; ++k) {
+            const unsigned long long m = __ballot((mask >> k) & 1u);
+            rank[k] = __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+            if (__lane_id() == 0) c[k * W + wave] = (unsigned)__popcll(m);
+        }
+        __syncthreads();
+        if (wave == 0) {
+            const int lane = (int)__lane_id();
+            const unsigned n = lane < N ? c[lane] : 0u;
+            unsigned incl = n;
+            for (int d = 1; d < N; d <<= 1) {
+                const unsigned up = __shfl_up(incl, d);
+                if (lane >= d) incl += up;
+            }
+            if (lane < N) c[lane] = incl - n;
+            if (lane == N - 1) c[N] = incl ? atomicAdd(counter, incl) : 0u;
+        }
+        __syncthreads();
+    }
+    __device__ inline unsigned pos(int k) const { return b[N] + b[k * W + (int)(threadIdx.x >> 6)] + rank[k]; }
 };
 
 // Index of the last entry whose field KEY is <= x (entries sorted by KEY,
@@ -421,6 +473,20 @@ constexpr GgxTables make_ggx_tables()
 
 __constant__ GgxTables c_ggx = make_ggx_tables();
 
+// One GGX material's Fresnel averages in air, n-major: n and k from the
+// material's step spectra with 0 appended (outside their range), or the
+// default alone.
+__global__ void k_ggx_favg(float* out, const float* amp, int ior_offset, int n_ior, int ext_offset, int n_ext)
+{
+    const int rows = ior_offset >= 0 ? n_ior + 1 : 1, cols = ext_offset >= 0 ? n_ext + 1 : 1;
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < rows * cols; i += gridDim.x * blockDim.x) {
+        const int r = i / cols, c = i % cols;
+        const float n = ior_offset < 0 ? 2.45f : r < n_ior ? amp[ior_offset + r] : 0.0f;
+        const float k = ext_offset < 0 ? 3.45f : c < n_ext ? amp[ext_offset + c] : 0.0f;
+        out[i] = fresnel_avg(c_ggx, 1.0f, n, k);
+    }
+}
+
 // Painter defaults of the scene-file chunks when a spectrum is absent:
 // ggx_material ior 2.45, extinction 3.45; dielectric_material ior 1.33, tau
 // none (ChunkParserRegistry.cpp:3206-3207, 3835-3836).
@@ -435,13 +501,55 @@ __device__ inline GgxParams ggx_params(const PtSceneView& sc, const DevMaterial&
                      spd_or(sc, m.ior_spd, nm, 2.45f), spd_or(sc, m.ext_spd, nm, 3.45f), amb};
 }
 
-// IBSDF::valueNM of a non-delta material of kind MAT (the dielectric has no BSDF).
+// The Fresnel average of a GGX material at nm in a medium of index amb: from
+// the scene's table in air (the spectra take few values there, and the
+// 21-point rule is some 2300 instructions), else by the rule itself.  A k_shade
+// vertex evaluates the BSDF up to 15 times; with the rule at each, k_shade of
+// GGX hits took 2430 us of the 333 x 250 x 9 materials render, with the table
+// and the wavelength loops rolled 1260.
+__device__ inline float ggx_favg(const PtSceneView& sc, const DevMaterial& m, float nm, const GgxParams& g)
+{
+    if (m.favg >= 0 && g.amb == 1.0f) {
+        int row = 0, col = 0;  // an absent spectrum has the one default value; outside its range a spectrum is 0, the last entry
+        if (m.ior_spd >= 0) {
+            const DevSpd d = sc.spds[m.ior_spd];
+            row = (nm < d.begin || nm > d.end) ? d.n : spd_bin(d, nm);
+        }
+        if (m.ext_spd >= 0) {
+            const DevSpd d = sc.spds[m.ext_spd];
+            col = (nm < d.begin || nm > d.end) ? d.n : spd_bin(d, nm);
+        }
+        return sc.ggx_favg[m.favg + row * m.favg_stride + col];
+    }
+    return fresnel_avg(c_ggx, g.amb, g.ior, g.ext);
+}
+
+// IBSDF::valueNM of a non-delta material of kind MAT (the dielectric has no
+// BSDF): what depends on the direction alone, then the value at a wavelength.
 template <int MAT>
-__device__ inline float bsdf_value(const PtSceneView& sc, const DevMaterial& m, const Surf& h, f3 v, float nm,
+struct BsdfDir {
+    bool reflects;  // Lambertian
+    GgxDir ggx;
+};
+
+template <int MAT>
+__device__ inline BsdfDir<MAT> bsdf_dir(const DevMaterial& m, const Surf& h, f3 v)
+{
+    BsdfDir<MAT> d{};
+    if (MAT == kMatLambert) d.reflects = should_reflect(h, v);
+    if (MAT == kMatGgx) d.ggx = ggx_dir(c_ggx, h, m.alpha, v);
+    return d;
+}
+
+template <int MAT>
+__device__ inline float bsdf_value(const PtSceneView& sc, const DevMaterial& m, const BsdfDir<MAT>& d, float nm,
                                    float amb)
 {
-    if (MAT == kMatLambert) return lambert_value(sc, h, m.refl_spd, v, nm);
-    if (MAT == kMatGgx) return ggx_value(c_ggx, h, ggx_params(sc, m, nm, amb), v);
+    if (MAT == kMatLambert) return d.reflects ? spd_value(sc, m.refl_spd, nm) * kInvPi : 0.0f;
+    if (MAT == kMatGgx && d.ggx.ok) {
+        const GgxParams g = ggx_params(sc, m, nm, amb);
+        return ggx_value(d.ggx, g, d.ggx.ms ? ggx_favg(sc, m, nm, g) : 0.0f);
+    }
     return 0.0f;
 }
 
@@ -460,7 +568,10 @@ template <int MAT>
 __device__ inline ScatterOut bsdf_scatter(const PtSceneView& sc, const DevMaterial& m, const Surf& h, float nm,
                                           float amb, float u1, float u2, float u3)
 {
-    if (MAT == kMatGgx) return ggx_scatter(c_ggx, h, ggx_params(sc, m, nm, amb), u3, u1, u2);
+    if (MAT == kMatGgx) {
+        const GgxParams g = ggx_params(sc, m, nm, amb);
+        return ggx_scatter(c_ggx, h, g, u3, u1, u2, [&] { return ggx_favg(sc, m, nm, g); });
+    }
     // LambertianSPF::ScatterNM (Materials/LambertianSPF.cpp:90-131).
     ScatterOut out{false, mk3(0, 0, 0), 0.0f, 0.0f, 0};
     Onb fr = h.frame;
@@ -479,19 +590,18 @@ __device__ inline ScatterOut bsdf_scatter(const PtSceneView& sc, const DevMateri
 
 // The BSDF's sampler draws at a vertex whose BSDF dimensions start at s0, in
 // the reference's order (GGX: the lobe, then two, GGXSPF.cpp:479-519;
-// Lambertian: two, LambertianSPF.cpp:90-99), after them the lobe choice;
+// Lambertian: two, LambertianSPF.cpp:90-99), after them the lobe choice; s0 is
+// even (32 dimensions a vertex, an even number a light sample);
 // returns the dimension of the Russian-roulette draw.
 template <int MAT>
 __device__ inline unsigned bsdf_draws(const SampleKey& k, unsigned s0, float& u1, float& u2, float& u3)
 {
     if (MAT == kMatGgx) {
-        u3 = sample_u(k, s0);
-        u1 = sample_u(k, s0 + 1);
+        sample_pair(k, s0 >> 1, u3, u1);
         u2 = sample_u(k, s0 + 2);
         return s0 + 4;
     }
-    u1 = sample_u(k, s0);
-    u2 = sample_u(k, s0 + 1);
+    sample_pair(k, s0 >> 1, u1, u2);
     u3 = 0.0f;
     return s0 + 3;
 }
@@ -706,7 +816,9 @@ __device__ inline int lane_medium_object(const PtSceneView& sc, const Paths& S, 
 // -> HomogeneousMedium::SampleDistanceNM, HomogeneousMedium.cpp:150-172): a
 // scatter before the hit goes to the volume bin with its distance in hit_t;
 // otherwise the lane takes the survival weight Tr / pSurvival (:1895-1910,
-// IMedium.h:235-251) and goes on to the surface or the escape.
+// IMedium.h:235-251) and goes on to the surface or the escape.  SKY: some
+// scene of the pass has a sky that escaping rays see.
+template <bool SKY>
 __global__ __launch_bounds__(kShadeBlock) void k_bin(const ReqInfo* __restrict__ reqs, Paths S, int depth)
 {
     __shared__ unsigned lds[2 * kBins * (kShadeBlock / 64 + 1)];
@@ -757,12 +869,11 @@ __global__ __launch_bounds__(kShadeBlock) void k_bin(const ReqInfo* __restrict__
             } else if (leaf != 0xffffffffu) {
                 const int obj = float_to_bits(reinterpret_cast<const float4*>(sc.tris + leaf)[1].w);
                 kind = sc.materials[sc.objects[obj].material].type;
-            } else if (sc.sky.on && (depth > 0 || R.sky_background)) {
+            } else if (SKY && sc.sky.on && (depth > 0 || R.sky_background)) {
                 // Escape (PathTracingIntegrator.cpp:4230-4290, 5070-5110 and the
                 // single-wavelength twin): the sky at each wavelength the ray
                 // carries.
-                float lam[kHwss];
-                wavelengths(S.lambda0[slot], R.lambda_begin, R.lambda_end, lam);
+                const float lam0 = S.lambda0[slot];
                 const f3 d = mk3(S.dx[li], S.dy[li], S.dz[li]);
                 // A BSDF-sampled ray is weighed against the environment light
                 // sample by the power heuristic (:4259-4282); camera rays and
@@ -774,9 +885,14 @@ __global__ __launch_bounds__(kShadeBlock) void k_bin(const ReqInfo* __restrict__
                     const float pe = (float)env_pdf(*sc.env, dd);
                     if (pe > 0.0f) wmis = power_heuristic(pin, pe);
                 }
-                for (int w = 0; w < kHwss; ++w)
-                    if (!nm) S.res[w * S.cap + slot] += S.thr[w * S.cap + slot] * (sky_radiance(sc.sky, d, lam[w]) * wmis);
-                if (nm) S.res[li] += S.thr0[li] * (S.thr[li] * (sky_radiance(sc.sky, d, lam[lane]) * wmis));
+                const SkyDir sd = sky_dir(sc.sky, d);
+#pragma unroll 1
+                for (int w = nm ? (int)lane : 0; w < (nm ? (int)lane + 1 : kHwss); ++w) {
+                    const unsigned lw = (unsigned)w * (unsigned)S.cap + slot;
+                    const float L = sky_radiance(sc.sky, sd, wavelength(lam0, R.lambda_begin, R.lambda_end, w)) * wmis;
+                    if (nm) S.res[lw] += S.thr0[lw] * (S.thr[lw] * L);
+                    else S.res[lw] += S.thr[lw] * L;
+                }
             }
         }
         const unsigned at = push(cnt, kind);  // kind kMatVolume only when the pass has media
@@ -791,13 +907,11 @@ __device__ inline f3 surface_origin(const Surf& h, f3 dir)
     return offset_ray(h.p, dot3(dir, h.ng) > 0.0f ? h.ng : -h.ng);
 }
 
-// Writes lane w's next ray from `no` and appends it to the next extension
-// queue at `at`.
-__device__ inline void write_continuation(Paths& S, f3 no, unsigned slot, unsigned w, unsigned* at, f3 dir, float pdf,
-                                          float imp, unsigned bounces, const IorStack& st, unsigned vbn)
+// Writes the next ray of lane entry lw (w * cap + slot) from `no`.
+__device__ inline void write_lane(Paths& S, f3 no, unsigned lw, f3 dir, float pdf, float imp, unsigned bounces,
+                                  const IorStack& st, unsigned vbn)
 {
-    const unsigned cap = (unsigned)S.cap, lw = w * cap + slot;
-    *at = slot * 4u + w;
+    const unsigned cap = (unsigned)S.cap;
     if (S.vb) S.vb[lw] = (unsigned char)vbn;
     S.ox[lw] = no.x;
     S.oy[lw] = no.y;
@@ -812,18 +926,43 @@ __device__ inline void write_continuation(Paths& S, f3 no, unsigned slot, unsign
         if (k < st.n) S.ior_obj[k * 4 * cap + lw] = st.obj[k];
 }
 
+// The same for lane w of a path, appended to the next extension queue at `at`.
+__device__ inline void write_continuation(Paths& S, f3 no, unsigned slot, unsigned w, unsigned* at, f3 dir, float pdf,
+                                          float imp, unsigned bounces, const IorStack& st, unsigned vbn)
+{
+    *at = slot * 4u + w;
+    write_lane(S, no, w * (unsigned)S.cap + slot, dir, pdf, imp, bounces, st, vbn);
+}
+
 // One bounce for the active queue: IntegrateFromHitHWSS
 // (PathTracingIntegrator.cpp:3939-4822) for paths still sharing one ray, and
 // the single-wavelength loop IntegrateFromHitNM (:1561-3377) for paths that
 // hit a dielectric, whose wavelengths then continue as separate lanes.  Every
 // thread of a wave runs the same loop trips (the queue bound is uniform per
-// block) so the compaction ballots see all lanes; each shadow record is
-// written as soon as it is made, which keeps one record live at a time.
-template <int MAT>
-__global__ __launch_bounds__(kShadeBlock) void k_shade(const ReqInfo* __restrict__ reqs, Paths S, int depth)
+// block) so the compaction ballots see all lanes.  The shadow records of a
+// vertex's wavelengths are staged in LDS and reserved together (BlockPush4).
+// SKY: some scene of the pass has an environment sample or directional lights;
+// without them the kernel holds neither their code nor its registers.
+// Bound by latency at few waves: the loops over the wavelengths are kept
+// rolled (unrolled, the GGX kernel was 24k instructions, over twice the
+// instruction cache, and one vertex took 150 us) and a wave of lanes that
+// carry one wavelength each makes one trip instead of four.  Cornell box
+// 256 x 256 x 16: 988 -> 595 us in this kernel; 1080p terrain, Lambertian 2359
+// -> 1754, GGX 5369 -> 2750, dielectric 1807 -> 1498 us.  (At 4 waves the GGX
+// kernel spills 54 registers and is 5% slower than at 3.)
+constexpr int kShadeWaves[3] = {4, 3, 4};  // per SIMD, by material kind: what the registers are budgeted for
+
+template <int MAT, bool SKY>
+__global__ __launch_bounds__(kShadeBlock, kShadeWaves[MAT]) void k_shade(const ReqInfo* __restrict__ reqs, Paths S,
+                                                                         int depth)
 {
     __shared__ unsigned lds[2 * (kShadeBlock / 64 + 1)];
+    __shared__ unsigned lds4[2 * (4 * (kShadeBlock / 64) + 1)];
+    __shared__ float stage[MAT != kMatDielectric ? 4 : 1][5][MAT != kMatDielectric ? kShadeBlock : 1];
     BlockPush<kShadeBlock, 1> push{lds, 0};
+    BlockPush4<kShadeBlock> push4;
+    push4.lds = lds4;
+    push4.flip = 0;
     const unsigned n = S.cnt_mat[MAT * (kMaxPathDepth + 1) + depth];
     const unsigned* qin = S.mqueue[MAT];
     unsigned* qout = S.queue[(depth + 1) & 1];
@@ -853,7 +992,7 @@ __global__ __launch_bounds__(kShadeBlock) void k_shade(const ReqInfo* __restrict
         DevMaterial mat{};
         SampleKey key{0u, 0u, 0u};
         f3 o = mk3(0, 0, 0);
-        float lam[kHwss] = {0, 0, 0, 0};
+        float lam0 = 0.0f;
         float pdf_in = 0.0f, imp = 1.0f;
         unsigned bst = 0, vbn = 0;
         int mobj = -1;  // object whose medium holds the hit point (single-wavelength lanes)
@@ -862,7 +1001,7 @@ __global__ __launch_bounds__(kShadeBlock) void k_shade(const ReqInfo* __restrict
             key = sample_key(R, S.path_id[slot]);
             o = mk3(S.ox[li], S.oy[li], S.oz[li]);
             const f3 d = mk3(S.dx[li], S.dy[li], S.dz[li]);
-            wavelengths(S.lambda0[slot], R.lambda_begin, R.lambda_end, lam);
+            lam0 = S.lambda0[slot];
             pdf_in = S.pdf[li];
             imp = S.imp[li];
             bst = S.state[li];
@@ -894,7 +1033,10 @@ __global__ __launch_bounds__(kShadeBlock) void k_shade(const ReqInfo* __restrict
         // on as its own lane from this hit (:4348-4365).
         const bool branch = valid && !nm && MAT == kMatDielectric;
         const bool surface = valid && MAT != kMatDielectric;  // emission, NEE, BSDF sampling
-        const float amb = nm ? ior_top(sc, ist, lam[lane]) : 1.0f;
+        // Wavelength w of the path, computed where it is needed: the loops over the
+        // wavelengths are not unrolled (their bodies are the bulk of the kernel).
+        auto lam_of = [&](unsigned w) { return wavelength(lam0, R.lambda_begin, R.lambda_end, (int)w); };
+        const float amb = nm ? ior_top(sc, ist, lam_of(lane)) : 1.0f;
 
         // Emission with MIS against NEE (:4422-4515).
         if (MAT == kMatLambert && valid && mat.emit_spd >= 0) {
@@ -908,9 +1050,13 @@ __global__ __launch_bounds__(kShadeBlock) void k_shade(const ReqInfo* __restrict
                     mis = power_heuristic(pdf_in, ps * (dist * dist) / (L.area * cos_l));
                 }
             }
-            for (int w = 0; w < kHwss; ++w)
-                if (!nm) S.res[w * cap + slot] += S.thr[w * cap + slot] * (emitted(sc, mat, -h.dir, h.ng, lam[w]) * mis);
-            if (nm) S.res[li] += S.thr0[li] * (S.thr[li] * (emitted(sc, mat, -h.dir, h.ng, lam[lane]) * mis));
+#pragma unroll 1
+            for (unsigned w = nm ? lane : 0u; w < (nm ? lane + 1u : (unsigned)kHwss); ++w) {
+                const unsigned lw = w * cap + slot;
+                const float e = emitted(sc, mat, -h.dir, h.ng, lam_of(w)) * mis;
+                if (nm) S.res[lw] += S.thr0[lw] * (S.thr[lw] * e);
+                else S.res[lw] += S.thr[lw] * e;
+            }
         }
 
         // Next-event estimation (:4521-4552 and the NM twin ->
@@ -920,89 +1066,107 @@ __global__ __launch_bounds__(kShadeBlock) void k_shade(const ReqInfo* __restrict
         // every directional light deterministically.  Each kind of contribution
         // has its own shadow record and result array, so no two records of a
         // bounce add into the same place.
+        // A shared ray's wavelengths take a trip each, a single-wavelength lane
+        // the first one.
         const unsigned ls_dims = light_sample_dims(sc);
-        const bool blk_env = __syncthreads_or(surface && sc.env != nullptr);
-        const bool blk_dir = __syncthreads_or(surface && sc.n_dir > 0);
-        for (int w = 0; w < kHwss; ++w) {
-            const bool mine = surface && (!nm || (unsigned)w == lane);
-            const unsigned dim = nm ? base_dim : base_dim + ls_dims * (unsigned)w;
-            bool has = false;
-            float v = 0.0f, stm = 0.0f;
-            f3 sorg = mk3(0, 0, 0), to = mk3(0, 0, 0);
-            if (mine && sc.n_lums > 0) {
-                const float usel = sample_u(key, dim);
+        const int trips = __ballot(surface && !nm) != 0ull ? kHwss : 1;
+        if constexpr (MAT != kMatDielectric) {
+            // The record's stage slot of trip k: direction, distance, value.
+            auto put = [&](int k, f3 to, float dist, float v) {
+                stage[k][0][threadIdx.x] = to.x;
+                stage[k][1][threadIdx.x] = to.y;
+                stage[k][2][threadIdx.x] = to.z;
+                stage[k][3][threadIdx.x] = dist;
+                stage[k][4][threadIdx.x] = v;
+            };
+            auto flush = [&](unsigned mask, unsigned kind) {
+                push4.reserve(cnt_sh, mask);
+                for (int k = 0; k < kHwss; ++k) {
+                    if (!((mask >> k) & 1u)) continue;
+                    const f3 to = mk3(stage[k][0][threadIdx.x], stage[k][1][threadIdx.x], stage[k][2][threadIdx.x]);
+                    const f3 so = offset_ray(h.p, dot3(to, h.ng) > 0.0f ? h.ng : -h.ng);
+                    write_shadow(S, push4.pos(k), so, to, stage[k][3][threadIdx.x], stage[k][4][threadIdx.x],
+                                 (slot * 4u + (nm ? lane : (unsigned)k)) | kind, (unsigned)(mobj + 1));
+                }
+            };
+            unsigned mask = 0;
+#pragma unroll 1
+            for (int k = 0; k < trips; ++k) {
+                if (!surface || (nm && k > 0) || sc.n_lums <= 0) continue;
+                const unsigned w = nm ? lane : (unsigned)k;
+                const float lw = lam_of(w);
+                const unsigned dim = nm ? base_dim : base_dim + ls_dims * w;
+                float usel, ux, uy, uz;
+                sample_pair(key, dim >> 1, usel, ux);
                 int li_ = 0;
                 while (li_ < sc.n_lums - 1 && !(usel < sc.lums[li_].cdf_select)) ++li_;
-                if (li_ != ob.luminary) {  // never the shading object itself (:2061)
-                    const DevLuminary L = sc.lums[li_];
-                    const float ux = sample_u(key, dim + 1), uy = sample_u(key, dim + 2), uz = sample_u(key, dim + 3);
-                    // UniformRandomPoint: first CDF entry >= uz, then PointOnTriangle
-                    // (TriangleMeshGeometryIndexed.cpp:207-218, GeometricUtilities.cpp:543-560).
-                    int k = 0;
-                    while (k < L.tri_count - 1 && sc.lum_cdf[L.tri_first + k] < uz) ++k;
-                    const float4* lp = reinterpret_cast<const float4*>(sc.tris + sc.lum_tris[L.tri_first + k]);
-                    const float4 la = lp[0], lb = lp[1], lc = lp[2];
-                    const f3 a0 = mk3(la.x, la.y, la.z), a1 = mk3(lb.x, lb.y, lb.z), a2 = mk3(lc.x, lc.y, lc.z);
-                    const float sa = sqrtf(1.0f - ux);
-                    const float al = 1.0f - sa, be = sa * uy, ga = 1.0f - al - be;
-                    const f3 pl = a1 * al + a2 * be + a0 * ga;
-                    const f3 ln = norm3(cross3(a1 - a0, a2 - a0));
-                    to = pl - h.p;
-                    const float dist = len3(to);
-                    if (dist > 0.0f) to = to * (1.0f / dist);
-                    const float cos_s = dot3(to, h.n);
-                    const float cos_l = dot3(-to, ln);
-                    if (cos_l > 0.0f && cos_s > 0.0f) {
-                        const DevMaterial lm = sc.materials[L.material];
-                        const float le = emitted(sc, lm, -to, ln, lam[w]);
-                        const float geom = L.area * cos_l / (dist * dist);
-                        float contrib = le * cos_s * geom * bsdf_value<MAT>(sc, mat, h, to, lam[w], amb);
-                        const float p_light = L.pdf_select * (dist * dist) / (L.area * cos_l);
-                        const float p_bsdf = bsdf_pdf<MAT>(sc, mat, h, to, lam[w], amb);
-                        if (p_bsdf > 0.0f) contrib *= power_heuristic(p_light, p_bsdf);
-                        contrib /= L.pdf_select;
-                        v = nm ? S.thr0[li] * (S.thr[li] * contrib) : S.thr[w * cap + slot] * contrib;
-                        if (v > 0.0f) {
-                            has = true;
-                            sorg = offset_ray(h.p, dot3(to, h.ng) > 0.0f ? h.ng : -h.ng);
-                            stm = dist;
-                        }
-                    }
+                if (li_ == ob.luminary) continue;  // never the shading object itself (:2061)
+                sample_pair(key, (dim >> 1) + 1u, uy, uz);
+                const DevLuminary L = sc.lums[li_];
+                // UniformRandomPoint: first CDF entry >= uz, then PointOnTriangle
+                // (TriangleMeshGeometryIndexed.cpp:207-218, GeometricUtilities.cpp:543-560).
+                int t = 0;
+                while (t < L.tri_count - 1 && sc.lum_cdf[L.tri_first + t] < uz) ++t;
+                const float4* lp = reinterpret_cast<const float4*>(sc.tris + sc.lum_tris[L.tri_first + t]);
+                const float4 la = lp[0], lb = lp[1], lc = lp[2];
+                const f3 a0 = mk3(la.x, la.y, la.z), a1 = mk3(lb.x, lb.y, lb.z), a2 = mk3(lc.x, lc.y, lc.z);
+                const float sa = sqrtf(1.0f - ux);
+                const float al = 1.0f - sa, be = sa * uy, ga = 1.0f - al - be;
+                const f3 pl = a1 * al + a2 * be + a0 * ga;
+                const f3 ln = norm3(cross3(a1 - a0, a2 - a0));
+                f3 to = pl - h.p;
+                const float dist = len3(to);
+                if (dist > 0.0f) to = to * (1.0f / dist);
+                const float cos_s = dot3(to, h.n);
+                const float cos_l = dot3(-to, ln);
+                if (!(cos_l > 0.0f && cos_s > 0.0f)) continue;
+                const DevMaterial lm = sc.materials[L.material];
+                const float le = emitted(sc, lm, -to, ln, lw);
+                const float geom = L.area * cos_l / (dist * dist);
+                float contrib = le * cos_s * geom * bsdf_value(sc, mat, bsdf_dir<MAT>(mat, h, to), lw, amb);
+                const float p_light = L.pdf_select * (dist * dist) / (L.area * cos_l);
+                const float p_bsdf = bsdf_pdf<MAT>(sc, mat, h, to, lw, amb);
+                if (p_bsdf > 0.0f) contrib *= power_heuristic(p_light, p_bsdf);
+                contrib /= L.pdf_select;
+                const float v = nm ? S.thr0[li] * (S.thr[li] * contrib) : S.thr[w * cap + slot] * contrib;
+                if (v > 0.0f) {
+                    mask |= 1u << k;
+                    put(k, to, dist, v);
                 }
             }
-            const unsigned si = push(cnt_sh, has);
-            if (has) write_shadow(S, si, sorg, to, stm, v, slot * 4u + (unsigned)w, (unsigned)(mobj + 1));
+            flush(mask, kRecLum << kRecKindShift);
 
             // Environment sample (:2278-2358): a direction from the sky's
             // importance table, the sky at this wavelength, power heuristic
             // against the BSDF's pdf, a shadow ray to infinity.
-            if (blk_env) {
-                bool has_e = false;
-                float ve = 0.0f;
-                f3 ed = mk3(0, 0, 0), eo = mk3(0, 0, 0);
-                if (mine && sc.env) {
-                    const unsigned ed0 = dim + (sc.n_lums > 0 ? kNeeDims : 0u);
+            if (SKY && __syncthreads_or(surface && sc.env != nullptr)) {
+                mask = 0;
+#pragma unroll 1
+                for (int k = 0; k < trips; ++k) {
+                    if (!surface || (nm && k > 0) || !sc.env) continue;
+                    const unsigned w = nm ? lane : (unsigned)k;
+                    const float lw = lam_of(w);
+                    const unsigned ed0 =
+                        (nm ? base_dim : base_dim + ls_dims * w) + (sc.n_lums > 0 ? kNeeDims : 0u);
+                    float u1, u2;
+                    sample_pair(key, ed0 >> 1, u1, u2);
                     double dd[3], epdf;
-                    env_sample(*sc.env, sample_u(key, ed0), sample_u(key, ed0 + 1), dd, epdf);
-                    ed = mk3((float)dd[0], (float)dd[1], (float)dd[2]);
+                    env_sample(*sc.env, u1, u2, dd, epdf);
+                    const f3 ed = mk3((float)dd[0], (float)dd[1], (float)dd[2]);
                     const float cos_e = dot3(ed, h.n);
-                    if (cos_e > 0.0f && epdf > 0.0) {
-                        const float pe = (float)epdf;
-                        float contrib = sky_radiance(sc.sky, ed, lam[w]) *
-                                        bsdf_value<MAT>(sc, mat, h, ed, lam[w], amb) * cos_e / pe;
-                        const float p_bsdf = bsdf_pdf<MAT>(sc, mat, h, ed, lam[w], amb);
-                        if (p_bsdf > 0.0f) contrib *= power_heuristic(pe, p_bsdf);
-                        ve = nm ? S.thr0[li] * (S.thr[li] * contrib) : S.thr[w * cap + slot] * contrib;
-                        if (ve > 0.0f) {
-                            has_e = true;
-                            eo = offset_ray(h.p, dot3(ed, h.ng) > 0.0f ? h.ng : -h.ng);
-                        }
+                    if (!(cos_e > 0.0f && epdf > 0.0)) continue;
+                    const float pe = (float)epdf;
+                    float contrib = sky_radiance(sc.sky, sky_dir(sc.sky, ed), lw) *
+                                    bsdf_value(sc, mat, bsdf_dir<MAT>(mat, h, ed), lw, amb) * cos_e / pe;
+                    const float p_bsdf = bsdf_pdf<MAT>(sc, mat, h, ed, lw, amb);
+                    if (p_bsdf > 0.0f) contrib *= power_heuristic(pe, p_bsdf);
+                    const float ve = nm ? S.thr0[li] * (S.thr[li] * contrib) : S.thr[w * cap + slot] * contrib;
+                    if (ve > 0.0f) {
+                        mask |= 1u << k;
+                        put(k, ed, INFINITY, ve);
                     }
                 }
-                const unsigned se = push(cnt_sh, has_e);
-                if (has_e)
-                    write_shadow(S, se, eo, ed, INFINITY, ve, (slot * 4u + (unsigned)w) | (kRecEnv << kRecKindShift),
-                                 (unsigned)(mobj + 1));
+                flush(mask, kRecEnv << kRecKindShift);
             }
         }
         // Directional lights (:1968-2000 -> DirectionalLight::ComputeDirectLightingNM,
@@ -1010,7 +1174,8 @@ __global__ __launch_bounds__(kShadeBlock) void k_shade(const ReqInfo* __restrict
         // the light's direction, shadow ray to infinity, no transmittance walk.  A
         // shared ray's four wavelengths share one shadow ray: their values wait in
         // dir_val and the record adds all four.
-        if (blk_dir) {
+        if constexpr (SKY && MAT != kMatDielectric) {
+#pragma unroll 1
             for (int l = 0; l < kMaxDirLights; ++l) {
                 if (!__syncthreads_or(surface && l < sc.n_dir)) break;
                 bool has_d = false;
@@ -1021,13 +1186,15 @@ __global__ __launch_bounds__(kShadeBlock) void k_shade(const ReqInfo* __restrict
                     dd = mk3(L.d[0], L.d[1], L.d[2]);
                     const float cosd = dot3(dd, h.n);
                     if (cosd > 0.0f) {
+                        const BsdfDir<MAT> bd = bsdf_dir<MAT>(mat, h, dd);
                         if (nm) {
-                            vd = S.thr0[li] * (S.thr[li] * (L.le * bsdf_value<MAT>(sc, mat, h, dd, lam[lane], amb) * cosd));
+                            vd = S.thr0[li] * (S.thr[li] * (L.le * bsdf_value(sc, mat, bd, lam_of(lane), amb) * cosd));
                             has_d = vd > 0.0f;
                         } else {
+#pragma unroll 1
                             for (int w = 0; w < kHwss; ++w) {
                                 const float x = S.thr[w * cap + slot] *
-                                                (L.le * bsdf_value<MAT>(sc, mat, h, dd, lam[w], 1.0f) * cosd);
+                                                (L.le * bsdf_value(sc, mat, bd, lam_of((unsigned)w), 1.0f) * cosd);
                                 S.dir_val[l][w * cap + slot] = x;
                                 has_d = has_d || x > 0.0f;
                             }
@@ -1056,13 +1223,14 @@ __global__ __launch_bounds__(kShadeBlock) void k_shade(const ReqInfo* __restrict
                 // Hero ScatterNM, companions at the hero's direction (:4620-4718).
                 float u1, u2, u3;
                 const unsigned rr_dim = bsdf_draws<MAT>(key, base_dim + kHwss * ls_dims, u1, u2, u3);
-                const ScatterOut hs = bsdf_scatter<MAT>(sc, mat, h, lam[0], 1.0f, u1, u2, u3);
+                const ScatterOut hs = bsdf_scatter<MAT>(sc, mat, h, lam0, 1.0f, u1, u2, u3);
                 if (hs.ok) {
                     float thr[kHwss], sc4[kHwss];
                     for (int w = 0; w < kHwss; ++w) thr[w] = S.thr[w * cap + slot];
                     sc4[0] = hs.kray;
+                    const BsdfDir<MAT> bd = bsdf_dir<MAT>(mat, h, hs.dir);
                     for (int w = 1; w < kHwss; ++w) {
-                        float cwt = bsdf_value<MAT>(sc, mat, h, hs.dir, lam[w], 1.0f) * fabsf(dot3(hs.dir, h.n));
+                        float cwt = bsdf_value(sc, mat, bd, lam_of((unsigned)w), 1.0f) * fabsf(dot3(hs.dir, h.n));
                         if (hs.pdf > 0.0f) cwt /= hs.pdf;
                         sc4[w] = cwt > 0.0f ? cwt : 0.0f;
                     }
@@ -1107,7 +1275,7 @@ __global__ __launch_bounds__(kShadeBlock) void k_shade(const ReqInfo* __restrict
                 // IntegrateFromHitNM PART 3 at the lane's wavelength (:2905-3290).
                 float u1, u2, u3;
                 const unsigned rr_dim = bsdf_draws<MAT>(key, base_dim + ls_dims, u1, u2, u3);
-                const ScatterOut so = bsdf_scatter<MAT>(sc, mat, h, lam[lane], amb, u1, u2, u3);
+                const ScatterOut so = bsdf_scatter<MAT>(sc, mat, h, lam_of(lane), amb, u1, u2, u3);
                 float scat = so.kray;
                 bool go = so.ok && fabsf(scat) > kNearZeroF;
                 if (go && depth >= R.rr_min_depth) {
@@ -1134,32 +1302,35 @@ __global__ __launch_bounds__(kShadeBlock) void k_shade(const ReqInfo* __restrict
         } else {
             // A dielectric: for a lane already on its own, and for each wavelength of
             // a shared ray that branches here (:2634-2760; no NEE or RR at this vertex).
-            for (int w = 0; w < kHwss; ++w) {
-                bool cont = false;
+            const int dtrips = __ballot(valid && !nm) != 0ull ? kHwss : 1;
+            unsigned mask = 0;
+#pragma unroll 1
+            for (int k = 0; k < dtrips; ++k) {
+                if (!valid || (nm && k > 0)) continue;
+                const unsigned w = nm ? lane : (unsigned)k, lw = w * cap + slot;
                 f3 nd = mk3(0, 0, 0);
                 float wgt = 0.0f;
                 int type = 0;
                 IorStack nst = ist;
                 unsigned nb = bst;
                 bool dropped = false;
-                if (valid && (!nm || (unsigned)w == lane)) {
-                    if (dielectric_scatter(sc, mat, h, o, lam[w], ist, sample_u(key, base_dim + 2u), nd, wgt, type,
-                                           nst, dropped) &&
-                        bump_bounces(nb, type, R)) {
-                        // A shared ray's wavelength starts its own loop at throughput 1
-                        // (PathTracingIntegrator.cpp:1593), its shared throughput kept aside.
-                        if (!nm) S.thr0[w * cap + slot] = S.thr[w * cap + slot];
-                        const float t = (nm ? S.thr[w * cap + slot] : 1.0f) * wgt;
-                        S.thr[w * cap + slot] = t;
-                        cont = fabsf(t) <= 1e6f;
-                    }
-                }
-                if (cont && dropped) atomicAdd(S.cnt_ovf, 1u);
-                const unsigned qi = push(cnt_next, cont);
-                if (cont)
-                    write_continuation(S, surface_origin(h, nd), slot, (unsigned)w, qout + qi, nd, 0.0f, imp * fabsf(wgt),
-                                       nb, nst, vbn);
+                if (!dielectric_scatter(sc, mat, h, o, lam_of(w), ist, sample_u(key, base_dim + 2u), nd, wgt, type, nst,
+                                        dropped) ||
+                    !bump_bounces(nb, type, R))
+                    continue;
+                // A shared ray's wavelength starts its own loop at throughput 1
+                // (PathTracingIntegrator.cpp:1593), its shared throughput kept aside.
+                if (!nm) S.thr0[lw] = S.thr[lw];
+                const float t = (nm ? S.thr[lw] : 1.0f) * wgt;
+                S.thr[lw] = t;
+                if (!(fabsf(t) <= 1e6f)) continue;
+                if (dropped) atomicAdd(S.cnt_ovf, 1u);
+                mask |= 1u << k;
+                write_lane(S, surface_origin(h, nd), lw, nd, 0.0f, imp * fabsf(wgt), nb, nst, vbn);
             }
+            push4.reserve(cnt_next, mask);
+            for (int k = 0; k < kHwss; ++k)
+                if ((mask >> k) & 1u) qout[push4.pos(k)] = slot * 4u + (nm ? lane : (unsigned)k);
             if (branch) S.flags[slot] |= kModeNm;
         }
     }
@@ -1256,9 +1427,7 @@ __global__ __launch_bounds__(kShadeBlock) void k_volume(const ReqInfo* __restric
             d = mk3(S.dx[li], S.dy[li], S.dz[li]);
             const float tm = S.hit_t[li];
             p = mk3(S.ox[li], S.oy[li], S.oz[li]) + d * tm;
-            float lam[kHwss];
-            wavelengths(S.lambda0[slot], R.lambda_begin, R.lambda_end, lam);
-            nm = lam[lane];
+            nm = wavelength(S.lambda0[slot], R.lambda_begin, R.lambda_end, (int)lane);
             imp = S.imp[li];
             bst = S.state[li];
             vbn = S.vb[li];
@@ -1333,7 +1502,7 @@ __global__ __launch_bounds__(kShadeBlock) void k_volume(const ReqInfo* __restric
                 if (epdf > 0.0) {
                     const float pe = (float)epdf;
                     const float ph = hg_eval(dot3(ed, d), M.g);
-                    float contrib = sky_radiance(sc.sky, ed, nm) * ph / pe;
+                    float contrib = sky_radiance(sc.sky, sky_dir(sc.sky, ed), nm) * ph / pe;
                     if (ph > 0.0f) contrib *= power_heuristic(pe, ph);
                     ve = S.thr0[li] * (thr * contrib);
                     has_e = ve > 0.0f;
@@ -1646,6 +1815,16 @@ __global__ void k_resolve(const ReqInfo* __restrict__ reqs, int req)
     }
 }
 
+}  // namespace
+
+hipError_t rise_hip::fill_ggx_favg(float* out, const float* amp, int ior_offset, int n_ior, int ext_offset, int n_ext)
+{
+    hipLaunchKernelGGL(k_ggx_favg, dim3(64), dim3(256), 0, nullptr, out, amp, ior_offset, n_ior, ext_offset, n_ext);
+    return hipGetLastError();
+}
+
+namespace {
+
 size_t align_up(size_t x) { return (x + 255) & ~size_t(255); }
 
 // Carves the path pool for `cap` paths plus `passes` counter blocks from
@@ -1779,6 +1958,9 @@ void choose_traversal(const rise_hip_batch_tuning& tn, int depth, int64_t max_tr
         gc = grid_for(4 * cap, block, 8192);
     }
 }
+
+// Whether the scene needs the kernels' sky variants.
+bool has_sky_light(const PtSceneView& v) { return v.sky.on || v.env != nullptr || v.n_dir > 0; }
 
 rise_hip_status validate(const rise_hip_render_request& q, size_t k)
 {
@@ -1940,6 +2122,7 @@ struct rise_hip_batch {
     TraceKernel ext_fn = nullptr, con_fn = nullptr;
     unsigned grid_ext = 1, grid_con = 1;  // workgroups of the traversal kernels
     unsigned mat_mask = 0;                // material kinds present in the batch's scenes
+    bool sky = false;                     // some scene has a sky or directional lights
     int64_t cap = 0;                   // path pool size
     std::vector<rise_hip_render_request> requests;
     std::vector<PassEntry> entries;    // all passes, concatenated
@@ -2010,7 +2193,7 @@ rise_hip_status plan(rise_hip_batch* b, const rise_hip_render_request* reqs, siz
     int bounces = 1, depth = 1;
     int64_t max_tris = 0;
     unsigned mat_mask = 0;
-    bool has_media = false, has_env = false;
+    bool has_media = false, has_env = false, has_sky = false;
     int n_dir = 0;
     std::vector<int64_t> req_px(n, 0);
     size_t film_floats = 0;
@@ -2035,6 +2218,7 @@ rise_hip_status plan(rise_hip_batch* b, const rise_hip_render_request* reqs, siz
         mat_mask |= reqs[k].scene->material_kinds | (sc->has_media ? 1u << kMatVolume : 0u);
         has_media = has_media || sc->has_media;
         has_env = has_env || sc->view.env != nullptr;
+        has_sky = has_sky || has_sky_light(sc->view);
         n_dir = std::max(n_dir, sc->view.n_dir);
         max_tris = std::max<int64_t>(max_tris, reqs[k].scene->n_tris);
         film_floats += 12 * (size_t)req_px[k];
@@ -2105,6 +2289,7 @@ rise_hip_status plan(rise_hip_batch* b, const rise_hip_render_request* reqs, siz
                      b->grid_ext, b->grid_con);
     b->bounces = bounces;
     b->mat_mask = mat_mask;
+    b->sky = has_sky;
     b->n_req = (int)n;
     b->requests.assign(reqs, reqs + n);
     b->launched = false;
@@ -2119,6 +2304,7 @@ struct PassShape {
     int64_t cap;
     int bounces;
     unsigned mat_mask;
+    bool sky;  // some scene has a sky or directional lights
 };
 
 // Kernels of one pass over `n_ent` chunks at `ent` (paths and film threads
@@ -2135,13 +2321,18 @@ void launch_pass(const ReqInfo* d_info, Paths S, const PassEntry* ent, int n_ent
     for (int d = 0; d < sh.bounces; ++d) {
         void* args[] = {(void*)&d_info, &S, &d};
         hipLaunchKernel((const void*)sh.ext_fn, dim3(sh.ge), dim3(sh.block), args, 0, stream);
-        hipLaunchKernelGGL(k_bin, dim3(gs), dim3(kShadeBlock), 0, stream, d_info, S, d);
-        if (sh.mat_mask & (1u << kMatLambert))
-            hipLaunchKernelGGL(k_shade<kMatLambert>, dim3(gs), dim3(kShadeBlock), 0, stream, d_info, S, d);
-        if (sh.mat_mask & (1u << kMatGgx))
-            hipLaunchKernelGGL(k_shade<kMatGgx>, dim3(gs), dim3(kShadeBlock), 0, stream, d_info, S, d);
+#define RISE_LAUNCH_SHADE(K, KIND)                                                                     \
+    if (sh.mat_mask & (1u << (KIND))) {                                                                \
+        if (sh.sky) hipLaunchKernelGGL((K<KIND, true>), dim3(gs), dim3(kShadeBlock), 0, stream, d_info, S, d); \
+        else hipLaunchKernelGGL((K<KIND, false>), dim3(gs), dim3(kShadeBlock), 0, stream, d_info, S, d); \
+    }
+        if (sh.sky) hipLaunchKernelGGL(k_bin<true>, dim3(gs), dim3(kShadeBlock), 0, stream, d_info, S, d);
+        else hipLaunchKernelGGL(k_bin<false>, dim3(gs), dim3(kShadeBlock), 0, stream, d_info, S, d);
+        RISE_LAUNCH_SHADE(k_shade, kMatLambert)
+        RISE_LAUNCH_SHADE(k_shade, kMatGgx)
         if (sh.mat_mask & (1u << kMatDielectric))
-            hipLaunchKernelGGL(k_shade<kMatDielectric>, dim3(gs), dim3(kShadeBlock), 0, stream, d_info, S, d);
+            hipLaunchKernelGGL((k_shade<kMatDielectric, false>), dim3(gs), dim3(kShadeBlock), 0, stream, d_info, S, d);
+#undef RISE_LAUNCH_SHADE
         if (sh.mat_mask & (1u << kMatVolume))
             hipLaunchKernelGGL(k_volume, dim3(gs), dim3(kShadeBlock), 0, stream, d_info, S, d);
         hipLaunchKernel((const void*)sh.con_fn, dim3(sh.gc), dim3(sh.block), args, 0, stream);
@@ -2166,7 +2357,7 @@ hipError_t launch(rise_hip_batch* b, hipStream_t stream)
     hipLaunchKernelGGL(k_fill, dim3(grid_for((int64_t)b->film_floats, 256, 4096)), dim3(256), 0, stream, b->d_film,
                        b->film_floats);
     const PassShape sh{b->ext_fn, b->con_fn, b->grid_ext, b->grid_con, (unsigned)b->trace_block,
-                       b->cap,    b->bounces, b->mat_mask};
+                       b->cap,    b->bounces, b->mat_mask, b->sky};
     const int passes = (int)b->pass_paths.size();
     for (int p = 0; p < passes; ++p) {
         const Paths S = pass_counters(b->S, b->counters + (size_t)p * kCounters);
@@ -2346,6 +2537,7 @@ struct ServerReq {
     int depth = 1;                 // tree depth of its scene
     int64_t tris = 0;
     unsigned kinds = 0;
+    bool sky = false;              // its scene has a sky or directional lights
 };
 
 int64_t now_ns()
@@ -2503,6 +2695,7 @@ rise_hip_status server_admit(rise_hip_server* sv)
         ReqInfo info;
         rise_hip_status st = make_info(r.q, info);
         if (st != RISE_HIP_OK) return st;
+        r.sky = has_sky_light(info.sc);
         hipError_t e;
         if (sv->inject_alloc_failures > 0) {
             --sv->inject_alloc_failures;
@@ -2553,6 +2746,7 @@ rise_hip_status server_launch(rise_hip_server* sv)
         int64_t paths = 0, film = 0, tris = 0;
         int bounces = 1, depth = 1;
         unsigned kinds = 0;
+        bool sky = false;
         std::vector<ServerReq*> finishing;
         std::vector<PassSource> src;
         src.reserve(sv->active.size());
@@ -2572,6 +2766,7 @@ rise_hip_status server_launch(rise_hip_server* sv)
             depth = std::max(depth, r.depth);
             tris = std::max(tris, r.tris);
             kinds |= r.kinds;
+            sky = sky || r.sky;
             if (r.next == r.chunks.size()) finishing.push_back(&r);
         }
         PassShape sh{};
@@ -2582,6 +2777,7 @@ rise_hip_status server_launch(rise_hip_server* sv)
         sh.cap = sv->cap;
         sh.bounces = bounces;
         sh.mat_mask = kinds;
+        sh.sky = sky;
         PassEntry* d_ent = sv->d_ent + (size_t)k * kPassEntries;
         hipError_t e = hipMemcpyAsync(d_ent, ent, (size_t)n_ent * sizeof(PassEntry), hipMemcpyHostToDevice, sv->stream);
         if (e != hipSuccess) return fail_hip(e, "pass table");

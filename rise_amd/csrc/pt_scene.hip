@@ -40,6 +40,27 @@ rise_hip_status upload(rise_hip_pt_scene* s, const std::vector<T>& v, const T** 
     return RISE_HIP_OK;
 }
 
+// The Fresnel averages of the materials that have a table (DevMaterial::favg).
+rise_hip_status fill_favg(rise_hip_pt_scene* s, const std::vector<DevMaterial>& mats, const std::vector<DevSpd>& spds,
+                          size_t n)
+{
+    float* out = nullptr;
+    hipError_t e = hipMalloc((void**)&out, n * sizeof(float));
+    if (e != hipSuccess) return fail_hip(e, "hipMalloc (scene)");
+    s->allocs.push_back(out);
+    for (const DevMaterial& m : mats) {
+        if (e != hipSuccess || m.favg < 0) continue;
+        const bool has_n = m.ior_spd >= 0, has_k = m.ext_spd >= 0;
+        e = fill_ggx_favg(out + m.favg, s->view.spd_amp, has_n ? spds[(size_t)m.ior_spd].offset : -1,
+                          has_n ? spds[(size_t)m.ior_spd].n : 0, has_k ? spds[(size_t)m.ext_spd].offset : -1,
+                          has_k ? spds[(size_t)m.ext_spd].n : 0);
+    }
+    if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
+    if (e != hipSuccess) return fail_hip(e, "Fresnel averages");
+    s->view.ggx_favg = out;
+    return RISE_HIP_OK;
+}
+
 void free_scene(rise_hip_pt_scene* s)
 {
     release_solo_batch(s);
@@ -155,10 +176,25 @@ rise_hip_status rise_hip::pt_scene_create(const rise_hip_object_desc* objects, s
         if (m.type == RISE_HIP_MATERIAL_GGX && !(m.alpha >= 0.0f))
             return fail(RISE_HIP_ERR_INVALID_ARGUMENT, who + "negative or NaN roughness");
         dmat[i] = DevMaterial{m.type,        m.reflectance_spd, m.emission_spd,    m.emission_scale,
-                              m.specular_spd, m.ior_spd,         m.extinction_spd, m.alpha};
+                              m.specular_spd, m.ior_spd,         m.extinction_spd, m.alpha,
+                              -1,             0,                 {0, 0}};
         material_kinds |= 1u << m.type;
         if (m.type == RISE_HIP_MATERIAL_GGX) has_glossy = true;
         if (m.type == RISE_HIP_MATERIAL_DIELECTRIC) has_glossy = has_transmission = true;
+    }
+    // Tables of the GGX materials' Fresnel averages, where both spectra are steps
+    // (or absent) and the pairs of their values few.
+    constexpr int64_t kMaxFavgPairs = 1 << 16, kMaxFavg = 1 << 20;
+    int64_t n_favg = 0;
+    for (DevMaterial& m : dmat) {
+        if (m.type != RISE_HIP_MATERIAL_GGX) continue;
+        const int64_t rows = m.ior_spd < 0 ? 1 : (int64_t)dspd[(size_t)m.ior_spd].n + 1;
+        const int64_t cols = m.ext_spd < 0 ? 1 : (int64_t)dspd[(size_t)m.ext_spd].n + 1;
+        if (rows < 1 || cols < 1) continue;  // a sigmoid spectrum
+        if (rows > kMaxFavgPairs / cols || n_favg + rows * cols > kMaxFavg) continue;
+        m.favg = (int)n_favg;
+        m.favg_stride = (int)cols;
+        n_favg += rows * cols;
     }
     // Objects -> one triangle list.
     int64_t total = 0;
@@ -326,6 +362,7 @@ rise_hip_status rise_hip::pt_scene_create(const rise_hip_object_desc* objects, s
     if (st == RISE_HIP_OK) st = upload(s, dmat, &v.materials);
     if (st == RISE_HIP_OK) st = upload(s, dspd, &v.spds);
     if (st == RISE_HIP_OK) st = upload(s, amps, &v.spd_amp);
+    if (st == RISE_HIP_OK && n_favg > 0) st = fill_favg(s, dmat, dspd, (size_t)n_favg);
     if (st == RISE_HIP_OK) st = upload(s, lums, &v.lums);
     if (st == RISE_HIP_OK) st = upload(s, lum_tris, &v.lum_tris);
     if (st == RISE_HIP_OK) st = upload(s, lum_cdf, &v.lum_cdf);
