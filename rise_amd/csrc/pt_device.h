@@ -318,19 +318,23 @@ RISE_HD inline int spd_bin(const DevSpd& d, float nm)
     return idx;
 }
 
+// Sigmoid-polynomial spectrum (RGBSigmoidPolynomial::Eval): amplitudes hold
+// c0, c1, c2 and a scale; the range is [380, 780] nm.  Called, not inlined: the
+// kernels read a spectrum in some twenty places, and their code has to stay
+// within the 64 KB instruction cache.
+__attribute__((noinline)) RISE_HD inline float sigmoid_spectrum(const float* c, float nm)
+{
+    const float t = (nm - 380.0f) * (1.0f / 400.0f);
+    const float x = (c[0] * t + c[1]) * t + c[2];
+    return c[3] * (0.5f + x / (2.0f * sqrtf(1.0f + x * x)));
+}
+
 // SpectralPacket::ValueAtNM (Utilities/Color/SpectralPacket.h:285-297).
 RISE_HD inline float spd_value(const PtSceneView& s, int spd, float nm)
 {
     const DevSpd d = s.spds[spd];
     if (nm < d.begin || nm > d.end) return 0.0f;
-    if (d.n < 0) {
-        // Sigmoid-polynomial spectrum (RGBSigmoidPolynomial::Eval): amplitudes
-        // hold c0, c1, c2 and a scale; the range is [380, 780] nm.
-        const float* c = s.spd_amp + d.offset;
-        const float t = (nm - 380.0f) * (1.0f / 400.0f);
-        const float x = (c[0] * t + c[1]) * t + c[2];
-        return c[3] * (0.5f + x / (2.0f * sqrtf(1.0f + x * x)));
-    }
+    if (d.n < 0) return sigmoid_spectrum(s.spd_amp + d.offset, nm);
     return s.spd_amp[d.offset + spd_bin(d, nm)];
 }
 

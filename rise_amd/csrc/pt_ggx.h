@@ -66,8 +66,6 @@ RISE_HD inline float ggx_lambda(float a, f3 v)
     return (-1.0f + sqrtf(1.0f + a2 / vz2)) * 0.5f;
 }
 
-RISE_HD inline float ggx_g1(float a, f3 v) { return 1.0f / (1.0f + ggx_lambda(a, v)); }
-RISE_HD inline float ggx_g2(float a, f3 wi, f3 wo) { return 1.0f / (1.0f + ggx_lambda(a, wi) + ggx_lambda(a, wo)); }
 
 RISE_HD inline float ggx_d(float a, f3 h)
 {
@@ -92,19 +90,6 @@ RISE_HD inline f3 vndf_sample(f3 wi, const Onb& b, float a, float u1, float u2)
     const f3 c = mk3(st * cosf(phi) + wh.x, st * sinf(phi) + wh.y, z + wh.z);
     const f3 ml = norm3(mk3(a * c.x, a * c.y, c.z));
     return norm3(b.u * ml.x + b.v * ml.y + b.w * ml.z);
-}
-
-RISE_HD inline float vndf_pdf(f3 wi, f3 wo, const Onb& b, float a)
-{
-    if (a < 1e-6f) return 0.0f;
-    const float cos_wi = dot3(wi, b.w);
-    if (cos_wi < 1e-10f) return 0.0f;
-    const f3 h = norm3(wi + wo);
-    const float wih = dot3(wi, h), woh = dot3(wo, h);
-    if (wih <= 0.0f || woh < 1e-10f) return 0.0f;
-    const f3 hl = to_local(b, h);
-    if (hl.z <= 0.0f) return 0.0f;
-    return ggx_g1(a, to_local(b, wi)) * wih * ggx_d(a, hl) / cos_wi / (4.0f * woh);
 }
 
 // ---- energy tables (MicrofacetEnergyLUT.h) ----------------------------------
@@ -235,7 +220,8 @@ RISE_HD inline float fresnel_conductor(float cos_i, float ni, float nt, float kt
     return 0.5f * (rp + rs);
 }
 
-RISE_HD inline float fresnel_avg(const GgxTables& T, float ni, float nt, float kt)
+// Called, not inlined: rare (ggx_favg's table serves most vertices).
+__attribute__((noinline)) RISE_HD inline float fresnel_avg(const GgxTables& T, float ni, float nt, float kt)
 {
     float sum = 0.0f;
 #pragma unroll 1
@@ -255,55 +241,102 @@ struct GgxParams {
     float rd, rs, alpha, ior, ext, amb;
 };
 
-// Ray-facing ONB (FlipW) and geometric normal oriented against the ray.
-RISE_HD inline void ggx_facing(const Surf& h, Onb& b, f3& gn)
-{
-    b = h.frame;
-    if (dot3(h.dir, h.frame.w) > kNearZeroF) {
-        b.w = -b.w;
-        b.u = -b.u;
-    }
-    const f3 raw = dot3(h.ng, h.ng) > 1e-12f ? h.ng : b.w;
-    gn = dot3(raw, h.dir) < 0.0f ? raw : -raw;
-}
-
-// GGXBRDF::valueNM (GGXBRDF.cpp:339-498), conductor Fresnel, in two parts:
-// what depends on the directions alone, and the value at one wavelength.
-struct GgxDir {
-    bool ok;
-    bool ms;        // the multiscatter lobe counts
-    float sf;       // D G2 / (4 cos cos)
-    float shape;    // multiscatter lobe over its Fresnel factor
-    float cos_h;    // cosine of the Fresnel term
-    float eavg;
-};
-
-RISE_HD inline GgxDir ggx_dir(const GgxTables& T, const Surf& h, float alpha, f3 vin)
-{
-    GgxDir d{false, false, 0.0f, 0.0f, 0.0f, 0.0f};
+// What a GGX vertex's evaluations share: the ray-facing ONB (FlipW), the
+// geometric normal oriented against the ray, the direction back along the ray
+// and its terms, the energy tables at the roughness.
+struct GgxVertex {
     Onb b;
     f3 gn;
-    ggx_facing(h, b, gn);
-    const f3 n = b.w, v = norm3(vin), r = norm3(-h.dir);
-    const float nr = dot3(n, r), nv = dot3(n, v);
-    if (nr < kNearZeroF || nv < kNearZeroF) return d;
-    if (dot3(v, gn) <= 0.0f || dot3(r, gn) <= 0.0f) return d;
-    const float a = fmaxf(alpha, 1e-4f);
-    const f3 hv = norm3(v + r);
-    d.ok = true;
-    d.sf = ggx_d(a, to_local(b, hv)) * ggx_g2(a, to_local(b, v), to_local(b, r)) / (4.0f * nv * nr);
-    d.cos_h = dot3(h.dir, hv);
-    d.eavg = lookup_eavg(T, a);
-    if (1.0f - d.eavg > 1e-10f) {
-        d.ms = true;
-        d.shape = (1.0f - lookup_ess(T, nr, a)) * (1.0f - lookup_ess(T, nv, a)) /
-                  (3.14159265358979f * (1.0f - d.eavg));
+    f3 r;          // unit, toward the ray's origin
+    float a;       // roughness, at least 1e-4
+    float nr;      // cosine of r
+    float lam_r;   // Smith lambda of r
+    float ess_r;   // directional albedo at r
+    float eavg, z;
+};
+
+RISE_HD inline GgxVertex ggx_vertex(const GgxTables& T, const Surf& h, float alpha)
+{
+    GgxVertex V;
+    V.b = h.frame;
+    if (dot3(h.dir, h.frame.w) > kNearZeroF) {
+        V.b.w = -V.b.w;
+        V.b.u = -V.b.u;
+    }
+    const f3 raw = dot3(h.ng, h.ng) > 1e-12f ? h.ng : V.b.w;
+    V.gn = dot3(raw, h.dir) < 0.0f ? raw : -raw;
+    V.r = norm3(-h.dir);
+    V.a = fmaxf(alpha, 1e-4f);
+    V.nr = dot3(V.b.w, V.r);
+    V.lam_r = ggx_lambda(V.a, to_local(V.b, V.r));
+    V.ess_r = lookup_ess(T, V.nr, V.a);
+    V.eavg = lookup_eavg(T, V.a);
+    V.z = ms_z(T, V.a);
+    return V;
+}
+
+// The VNDF's pdf of reflecting into wo with half vector h (MicrofacetUtils.h).
+RISE_HD inline float vndf_pdf(const GgxVertex& V, f3 wo, f3 h, float d)
+{
+    if (V.nr < 1e-10f) return 0.0f;
+    const float wih = dot3(V.r, h), woh = dot3(wo, h);
+    if (wih <= 0.0f || woh < 1e-10f) return 0.0f;
+    if (dot3(h, V.b.w) <= 0.0f) return 0.0f;
+    return 1.0f / (1.0f + V.lam_r) * wih * d / V.nr / (4.0f * woh);
+}
+RISE_HD inline float vndf_pdf(const GgxVertex& V, f3 wo)
+{
+    const f3 h = norm3(V.r + wo);
+    return vndf_pdf(V, wo, h, ggx_d(V.a, to_local(V.b, h)));
+}
+
+// A direction's part of GGXBRDF::valueNM (GGXBRDF.cpp:339-498, conductor
+// Fresnel) and of GGXSPF::PdfNM (GGXSPF.cpp:740-790): all but the material's
+// values at the wavelength.
+struct GgxDir {
+    bool ok;          // the value is not 0
+    bool pdf_ok;      // the pdf is not 0
+    bool ms;          // the multiscatter lobe counts
+    float sf;         // D G2 / (4 cos cos)
+    float shape;      // multiscatter lobe over its Fresnel factor
+    float cos_h;      // cosine of the Fresnel term
+    float ct;         // cosine
+    float spec_pdf;   // VNDF pdf
+    float multi_pdf;  // multiscatter lobe's pdf
+};
+
+// PDF: the pdf's part too.
+template <bool PDF>
+RISE_HD inline GgxDir ggx_dir(const GgxTables& T, const Surf& h, const GgxVertex& V, f3 vin)
+{
+    GgxDir d{};
+    const f3 v = norm3(vin);
+    d.ct = dot3(V.b.w, v);
+    if (!(dot3(v, V.gn) > 0.0f)) return d;
+    d.ok = !(V.nr < kNearZeroF || d.ct < kNearZeroF) && dot3(V.r, V.gn) > 0.0f;
+    d.pdf_ok = PDF && d.ct > 0.0f;
+    if (!d.ok && !d.pdf_ok) return d;
+    const f3 hv = norm3(v + V.r);
+    const float dd = ggx_d(V.a, to_local(V.b, hv));
+    if (d.ok) {
+        const float g2 = 1.0f / (1.0f + ggx_lambda(V.a, to_local(V.b, v)) + V.lam_r);
+        d.sf = dd * g2 / (4.0f * d.ct * V.nr);
+        d.cos_h = dot3(h.dir, hv);
+        if (1.0f - V.eavg > 1e-10f) {
+            d.ms = true;
+            d.shape = (1.0f - V.ess_r) * (1.0f - lookup_ess(T, d.ct, V.a)) /
+                      (3.14159265358979f * (1.0f - V.eavg));
+        }
+    }
+    if (d.pdf_ok) {
+        d.spec_pdf = vndf_pdf(V, v, hv, dd);
+        d.multi_pdf = ms_pdf(T, d.ct, V.a, V.z);
     }
     return d;
 }
 
 // f_avg: the hemispherical Fresnel average at (g.amb, g.ior, g.ext).
-RISE_HD inline float ggx_value(const GgxDir& d, const GgxParams& g, float f_avg)
+RISE_HD inline float ggx_value(const GgxVertex& V, const GgxDir& d, const GgxParams& g, float f_avg)
 {
     if (!d.ok) return 0.0f;
     float spec = 0.0f;
@@ -311,26 +344,17 @@ RISE_HD inline float ggx_value(const GgxDir& d, const GgxParams& g, float f_avg)
         const float f = fresnel_conductor(d.cos_h, g.amb, g.ior, g.ext);
         if (f > 0.0f) spec = g.rs * f * d.sf;
     }
-    if (d.ms) spec += ggx_fms(g.rs * f_avg, d.eavg) * d.shape;
+    if (d.ms) spec += ggx_fms(g.rs * f_avg, V.eavg) * d.shape;
     return g.rd * kInvPi + spec;
 }
 
-// GGXSPF::PdfNM (GGXSPF.cpp:740-790).
-RISE_HD inline float ggx_pdf(const GgxTables& T, const Surf& h, const GgxParams& g, f3 wo)
+RISE_HD inline float ggx_pdf(const GgxVertex& V, const GgxDir& d, const GgxParams& g)
 {
-    Onb b;
-    f3 gn;
-    ggx_facing(h, b, gn);
-    const f3 n = b.w, won = norm3(wo);
-    const float ct = dot3(won, n);
-    if (ct <= 0.0f || dot3(won, gn) <= 0.0f) return 0.0f;
-    const f3 wi = norm3(-h.dir);
-    const float a = fmaxf(g.alpha, 1e-4f);
-    const float wms = g.rs * (1.0f - lookup_ess(T, dot3(wi, n), a));
+    if (!d.pdf_ok) return 0.0f;
+    const float wms = g.rs * (1.0f - V.ess_r);
     const float total = g.rd + g.rs + wms;
-    if (total < 1e-10f) return ct * kInvPi;
-    const float spec_pdf = a >= 1e-6f ? vndf_pdf(wi, won, b, a) : 0.0f;
-    return (g.rd * ct * kInvPi + wms * ms_pdf(T, ct, a, ms_z(T, a)) + g.rs * spec_pdf) / total;
+    if (total < 1e-10f) return d.ct * kInvPi;
+    return (g.rd * d.ct * kInvPi + wms * d.multi_pdf + g.rs * d.spec_pdf) / total;
 }
 
 struct ScatterOut {
@@ -346,20 +370,15 @@ struct ScatterOut {
 // f_avg() gives the Fresnel average at (g.amb, g.ior, g.ext), which only the
 // multiscatter lobe needs.
 template <class Favg>
-RISE_HD inline ScatterOut ggx_scatter(const GgxTables& T, const Surf& h, const GgxParams& g, float u_lobe, float u1,
-                                      float u2, Favg f_avg)
+RISE_HD inline ScatterOut ggx_scatter(const GgxTables& T, const Surf& h, const GgxVertex& V, const GgxParams& g,
+                                      float u_lobe, float u1, float u2, Favg f_avg)
 {
     ScatterOut out{false, mk3(0, 0, 0), 0.0f, 0.0f, 0};
-    Onb b;
-    f3 gn;
-    ggx_facing(h, b, gn);
-    const f3 n = b.w, wi = norm3(-h.dir);
-    const float a = fmaxf(g.alpha, 1e-4f);
-    const float eavg = lookup_eavg(T, a);
-    const float ess_i = lookup_ess(T, dot3(wi, n), a);
+    const Onb& b = V.b;
+    const f3 gn = V.gn, n = b.w, wi = V.r;
+    const float a = V.a, eavg = V.eavg, ess_i = V.ess_r, z = V.z;
     const float wd = g.rd, ws = g.rs, wms = ws * (1.0f - ess_i);
     const float total = wd + ws + wms;
-    const float z = ms_z(T, a);
     const float p_diff = total > 1e-10f ? wd / total : 1.0f;
     const float p_spec = total > 1e-10f ? ws / total : 0.0f;
     auto mix = [&](float ct, float spec_pdf, float fallback) {
@@ -370,25 +389,23 @@ RISE_HD inline ScatterOut ggx_scatter(const GgxTables& T, const Surf& h, const G
         const f3 wo = onb_xform(b, mk3(cosf(phi) * st, sinf(phi) * st, ctt));
         const float ct = dot3(wo, n);
         if (ct > 0.0f && dot3(wo, gn) > 0.0f) {
-            const float sp = a >= 1e-6f ? vndf_pdf(wi, wo, b, a) : 0.0f;
+            const float sp = vndf_pdf(V, wo);
             out = ScatterOut{true, wo, wd / p_diff, mix(ct, sp, ct * kInvPi), 0};
         }
     } else if (u_lobe < p_diff + p_spec) {
-        if (a >= 1e-6f) {
-            const f3 m = vndf_sample(wi, b, a, u1, u2);
-            const float wim = dot3(wi, m);
-            if (wim > 0.0f) {
-                const f3 wo = norm3(m * (2.0f * wim) - wi);
-                const float ct = dot3(wo, n);
-                if (ct > 0.0f && dot3(wo, gn) > 0.0f) {
-                    const float vp = vndf_pdf(wi, wo, b, a);
-                    if (vp > 1e-10f) {
-                        const float F = g.rs * fresnel_conductor(dot3(h.dir, m), g.amb, g.ior, g.ext);
-                        const float G1 = ggx_g1(a, to_local(b, wi));
-                        const float kray = G1 > 1e-10f ? F * ggx_g2(a, to_local(b, wi), to_local(b, wo)) / (G1 * p_spec)
-                                                       : 0.0f;
-                        if (kray > 0.0f) out = ScatterOut{true, wo, kray, mix(ct, vp, vp), 1};
-                    }
+        const f3 m = vndf_sample(wi, b, a, u1, u2);
+        const float wim = dot3(wi, m);
+        if (wim > 0.0f) {
+            const f3 wo = norm3(m * (2.0f * wim) - wi);
+            const float ct = dot3(wo, n);
+            if (ct > 0.0f && dot3(wo, gn) > 0.0f) {
+                const float vp = vndf_pdf(V, wo);
+                if (vp > 1e-10f) {
+                    const float F = g.rs * fresnel_conductor(dot3(h.dir, m), g.amb, g.ior, g.ext);
+                    const float G1 = 1.0f / (1.0f + V.lam_r);
+                    const float G2 = 1.0f / (1.0f + V.lam_r + ggx_lambda(a, to_local(b, wo)));
+                    const float kray = G1 > 1e-10f ? F * G2 / (G1 * p_spec) : 0.0f;
+                    if (kray > 0.0f) out = ScatterOut{true, wo, kray, mix(ct, vp, vp), 1};
                 }
             }
         }
@@ -400,7 +417,7 @@ RISE_HD inline ScatterOut ggx_scatter(const GgxTables& T, const Surf& h, const G
             const float phi = kTwoPi * u2;
             const f3 wo = onb_xform(b, mk3(st * cosf(phi), st * sinf(phi), ct));
             if (ct > 0.0f && dot3(wo, gn) > 0.0f) {
-                const float sp = a >= 1e-6f ? vndf_pdf(wi, wo, b, a) : 0.0f;
+                const float sp = vndf_pdf(V, wo);
                 const float mp = ms_pdf(T, ct, a, z);
                 const float fms = ggx_fms(g.rs * f_avg(), eavg);
                 const float f_ms = fms * (1.0f - lookup_ess(T, ct, a)) * (1.0f - ess_i) * kInvPi / (1.0f - eavg);

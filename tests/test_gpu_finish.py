@@ -1,0 +1,92 @@
+"""Passes at the edges of k_finish, the launch that runs a small pass, or the
+last bounces of a large one, by itself: path counts around one workgroup's
+share and the resident workgroups' shares, both sides of the size from which
+the first bounces are separate launches, and scenes with and without a sky,
+conductors, glass and media.  The film of a request rendered as several sample
+ranges, each another pass size, is the sum of its samples whatever kernels ran
+them: parts rendered alone equal the same parts in one batch bit for bit, and
+the film of a small pass equals the same paths inside a large one.  A tree too
+deep for that launch's stack takes the separate launches, with the same film."""
+import dataclasses
+
+import numpy as np
+import pytest
+import torch
+
+from rise_amd import pt_scene, raycast, scenes
+from rise_amd.render import PathTracingSpectralRasterizer, RenderBatch
+from tests.conftest import log_case
+
+pytestmark = pytest.mark.gpu
+
+SCENES = {
+    "cornell": pt_scene.cornell_box,
+    "fog": pt_scene.cornell_fog,
+    "materials": pt_scene.cornell_materials,
+    "sky": lambda: pt_scene.sky_spheres(4),
+    "cloud": lambda: pt_scene.cloud_cornell(3, 20000),
+}
+
+
+@pytest.mark.parametrize("name", sorted(SCENES))
+def test_gpu_finish_pass_sizes(cuda, name):
+    s, r = SCENES[name]()
+    rast = PathTracingSpectralRasterizer(s)
+    # A large companion makes the batch's pass run its first bounces separately.
+    big = dataclasses.replace(r, width=512, height=512, spp=1, seed=99)
+    sizes = [(1, 1, 1), (5, 3, 1), (17, 1, 1), (16, 16, 1), (33, 31, 1), (67, 61, 2), (128, 128, 1), (362, 362, 1)]
+    small = [dataclasses.replace(r, width=w, height=h, spp=n, seed=7 + k) for k, (w, h, n) in enumerate(sizes)]
+    alone, stats = [], []
+    for q in small:
+        log_case(f"{name} {q.width}x{q.height}x{q.spp} alone")
+        film, sq, st = rast.rasterize_scene(q, want_sq=True)
+        alone.append((film.cpu().numpy(), sq.cpu().numpy()))
+        stats.append(st)
+    log_case(f"{name} batch with 512x512")
+    b = RenderBatch([(rast, q) for q in small] + [(rast, big)], want_sq=True)
+    b.launch()
+    torch.cuda.synchronize()
+    for k, (f, q) in enumerate(alone):
+        assert np.array_equal(b.films[k].cpu().numpy(), f), sizes[k]
+        assert np.array_equal(b.films_sq[k].cpu().numpy(), q), sizes[k]
+    film, _, st = rast.rasterize_scene(big)
+    assert np.array_equal(b.films[-1].cpu().numpy(), film.cpu().numpy())
+    # Ray counts do not depend on which launches traced them.
+    total = b.stats()
+    for key in ("extension_rays", "shadow_rays", "paths"):
+        assert total[key] == st[key] + sum(x[key] for x in stats), key
+    b.release()
+    rast.release()
+
+
+def deep_scene():
+    """Triangles at 150 geometric scales about a point, a light above: more levels than k_finish has room for."""
+    s, r = pt_scene.cornell_box()
+    g = np.random.default_rng(1)
+    scale = 0.6 * 1.3 ** -np.arange(150.0).repeat(20)[:, None]
+    c = scale * g.uniform(0.7, 1.0, (len(scale), 3))
+    e1, e2 = g.normal(0, 0.1, (2, len(scale), 3)) * scale
+    s.objects = [pt_scene.Object(np.concatenate([c, c + e1, c + e2], 1).astype(np.float32), 0, double_sided=True),
+                 pt_scene.Object(pt_scene.quad((0, 0.7, 0), (0.6, 0.7, 0), (0.6, 0.7, 0.6), (0, 0.7, 0.6)), 3)]
+    s.camera = dataclasses.replace(s.camera, position=(1.5, 0.5, 1.5), look_at=(0.2, 0.2, 0.2))
+    return s, r
+
+
+def test_gpu_finish_deep_tree(cuda):
+    scene = deep_scene()[0]
+    world = np.concatenate([o.tris for o in scene.objects]).astype(np.float32)
+    deep = PathTracingSpectralRasterizer(scene)
+    s, r = pt_scene.cornell_box()
+    flat = PathTracingSpectralRasterizer(s)
+    q = dataclasses.replace(r, width=37, height=29, spp=2, seed=5)
+    assert raycast.host_trace(world, scenes.incoherent_rays(8, 1))[3]["depth"] > 17
+    log_case("deep alone, flat alone, both")
+    a = [x.rasterize_scene(q)[0].cpu().numpy() for x in (deep, flat)]
+    b = RenderBatch([(deep, q), (flat, q)])
+    b.launch()
+    torch.cuda.synchronize()
+    for k in range(2):
+        assert a[k].any() and np.array_equal(b.films[k].cpu().numpy(), a[k])
+    b.release()
+    deep.release()
+    flat.release()
