@@ -76,7 +76,7 @@ __global__ __launch_bounds__(kObjBlock) void closest_objects(ObjectSceneView sc,
     __shared__ uint2 lds[STACK > 0 ? kObjLds * kObjBlock : 1];
     auto st = make_stack<STACK>(lds);
     ObjClosestQuery<A> Q;
-    ItemFetch fetch(next, n);
+    ItemFetch fetch(grid_items(next, n));
     long long ray = -1;
     bool busy = false;
     for (;;) {
@@ -130,7 +130,7 @@ __global__ __launch_bounds__(kObjBlock) void any_objects(ObjectSceneView sc, con
     __shared__ uint2 lds[STACK > 0 ? kObjLds * kObjBlock : 1];
     auto st = make_stack<STACK>(lds);
     ObjAnyQuery<A> Q;
-    ItemFetch fetch(next, n);
+    ItemFetch fetch(grid_items(next, n));
     long long ray = -1;
     bool busy = false;
     for (;;) {

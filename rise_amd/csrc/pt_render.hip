@@ -424,29 +424,16 @@ __device__ inline void extend_entry(const ReqInfo* __restrict__ reqs, const Path
     S.hit_t[slot] = id >= 0 ? (float)best : 0.0f;
 }
 
-// Closest hit for the active queue (ObjectManager::IntersectRay).
-// PERSIST: persistent waves take queue entries with a wave-wide fetch
-// (wave_fetch.h) and step one traversal iteration at a time, so lanes that
-// finish early are refilled; otherwise one thread traces one ray to the end
-// (grid-stride), which costs less per ray when trees are shallow.
-template <int STACK, int BLOCK, bool PERSIST>
-__global__ __launch_bounds__(BLOCK) void k_extend(const ReqInfo* __restrict__ reqs, Paths S, int depth)
+// The closest hits of queue entries, in persistent waves (persist_closest).
+template <class Stack>
+__device__ inline void extend_items(const ReqInfo* __restrict__ reqs, const Paths& S, const unsigned* q,
+                                    const ItemSource& items, Stack& st)
 {
-    __shared__ uint2 lds[STACK > 0 ? STACK * BLOCK : 1];
-    const unsigned n = ext_count(S, depth);
-    const unsigned* q = S.queue[depth & 1];
-    if constexpr (!PERSIST) {
-        auto st = make_stack<STACK>(lds, BLOCK);
-        for (unsigned i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
-            extend_entry(reqs, S, q[i], st);
-        return;
-    }
-    auto st = make_stack<STACK>(lds, BLOCK);
     const NodeSlot* nodes = nullptr;
     const Tri48* tris = nullptr;
     unsigned slot = 0, nn = 0, nt = 0;  // slot: lane * cap + path slot of the current item
     persist_closest<false, false, false, RayState>(
-        st, n, S.fetch + depth, nn, nt, nodes, tris, nullptr,
+        st, items, nn, nt, nodes, tris, nullptr,
         [&](int64_t item, RayState& r, ClosestState& s) {
             const unsigned code = q[item];
             slot = (code & 3u) * (unsigned)S.cap + (code >> 2);
@@ -461,6 +448,30 @@ __global__ __launch_bounds__(BLOCK) void k_extend(const ReqInfo* __restrict__ re
             S.hit_leaf[slot] = s.best_id >= 0 ? s.best_leaf : 0xffffffffu;
             S.hit_t[slot] = s.best_id >= 0 ? (float)s.best_t : 0.0f;
         });
+}
+
+// Waves per SIMD the persistent k_extend's registers are budgeted for.
+constexpr int kExtendWaves = 5;
+
+// Closest hit for the active queue (ObjectManager::IntersectRay).
+// PERSIST: persistent waves take queue entries with a wave-wide fetch
+// (wave_fetch.h) and step one traversal iteration at a time, so lanes that
+// finish early are refilled; otherwise one thread traces one ray to the end
+// (grid-stride), which costs less per ray when trees are shallow.
+template <int STACK, int BLOCK, bool PERSIST>
+__global__ __launch_bounds__(BLOCK, PERSIST ? kExtendWaves : 1) void k_extend(const ReqInfo* __restrict__ reqs, Paths S, int depth)
+{
+    __shared__ uint2 lds[STACK > 0 ? STACK * BLOCK : 1];
+    const unsigned n = ext_count(S, depth);
+    const unsigned* q = S.queue[depth & 1];
+    if constexpr (!PERSIST) {
+        auto st = make_stack<STACK>(lds, BLOCK);
+        for (unsigned i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
+            extend_entry(reqs, S, q[i], st);
+        return;
+    }
+    auto st = make_stack<STACK>(lds, BLOCK);
+    extend_items(reqs, S, q, grid_items(S.fetch + depth, n), st);
 }
 
 // ---- materials at one wavelength ------------------------------------------------
@@ -1765,6 +1776,36 @@ __device__ inline void connect_record(const ReqInfo* __restrict__ reqs, const Pa
     else add_shadow(S, code, S.sval[i], 1.0f);
 }
 
+// Shadow records from sh0 on, in persistent waves (persist_any).
+template <class Stack>
+__device__ inline void connect_items(const ReqInfo* __restrict__ reqs, const Paths& S, unsigned sh0,
+                                     const ItemSource& items, Stack& st)
+{
+    const NodeSlot* nodes = nullptr;
+    const Tri48* tris = nullptr;
+    bool media = false;
+    unsigned nn = 0, nt = 0;
+    persist_any<false, false, false, RayState>(
+        st, items, nn, nt, nodes, tris, nullptr,
+        [&](int64_t item, RayState& r, AnyState& s) {
+            const int64_t i = sh0 + item;
+            if (S.sinfo && (S.sinfo[i] & kShadowInScatter)) return false;  // no occlusion test; the walk adds it
+            const ReqInfo& R = reqs[S.req[(S.sslot[i] & kRecSlotMask) >> 2]];
+            nodes = R.sc.nodes;
+            tris = R.sc.tris;
+            media = R.sc.has_media;
+            init_ray(r, S.sox[i], S.soy[i], S.soz[i], S.sdx[i], S.sdy[i], S.sdz[i]);
+            any_begin(r, scale_how_far(r, (double)(S.stmax[i] - 0.001f)), s);
+            return true;
+        },
+        [&](int64_t item, const AnyState& s) {
+            if (s.hit) return;
+            const int64_t i = sh0 + item;
+            if (media) S.svis[i] = 1u;
+            else add_shadow(S, S.sslot[i], S.sval[i], 1.0f);
+        });
+}
+
 // Waves per SIMD k_connect's registers are budgeted for: 5, i.e. at most 96
 // VGPRs (it needs 98 unbudgeted, which leaves 4).
 constexpr int kConnectWaves = 5;
@@ -1787,27 +1828,7 @@ __global__ __launch_bounds__(BLOCK, kConnectWaves) void k_connect(const ReqInfo*
         return;
     }
     auto st = make_stack<STACK>(lds, BLOCK);
-    const NodeSlot* nodes = nullptr;
-    const Tri48* tris = nullptr;
-    bool media = false;
-    unsigned nn = 0, nt = 0;
-    persist_any<false, false, false, RayState>(
-        st, n, S.fetch + (kMaxPathDepth + 1) + depth, nn, nt, nodes, tris, nullptr,
-        [&](int64_t item, RayState& r, AnyState& s) {
-            if (S.sinfo && (S.sinfo[item] & kShadowInScatter)) return false;  // no occlusion test; the walk adds it
-            const ReqInfo& R = reqs[S.req[(S.sslot[item] & kRecSlotMask) >> 2]];
-            nodes = R.sc.nodes;
-            tris = R.sc.tris;
-            media = R.sc.has_media;
-            init_ray(r, S.sox[item], S.soy[item], S.soz[item], S.sdx[item], S.sdy[item], S.sdz[item]);
-            any_begin(r, scale_how_far(r, (double)(S.stmax[item] - 0.001f)), s);
-            return true;
-        },
-        [&](int64_t item, const AnyState& s) {
-            if (s.hit) return;
-            if (media) S.svis[item] = 1u;
-            else add_shadow(S, S.sslot[item], S.sval[item], 1.0f);
-        });
+    connect_items(reqs, S, 0u, grid_items(S.fetch + (kMaxPathDepth + 1) + depth, n), st);
 }
 
 // ---- the rest of a pass in one launch -----------------------------------------
@@ -1828,11 +1849,12 @@ constexpr unsigned kFinishMin = 8;  // entries a workgroup takes at a time, at l
 // workgroup's chains of dependent loads, at one to four busy waves.
 // More than `limit` entries are left to the separate launches, which use the
 // whole device better; the host tries again a few bounces on.  A workgroup
-// takes at most `most` entries at a time.
+// takes at most `most` entries at a time.  deep: trees worth the persistent
+// traversal, which ends in eight lanes a ray.
 // SURFACES: conductors or dielectrics among the materials; MEDIA: volumes.
 template <bool SURFACES, bool SKY, bool MEDIA>
 __global__ __launch_bounds__(kFinishBlock, 2) void k_finish(const ReqInfo* __restrict__ reqs, Paths S, int depth0,
-                                                            int bounces, unsigned limit, unsigned most)
+                                                            int bounces, unsigned limit, unsigned most, int deep)
 {
     constexpr int B = kFinishBlock, Q = 4 * B;  // an entry becomes at most four lanes
     constexpr int kStackWords = 2 * kFinishStack * B, kShadeWords = shade_lds_words<kMatLambert, B>();
@@ -1842,6 +1864,7 @@ __global__ __launch_bounds__(kFinishBlock, 2) void k_finish(const ReqInfo* __res
     __shared__ __align__(8) unsigned work[kStackWords > kShadeWords ? kStackWords : kShadeWords];
     __shared__ unsigned bin_words[kBinWords];
     __shared__ unsigned cnt[2 + kBins];  // next entries, shadow records, binned entries
+    __shared__ unsigned long long fetch[2];
     const unsigned n0 = S.cnt_ext[depth0], stop = *S.stop, tid = threadIdx.x;
     // The workgroups of this launch write depth0 + 1; an earlier launch less.
     if (n0 > limit || (stop != 0u && stop < (unsigned)depth0 + 1u)) return;
@@ -1858,8 +1881,11 @@ __global__ __launch_bounds__(kFinishBlock, 2) void k_finish(const ReqInfo* __res
         for (unsigned i = tid; i < n; i += B) queue[0][i] = q0[c + i];
         for (int d = depth0; d < bounces && n > 0; ++d) {
             if (tid < 2 + kBins) cnt[tid] = 0u;
+            if (tid < 2) fetch[tid] = 0ull;
             __syncthreads();
-            for (unsigned i = tid; i < n; i += B) extend_entry(reqs, S, queue[cur][i], st);
+            if (deep) extend_items(reqs, S, queue[cur], block_items<B>(&fetch[0], n), st);
+            else
+                for (unsigned i = tid; i < n; i += B) extend_entry(reqs, S, queue[cur][i], st);
             __syncthreads();
             bin_entries<SKY, B>(
                 reqs, S, d, queue[cur], n, 0u, (unsigned)B, cnt + 2, 1,
@@ -1886,7 +1912,9 @@ __global__ __launch_bounds__(kFinishBlock, 2) void k_finish(const ReqInfo* __res
             __syncthreads();
             const unsigned n_sh = cnt[1];
             n = cnt[0];
-            for (unsigned i = tid; i < n_sh; i += B) connect_record(reqs, S, sh0 + i, st);
+            if (deep) connect_items(reqs, S, sh0, block_items<B>(&fetch[1], n_sh), st);
+            else
+                for (unsigned i = tid; i < n_sh; i += B) connect_record(reqs, S, sh0 + i, st);
             __syncthreads();
             if (MEDIA) {
                 walk_records(reqs, S, sh0 + tid, sh0 + n_sh, (unsigned)B);
@@ -2514,8 +2542,13 @@ struct PassShape {
 // 25.3 ms, 1080p terrain 19.5 / 19.0 / 18.3 / 19.0 / 19.0 ms (4716 us, 23.3 ms
 // and 20.1 ms without k_finish).
 constexpr int kFinishPaths = 131072, kFinishDepth = 14, kFinishLimit = 131072;
+// Levels from which k_finish traverses with persistent waves.  From 2 / 4 / never:
+// fog 64 x 64 670 / 654 / 657 us, conductor and glass 333 x 250 x 9 3420 / 3410 /
+// 3475 us, 48 served previews 19.0 / 19.0 / 19.1 ms, 1080p terrain 17.9 / 18.0 /
+// 18.3 ms.
+constexpr int kFinishDeep = 4;
 
-using FinishKernel = void (*)(const ReqInfo*, Paths, int, int, unsigned, unsigned);
+using FinishKernel = void (*)(const ReqInfo*, Paths, int, int, unsigned, unsigned, int);
 
 FinishKernel pick_finish(const PassShape& sh)
 {
@@ -2547,8 +2580,8 @@ void launch_pass(const ReqInfo* d_info, Paths S, const PassEntry* ent, int n_ent
         const int64_t share = d == 0 ? (entries + grid - 1) / grid : sh.cap / grid;
         unsigned most = (unsigned)std::max<int64_t>(1, std::min<int64_t>(share, kFinishBlock));
         const unsigned blocks = (unsigned)std::min<int64_t>(grid, std::max<int64_t>(1, d == 0 ? grid : sh.cap / most));
-        int bounces = sh.bounces;
-        void* args[] = {(void*)&d_info, &S, &d, &bounces, &limit, &most};
+        int bounces = sh.bounces, deep = sh.depth >= kFinishDeep;
+        void* args[] = {(void*)&d_info, &S, &d, &bounces, &limit, &most, &deep};
         (void)hipLaunchKernel((const void*)fn, dim3(blocks), dim3(kFinishBlock), args, 0, stream);
     };
     const bool whole = can_finish && paths <= kFinishPaths;

@@ -516,28 +516,52 @@ RISE_HD inline unsigned accept_slots(const SlabAxis& ax, const SlabAxis& ay, con
     return acc;
 }
 
+// A node's three axes for a ray; an object-space ray's planes are widened by
+// the origin's rounding (ObjRayT).
 template <int A>
-RISE_HD inline unsigned node_accept_mask(const RayStateT<A>& r, const uint4& w0, const uint4& w2, const uint4& w3,
+RISE_HD inline void slab_axes(const RayStateT<A>& r, const uint4& w0, SlabAxis& ax, SlabAxis& ay, SlabAxis& az)
+{
+    ax = slab_axis(bits_to_float(w0.x), (int)(signed char)(w0.w & 0xff), r.ox, r.ix);
+    ay = slab_axis(bits_to_float(w0.y), (int)(signed char)((w0.w >> 8) & 0xff), r.oy, r.iy);
+    az = slab_axis(bits_to_float(w0.z), (int)(signed char)((w0.w >> 16) & 0xff), r.oz, r.iz);
+}
+template <int A>
+RISE_HD inline void slab_axes(const ObjRayT<A>& r, const uint4& w0, SlabAxis& ax, SlabAxis& ay, SlabAxis& az)
+{
+    ax = slab_axis_widened(bits_to_float(w0.x), (int)(signed char)(w0.w & 0xff), r.ox, r.ix, r.ex);
+    ay = slab_axis_widened(bits_to_float(w0.y), (int)(signed char)((w0.w >> 8) & 0xff), r.oy, r.iy, r.ey);
+    az = slab_axis_widened(bits_to_float(w0.z), (int)(signed char)((w0.w >> 16) & 0xff), r.oz, r.iz, r.ez);
+}
+
+template <class R>
+RISE_HD inline unsigned node_accept_mask(const R& r, const uint4& w0, const uint4& w2, const uint4& w3,
                                          const uint4& w4, float pad_limit)
 {
-    const SlabAxis ax = slab_axis(bits_to_float(w0.x), (int)(signed char)(w0.w & 0xff), r.ox, r.ix);
-    const SlabAxis ay = slab_axis(bits_to_float(w0.y), (int)(signed char)((w0.w >> 8) & 0xff), r.oy, r.iy);
-    const SlabAxis az = slab_axis(bits_to_float(w0.z), (int)(signed char)((w0.w >> 16) & 0xff), r.oz, r.iz);
+    SlabAxis ax, ay, az;
+    slab_axes(r, w0, ax, ay, az);
     return accept_slots(ax, ay, az, r.ix < 0.0f, r.iy < 0.0f, r.iz < 0.0f, w2, w3, w4, pad_limit);
 }
 
-// The same for an object-space ray: the float ray's planes widened by the
-// origin's rounding (ObjRayT).
-template <int A>
-RISE_HD inline unsigned node_accept_mask(const ObjRayT<A>& r, const uint4& w0, const uint4& w2, const uint4& w3,
-                                         const uint4& w4, float pad_limit)
+// One slot's box alone (accept_slots' test for that slot), for a lane that
+// shares the node with others: reads the slot's six bounds byte by byte.
+template <class R>
+RISE_HD inline bool slot_accepted(const R& r, const unsigned char* __restrict__ node, const uint4& w0, unsigned slot,
+                                  float pad_limit)
 {
-    const SlabAxis ax = slab_axis_widened(bits_to_float(w0.x), (int)(signed char)(w0.w & 0xff), r.ox, r.ix, r.ex);
-    const SlabAxis ay =
-        slab_axis_widened(bits_to_float(w0.y), (int)(signed char)((w0.w >> 8) & 0xff), r.oy, r.iy, r.ey);
-    const SlabAxis az =
-        slab_axis_widened(bits_to_float(w0.z), (int)(signed char)((w0.w >> 16) & 0xff), r.oz, r.iz, r.ez);
-    return accept_slots(ax, ay, az, r.ix < 0.0f, r.iy < 0.0f, r.iz < 0.0f, w2, w3, w4, pad_limit);
+    SlabAxis ax, ay, az;
+    slab_axes(r, w0, ax, ay, az);
+    const unsigned char* lo = node + 32 + slot;  // qlox, qloy, qloz, then qhix, qhiy, qhiz, 8 bytes each
+    const unsigned char* hi = node + 56 + slot;
+    const bool nx = r.ix < 0.0f, ny = r.iy < 0.0f, nz = r.iz < 0.0f;
+    const float tnx = fmaf((float)(nx ? hi : lo)[0], ax.s, ax.bn);
+    const float tny = fmaf((float)(ny ? hi : lo)[8], ay.s, ay.bn);
+    const float tnz = fmaf((float)(nz ? hi : lo)[16], az.s, az.bn);
+    const float tfx = fmaf((float)(nx ? lo : hi)[0], ax.sf, ax.bf);
+    const float tfy = fmaf((float)(ny ? lo : hi)[8], ay.sf, ay.bf);
+    const float tfz = fmaf((float)(nz ? lo : hi)[16], az.sf, az.bf);
+    const float tn = fmaxf(fmaxf(tnx, tny), fmaxf(tnz, 0.0f));
+    const float tf = fminf(fminf(tfx, tfy), fminf(tfz, pad_limit));
+    return tn <= tf;
 }
 
 // Bit s of the 8-bit mask x moved to bit s ^ o (0 <= o < 8): the exchanges of

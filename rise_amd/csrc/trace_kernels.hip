@@ -24,6 +24,8 @@ namespace {
 #define RISE_TRACE_BLOCK 128
 #endif
 constexpr int kBlock = RISE_TRACE_BLOCK;
+// Waves per SIMD the traversal kernels' registers are budgeted for (96 each).
+constexpr int kWaves = 5;
 
 __device__ inline void load_ray(const float* __restrict__ rays, int64_t n, int64_t i, float& ox, float& oy, float& oz,
                                 float& dx, float& dy, float& dz)
@@ -59,7 +61,7 @@ inline unsigned grid_for(int64_t n) { return (unsigned)((n + kBlock - 1) / kBloc
 
 // F64: certify on the leaf records' double vertices (tri64).
 template <bool COUNT, int STACK, int A, bool F64 = false>
-__global__ __launch_bounds__(kBlock) void closest_persistent(const NodeSlot* __restrict__ nodes,
+__global__ __launch_bounds__(kBlock, kWaves) void closest_persistent(const NodeSlot* __restrict__ nodes,
                                                              const Tri48* __restrict__ tris,
                                                              const float* __restrict__ rays, int64_t n,
                                                              int32_t* __restrict__ prim_id,
@@ -73,7 +75,7 @@ __global__ __launch_bounds__(kBlock) void closest_persistent(const NodeSlot* __r
     const Tri48* const tp = tris;
     unsigned nn = 0, nt = 0;
     persist_closest<COUNT, false, F64, RayStateT<A>>(
-        st, n, next, nn, nt, np, tp, tri64,
+        st, next ? grid_items(next, n) : sparse_items(n), nn, nt, np, tp, tri64,
         [&](int64_t i, RayStateT<A>& r, ClosestState& s) {
             init_ray_at(r, rays, n, i);
             closest_begin(r, s);
@@ -87,7 +89,7 @@ __global__ __launch_bounds__(kBlock) void closest_persistent(const NodeSlot* __r
 }
 
 template <bool COUNT, int STACK, int A, bool F64 = false>
-__global__ __launch_bounds__(kBlock) void any_persistent(const NodeSlot* __restrict__ nodes,
+__global__ __launch_bounds__(kBlock, kWaves) void any_persistent(const NodeSlot* __restrict__ nodes,
                                                          const Tri48* __restrict__ tris,
                                                          const float* __restrict__ rays,
                                                          const float* __restrict__ tmax, int64_t n,
@@ -101,7 +103,7 @@ __global__ __launch_bounds__(kBlock) void any_persistent(const NodeSlot* __restr
     const Tri48* const tp = tris;
     unsigned nn = 0, nt = 0;
     persist_any<COUNT, false, F64, RayStateT<A>>(
-        st, n, next, nn, nt, np, tp, tri64,
+        st, next ? grid_items(next, n) : sparse_items(n), nn, nt, np, tp, tri64,
         [&](int64_t i, RayStateT<A>& r, AnyState& s) {
             init_ray_at(r, rays, n, i);
             any_begin(r, scale_how_far(r, tmax ? (double)tmax[i] : kRiseInfinity), s);
@@ -165,7 +167,7 @@ __global__ __launch_bounds__(kBlock) void ex_records(const Tri48* __restrict__ t
 // Closest hit with the face selection of rise_hip_intersect_closest_ex; the
 // result is staged in hits for ex_records.
 template <int STACK, int A, bool F64 = false>
-__global__ __launch_bounds__(kBlock) void closest_ex_persistent(const NodeSlot* __restrict__ nodes,
+__global__ __launch_bounds__(kBlock, kWaves) void closest_ex_persistent(const NodeSlot* __restrict__ nodes,
                                                                 const Tri48* __restrict__ tris,
                                                                 const float* __restrict__ rays, int64_t n,
                                                                 unsigned faces, rise_hip_hit* __restrict__ hits,
@@ -179,7 +181,7 @@ __global__ __launch_bounds__(kBlock) void closest_ex_persistent(const NodeSlot* 
     const Tri48* const tp = tris;
     unsigned nn = 0, nt = 0;
     persist_closest<false, true, F64, RayStateT<A>>(
-        st, n, next, nn, nt, np, tp, tri64,
+        st, next ? grid_items(next, n) : sparse_items(n), nn, nt, np, tp, tri64,
         [&](int64_t i, RayStateT<A>& r, ClosestState& s) {
             init_ray_at(r, rays, n, i);
             closest_begin(r, s);
@@ -193,7 +195,7 @@ __global__ __launch_bounds__(kBlock) void closest_ex_persistent(const NodeSlot* 
 
 // Any hit with the face selection of rise_hip_intersect_any_ex.
 template <int STACK, int A, bool F64 = false>
-__global__ __launch_bounds__(kBlock) void any_ex_persistent(const NodeSlot* __restrict__ nodes,
+__global__ __launch_bounds__(kBlock, kWaves) void any_ex_persistent(const NodeSlot* __restrict__ nodes,
                                                             const Tri48* __restrict__ tris,
                                                             const float* __restrict__ rays,
                                                             const float* __restrict__ tmax, int64_t n,
@@ -207,7 +209,7 @@ __global__ __launch_bounds__(kBlock) void any_ex_persistent(const NodeSlot* __re
     const Tri48* const tp = tris;
     unsigned nn = 0, nt = 0;
     persist_any<false, true, F64, RayStateT<A>>(
-        st, n, next, nn, nt, np, tp, tri64,
+        st, next ? grid_items(next, n) : sparse_items(n), nn, nt, np, tp, tri64,
         [&](int64_t i, RayStateT<A>& r, AnyState& s) {
             init_ray_at(r, rays, n, i);
             any_begin(r, scale_how_far(r, tmax ? (double)tmax[i] : kRiseInfinity), s);
@@ -219,22 +221,39 @@ __global__ __launch_bounds__(kBlock) void any_ex_persistent(const NodeSlot* __re
 
 __global__ void reset_counter(unsigned long long* c) { *c = 0ull; }
 
-// Waves resident at once for a persistent kernel: CUs x blocks per CU.
-template <class K>
-unsigned persistent_grid(K kernel, int64_t n)
+// Workgroups of a persistent launch over n rays: those resident at once (CUs x
+// blocks per CU), or, when that leaves every ray kCoopLanes lanes, one wave for
+// each kCoopRays rays (`sparse`; such a launch needs no fetch counter).  The
+// line lies where the lanes run out: closest hits of 1000 / 7072 / 30,000 /
+// 40,960 rays into 20,000 triangles take 39 / 47 / 54 / 65 us sparse, 57 / 63 / 64
+// / 69 with one ray a lane from the start; into a million 131 / 171 / 228 / 244
+// and 187 / 217 / 240 / 250.
+struct TraceGrid {
+    unsigned blocks;
+    bool sparse;
+};
+
+// The cleared fetch counter of a launch, NULL for a sparse one.
+unsigned long long* fetch_counter(const TraceScene& s, const TraceGrid& g, hipStream_t stream)
 {
-    static int cus = 0;
-    if (cus == 0) {
-        int dev = 0;
-        (void)hipGetDevice(&dev);
-        (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-        if (cus <= 0) cus = 256;
-    }
-    int per_cu = 0;
+    if (g.sparse) return nullptr;
+    hipLaunchKernelGGL(reset_counter, dim3(1), dim3(1), 0, stream, s.fetch_counter);
+    return s.fetch_counter;
+}
+
+template <class K>
+TraceGrid trace_grid(K kernel, int64_t n, bool may_be_sparse)
+{
+    int dev = 0, cus = 0, per_cu = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+        cus = 256;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kBlock, 0) != hipSuccess || per_cu <= 0)
         per_cu = 4;
     const int64_t want = (int64_t)cus * per_cu;
-    return (unsigned)std::max<int64_t>(1, std::min<int64_t>(want, (int64_t)grid_for(n)));
+    const int64_t sparse = (n + kBlock / kCoopLanes - 1) / (kBlock / kCoopLanes);
+    if (may_be_sparse && sparse <= want) return TraceGrid{(unsigned)std::max<int64_t>(1, sparse), true};
+    return TraceGrid{(unsigned)std::max<int64_t>(1, std::min<int64_t>(want, (int64_t)grid_for(n))), false};
 }
 
 }  // namespace
@@ -248,10 +267,13 @@ hipError_t launch_closest(const TraceScene& s, const float* rays, int64_t n, int
     if (n <= 0) return hipSuccess;
     const int need = s.depth - 1;
     const dim3 block(kBlock);
-    hipLaunchKernelGGL(reset_counter, dim3(1), dim3(1), 0, stream, s.fetch_counter);
-#define RISE_LAUNCH_CLOSEST_F(C, S, A, F)                                                                   \
-    hipLaunchKernelGGL((closest_persistent<C, S, A, F>), dim3(persistent_grid(closest_persistent<C, S, A, F>, n)), \
-                       block, 0, stream, s.nodes, s.tris, rays, n, prim_id, t, counters, s.fetch_counter, s.tri64)
+#define RISE_LAUNCH_CLOSEST_F(C, S, A, F)                                                              \
+    do {                                                                                               \
+        const TraceGrid g = trace_grid(closest_persistent<C, S, A, F>, n, !C && S > 0);                 \
+        unsigned long long* const next = fetch_counter(s, g, stream);                                  \
+        hipLaunchKernelGGL((closest_persistent<C, S, A, F>), dim3(g.blocks), block, 0, stream, s.nodes, \
+                           s.tris, rays, n, prim_id, t, counters, next, s.tri64);                       \
+    } while (0)
 #define RISE_LAUNCH_CLOSEST(C, S, A)                   \
     do {                                               \
         if (s.tri64) RISE_LAUNCH_CLOSEST_F(C, S, A, true); \
@@ -283,10 +305,13 @@ hipError_t launch_any(const TraceScene& s, const float* rays, const float* tmax,
     if (n <= 0) return hipSuccess;
     const int need = s.depth - 1;
     const dim3 block(kBlock);
-    hipLaunchKernelGGL(reset_counter, dim3(1), dim3(1), 0, stream, s.fetch_counter);
-#define RISE_LAUNCH_ANY_F(C, S, A, F)                                                                        \
-    hipLaunchKernelGGL((any_persistent<C, S, A, F>), dim3(persistent_grid(any_persistent<C, S, A, F>, n)), block, \
-                       0, stream, s.nodes, s.tris, rays, tmax, n, occluded, counters, s.fetch_counter, s.tri64)
+#define RISE_LAUNCH_ANY_F(C, S, A, F)                                                                   \
+    do {                                                                                               \
+        const TraceGrid g = trace_grid(any_persistent<C, S, A, F>, n, !C && S > 0);                     \
+        unsigned long long* const next = fetch_counter(s, g, stream);                                  \
+        hipLaunchKernelGGL((any_persistent<C, S, A, F>), dim3(g.blocks), block, 0, stream, s.nodes, s.tris, rays, \
+                           tmax, n, occluded, counters, next, s.tri64);                                 \
+    } while (0)
 #define RISE_LAUNCH_ANY(C, S, A)                   \
     do {                                           \
         if (s.tri64) RISE_LAUNCH_ANY_F(C, S, A, true); \
@@ -318,12 +343,12 @@ hipError_t launch_closest_ex(const TraceScene& s, const float* rays, int64_t n, 
     if (n <= 0) return hipSuccess;
     const int need = s.depth - 1;
     const dim3 block(kBlock);
-    hipLaunchKernelGGL(reset_counter, dim3(1), dim3(1), 0, stream, s.fetch_counter);
 #define RISE_LAUNCH_EX_F(S, A, F)                                                                           \
     do {                                                                                                    \
-        hipLaunchKernelGGL((closest_ex_persistent<S, A, F>),                                                \
-                           dim3(persistent_grid(closest_ex_persistent<S, A, F>, n)), block, 0, stream, s.nodes, \
-                           s.tris, rays, n, faces, hits, s.fetch_counter, s.tri64, s.attr);                 \
+        const TraceGrid g = trace_grid(closest_ex_persistent<S, A, F>, n, S > 0);                           \
+        unsigned long long* const next = fetch_counter(s, g, stream);                                       \
+        hipLaunchKernelGGL((closest_ex_persistent<S, A, F>), dim3(g.blocks), block, 0, stream, s.nodes,     \
+                           s.tris, rays, n, faces, hits, next, s.tri64, s.attr);                            \
         hipLaunchKernelGGL((ex_records<A, F>), dim3(grid_for(n)), block, 0, stream, s.tris, rays, n, hits,  \
                            s.tri64, s.attr);                                                                \
     } while (0)
@@ -352,10 +377,13 @@ hipError_t launch_any_ex(const TraceScene& s, const float* rays, const float* tm
     if (n <= 0) return hipSuccess;
     const int need = s.depth - 1;
     const dim3 block(kBlock);
-    hipLaunchKernelGGL(reset_counter, dim3(1), dim3(1), 0, stream, s.fetch_counter);
-#define RISE_LAUNCH_EX_F(S, A, F)                                                                          \
-    hipLaunchKernelGGL((any_ex_persistent<S, A, F>), dim3(persistent_grid(any_ex_persistent<S, A, F>, n)), block, \
-                       0, stream, s.nodes, s.tris, rays, tmax, n, faces, occluded, s.fetch_counter, s.tri64)
+#define RISE_LAUNCH_EX_F(S, A, F)                                                                         \
+    do {                                                                                                 \
+        const TraceGrid g = trace_grid(any_ex_persistent<S, A, F>, n, S > 0);                             \
+        unsigned long long* const next = fetch_counter(s, g, stream);                                    \
+        hipLaunchKernelGGL((any_ex_persistent<S, A, F>), dim3(g.blocks), block, 0, stream, s.nodes, s.tris, rays, \
+                           tmax, n, faces, occluded, next, s.tri64);                                      \
+    } while (0)
 #define RISE_LAUNCH_EX(S, A)                   \
     do {                                       \
         if (s.tri64) RISE_LAUNCH_EX_F(S, A, true); \

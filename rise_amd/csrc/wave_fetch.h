@@ -56,35 +56,74 @@ __device__ inline typename StackKind<STACK>::type make_stack(uint2* lds, int str
     return st;
 }
 
+// Lanes that share one ray once few rays are left in a wave (coop_* below).
+constexpr int kCoopLanes = 8, kCoopRays = 64 / kCoopLanes;
+
+// Where a launch's items come from: `total` of them, the first `first` assigned
+// to the threads statically (thread `self` of them), the others claimed from
+// `next` (which counts from `first`).  per_wave < 64: each wave takes only that
+// many of its first items, its lowest lanes one each, and the launch has no
+// others.
+struct ItemSource {
+    unsigned long long* next;
+    unsigned long long total, first, self;
+    int per_wave;
+};
+
+// All items of a grid-wide launch.
+__device__ inline ItemSource grid_items(unsigned long long* next, int64_t n)
+{
+    return ItemSource{next, n > 0 ? (unsigned long long)n : 0ull, (unsigned long long)gridDim.x * blockDim.x,
+                      (unsigned long long)blockIdx.x * blockDim.x + threadIdx.x, 64};
+}
+
+// A grid-wide launch of kCoopRays items a wave.
+__device__ inline ItemSource sparse_items(int64_t n)
+{
+    const unsigned long long wave = ((unsigned long long)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+    return ItemSource{nullptr, n > 0 ? (unsigned long long)n : 0ull, n > 0 ? (unsigned long long)n : 0ull,
+                      wave * kCoopRays + __lane_id(), kCoopRays};
+}
+
+// n items of one workgroup of BLOCK threads: an even share for every wave while
+// there are at most BLOCK, so that no wave has more rays than it must; else
+// one a thread and the others from `next` (LDS, cleared).
+template <int BLOCK>
+__device__ inline ItemSource block_items(unsigned long long* next, unsigned n)
+{
+    const unsigned wave = threadIdx.x >> 6;
+    if (n > (unsigned)BLOCK) return ItemSource{next, n, (unsigned long long)BLOCK, threadIdx.x, 64};
+    const unsigned share = (n + BLOCK / 64 - 1) / (BLOCK / 64);
+    return ItemSource{nullptr, n, n, (unsigned long long)(wave * share + __lane_id()), (int)share};
+}
+
 // The next item of every idle lane of a wave (`busy` false), wave-wide: first
-// the thread's own (one per thread of the grid), so that a launch starts
-// without a burst of atomics on one address, then items of the wave's own
-// chunk, claimed from the shared counter (which counts from the grid's size)
+// the thread's own, so that a launch starts without a burst of atomics on one
+// address, then items of the wave's own chunk, claimed from the shared counter
 // with one atomic per chunk.  Atomics on one address serialize at about 10 ns
 // each, so a claim per refill bounds the launch; chunks shrink as the items
 // run out (a quarter of an even share, between 32 and RISE_CHUNK), so that
 // the waves end together.
 struct ItemFetch {
-    unsigned long long* next;
-    int64_t n;
+    ItemSource src;
     unsigned long long cur, end;  // wave-uniform: the claimed items not yet taken
     bool started;
     bool more;  // wave-uniform: the items may not be exhausted
 
-    __device__ inline ItemFetch(unsigned long long* counter, int64_t items)
-        : next(counter), n(items), cur(0), end(0), started(false), more(items > 0)
+    __device__ inline explicit ItemFetch(const ItemSource& s)
+        : src(s), cur(0), end(0), started(false), more(s.total > 0)
     {
     }
     // Every lane of the wave calls; the lane's new item, or -1.
     __device__ inline long long take(bool busy)
     {
-        const unsigned long long first = (unsigned long long)gridDim.x * blockDim.x, total = (unsigned long long)n;
+        const unsigned long long total = src.total;
         unsigned long long i;
         if (!started) {
-            i = (unsigned long long)blockIdx.x * blockDim.x + threadIdx.x;
-            more = total > first;
+            i = (int)__lane_id() < src.per_wave ? src.self : total;
+            more = total > src.first;
             started = true;
-            cur = end = first;
+            cur = end = src.first;
         } else {
             const unsigned long long im = __ballot(!busy);
             const unsigned want = (unsigned)__popcll(im), left = (unsigned)(end - cur);
@@ -93,14 +132,14 @@ struct ItemFetch {
             i = cur + rank;
             cur += want;
             if (want > left) {
-                const float share = (float)(total - end) * 16.0f / (float)first;  // a quarter of this wave's even share
+                const float share = (float)(total - end) * 16.0f / (float)src.first;  // a quarter of this wave's even share
                 const unsigned size = (unsigned)fminf(fmaxf(share, 32.0f), (float)RISE_CHUNK);
                 const unsigned need = want - left, take = size > need ? size : need;
                 unsigned long long base = 0;
-                if (__lane_id() == 0) base = atomicAdd(next, (unsigned long long)take);
+                if (__lane_id() == 0) base = atomicAdd(src.next, (unsigned long long)take);
                 const unsigned lo = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)base);
                 const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(base >> 32));
-                base = first + (((unsigned long long)hi << 32) | lo);
+                base = src.first + (((unsigned long long)hi << 32) | lo);
                 if (rank >= left) i = base + (rank - left);
                 cur = base + need;
                 end = base + take;
@@ -110,6 +149,196 @@ struct ItemFetch {
         }
         return !busy && i < total ? (long long)i : -1;
     }
+};
+
+// ---- one ray over eight lanes -------------------------------------------------
+//
+// Once a wave has at most kCoopRays rays left and none to fetch, each ray gets
+// kCoopLanes lanes: lane j of a group tests slot j ^ oinv of the ray's next
+// node, so one ballot gives every group its hit mask in visiting order, and the
+// lanes of accepted leaves test their triangles side by side.  A step is some
+// 120 instructions instead of 400, and what bounds the end of a launch (or a
+// launch of few rays) is the longest ray's chain of steps: 7072 rays into 20,000
+// triangles 107 -> 68 us, a million shadow rays into 200,000 574 -> 544 us (and
+// the additional code costs launches with no short end 0.5%: six million rays
+// into a million triangles 2836 -> 2850 us).
+
+__device__ inline long long shfl_i64(long long v, int src)
+{
+    const unsigned lo = (unsigned)__shfl((int)(unsigned)v, src), hi = (unsigned)__shfl((int)(unsigned)(v >> 32), src);
+    return (long long)(((unsigned long long)hi << 32) | lo);
+}
+__device__ inline double shfl_f64(double v, int src)
+{
+    return __builtin_bit_cast(double, shfl_i64(__builtin_bit_cast(long long, v), src));
+}
+
+// This lane's group's ray: the lane that holds it (the group-th busy lane of
+// bm), -1 for a group without one.
+__device__ inline int coop_owner(unsigned long long bm)
+{
+    const int group = (int)__lane_id() / kCoopLanes;
+    for (int k = 0; k < group; ++k) bm &= bm - 1ull;
+    return bm ? __builtin_ctzll(bm) : -1;
+}
+
+// One node visit of a group: like visit_node, with the group's lanes at its
+// slots.  leaf, count: the triangles of this lane's accepted leaf (count 0:
+// none).  Every lane of the wave calls; `on`: its group's ray goes on.
+template <class Stack, class R>
+__device__ inline void coop_visit(bool on, const R& r, const NodeSlot* __restrict__ nodes, Stack& st, NodeGroup& g,
+                                  float pad_limit, unsigned& leaf, unsigned& count)
+{
+    bool internal = false;
+    unsigned base = 0, imask = 0;
+    count = 0;
+    leaf = 0;
+    if (on) {
+        const unsigned k = __builtin_ctz(g.hits);
+        g.hits &= g.hits - 1u;
+        const unsigned at = k ^ r.oinv;
+        const unsigned ni = g.base + __builtin_popcount(g.imask & ((1u << at) - 1u));
+        if (g.hits) st.push(make_uint2(g.base, g.hits | (g.imask << 8)));  // every lane of the group writes the same entry
+        const unsigned char* node = reinterpret_cast<const unsigned char*>(nodes + ni);
+        const unsigned slot = (__lane_id() & (kCoopLanes - 1)) ^ r.oinv;
+        const uint4 w0 = *reinterpret_cast<const uint4*>(node);
+        const uint2 w1 = *reinterpret_cast<const uint2*>(node + 16);
+        const unsigned meta = node[24 + slot];
+        const bool hit = meta != 0u && slot_accepted(r, node, w0, slot, pad_limit);
+        imask = (w0.w >> 24) & 0xffu;
+        base = w1.x;
+        internal = hit && ((imask >> slot) & 1u);
+        if (hit && !internal) {
+            count = meta >> 5;
+            leaf = w1.y + (meta & 31u);
+        }
+    }
+    const unsigned long long im = __ballot(internal);
+    if (on) g = NodeGroup{base, (unsigned)(im >> (__lane_id() & ~(unsigned)(kCoopLanes - 1))) & 0xffu, imask};
+}
+
+// The rays of the busy lanes bm (at most kCoopRays) traced to their ends by
+// kCoopLanes lanes each.  Every lane of the wave calls, with its query's state;
+// no candidate waits.  `lds`: the workgroup's node-group stacks.
+template <bool CULL, bool F64, int STACK, class R, class Begin, class Finish>
+__device__ inline void coop_closest(unsigned long long bm, long long item, R& r, ClosestState& s, LdsStack<STACK>& st,
+                                    const NodeSlot* const& nodes, const Tri48* const& tris, const double* tri64,
+                                    Begin begin, Finish finish)
+{
+    const int owner = coop_owner(bm), from = owner < 0 ? 0 : owner;
+    bool on = owner >= 0;
+    item = shfl_i64(item, from);
+    ClosestState h;
+    h.g = NodeGroup{(unsigned)__shfl((int)s.g.base, from), (unsigned)__shfl((int)s.g.hits, from),
+                    (unsigned)__shfl((int)s.g.imask, from)};
+    h.best_leaf = (unsigned)__shfl((int)s.best_leaf, from);
+    h.best_id = __shfl(s.best_id, from);
+    h.tlim = __shfl(s.tlim, from);
+    h.best_t = shfl_f64(s.best_t, from);
+    const int sp = __shfl(st.sp, from);
+    LdsStack<STACK> gst = st;  // the owner's stack
+    gst.base = st.base + (from - (int)__lane_id());
+    gst.sp = sp;
+    if (on) begin(item, r, s);
+    s.g = h.g;
+    s.best_leaf = h.best_leaf;
+    s.best_id = h.best_id;
+    s.tlim = h.tlim;
+    s.best_t = h.best_t;
+    while (__ballot(on) != 0ull) {
+        unsigned leaf, count;
+        coop_visit(on, r, nodes, gst, s.g, s.tlim, leaf, count);
+        // This lane's closest certified triangle, compared in the order in which
+        // one lane would walk the slots: closer, then lower id, then lower slot.
+        double ct = kRiseInfinity;
+        int cid = 0;
+        unsigned cleaf = kNoLeaf;
+        for (; count; --count, ++leaf) {
+            if (!passes_filter<CULL, F64, false>(r, tris, tri64, leaf, s.faces, (float)s.best_t)) continue;
+            const float4* tp = reinterpret_cast<const float4*>(tris + leaf);
+            double tt;
+            if (F64 ? certify64(r, tri64 + 9 * (size_t)leaf, tt) : certify(r, tp[0], tp[1], tp[2], tt)) {
+                const int id = float_to_bits(tp[0].w);
+                if (cleaf == kNoLeaf || tt < ct || (tt == ct && id < cid)) {
+                    ct = tt;
+                    cid = id;
+                    cleaf = leaf;
+                }
+            }
+        }
+        if (__ballot(cleaf != kNoLeaf) != 0ull) {
+            // Leaf triangles of a node lie in slot order, so the lower leaf is the earlier one.
+            for (int d = 1; d < kCoopLanes; d <<= 1) {
+                const int peer = (int)__lane_id() ^ d;
+                const double pt = shfl_f64(ct, peer);
+                const int pid = __shfl(cid, peer);
+                const unsigned pleaf = (unsigned)__shfl((int)cleaf, peer);
+                const bool better = pleaf != kNoLeaf && (cleaf == kNoLeaf || pt < ct || (pt == ct && pid < cid) ||
+                                                         (pt == ct && pid == cid && pleaf < cleaf));
+                ct = better ? pt : ct;
+                cid = better ? pid : cid;
+                cleaf = better ? pleaf : cleaf;
+            }
+            if (cleaf != kNoLeaf && (ct < s.best_t || (ct == s.best_t && cid < s.best_id))) {
+                s.best_t = ct;
+                s.best_id = cid;
+                s.best_leaf = cleaf;
+                s.tlim = box_limit(r, s.best_t);
+            }
+        }
+        if (on && !next_group(gst, s.g)) {
+            if ((__lane_id() & (kCoopLanes - 1)) == 0) finish(item, r, s);
+            on = false;
+        }
+    }
+}
+
+// The same for any-hit queries: a group is done once one of its lanes
+// certifies a triangle within range.
+template <bool CULL, bool F64, int STACK, class R, class Begin, class Finish>
+__device__ inline void coop_any(unsigned long long bm, long long item, R& r, AnyState& s, LdsStack<STACK>& st,
+                                const NodeSlot* const& nodes, const Tri48* const& tris, const double* tri64,
+                                Begin begin, Finish finish)
+{
+    const int owner = coop_owner(bm), from = owner < 0 ? 0 : owner;
+    bool on = owner >= 0;
+    item = shfl_i64(item, from);
+    const NodeGroup g{(unsigned)__shfl((int)s.g.base, from), (unsigned)__shfl((int)s.g.hits, from),
+                      (unsigned)__shfl((int)s.g.imask, from)};
+    const int sp = __shfl(st.sp, from);
+    LdsStack<STACK> gst = st;
+    gst.base = st.base + (from - (int)__lane_id());
+    gst.sp = sp;
+    if (on) begin(item, r, s);
+    s.g = g;
+    while (__ballot(on) != 0ull) {
+        unsigned leaf, count;
+        coop_visit(on, r, nodes, gst, s.g, s.tlim, leaf, count);
+        bool hit = false;
+        for (; count && !hit; --count, ++leaf) {
+            if (!passes_filter<CULL, F64, true>(r, tris, tri64, leaf, s.faces, s.fbest)) continue;
+            s.pend = leaf;
+            any_commit<F64>(r, tris, tri64, s);
+            hit = s.hit;
+        }
+        const unsigned long long hm = __ballot(on && hit);
+        if (on) {
+            s.hit = ((hm >> (__lane_id() & ~(unsigned)(kCoopLanes - 1))) & 0xffull) != 0ull;
+            if (s.hit || !next_group(gst, s.g)) {
+                if ((__lane_id() & (kCoopLanes - 1)) == 0) finish(item, s);
+                on = false;
+            }
+        }
+    }
+}
+
+template <class Stack>
+struct CoopStack {
+    static constexpr bool value = false;  // a private array cannot be read by other lanes
+};
+template <int STACK>
+struct CoopStack<LdsStack<STACK>> {
+    static constexpr bool value = true;
 };
 
 // Closest-hit queries in persistent waves: each lane steps one query a node at
@@ -129,19 +358,27 @@ struct ItemFetch {
 // begin(item, r, s) starts a query, or returns false to skip the item;
 // finish(item, r, s) takes its result.
 template <bool COUNT, bool CULL, bool F64, class R, class Stack, class Begin, class Finish>
-__device__ inline void persist_closest(Stack& st, int64_t n, unsigned long long* next, unsigned& nn, unsigned& nt,
+__device__ inline void persist_closest(Stack& st, const ItemSource& items, unsigned& nn, unsigned& nt,
                                        const NodeSlot* const& nodes, const Tri48* const& tris, const double* tri64,
                                        Begin begin, Finish finish)
 {
     R r;
     ClosestState s;
     s.pend = kNoLeaf;
-    ItemFetch fetch(next, n);
+    ItemFetch fetch(items);
     long long item = -1;
     bool busy = false;
     for (;;) {
         if (busy) busy = closest_step<COUNT, CULL, F64, !COUNT>(r, nodes, tris, st, s, nn, nt, tri64);
         const unsigned long long bm = __ballot(busy);
+        if constexpr (CoopStack<Stack>::value && !COUNT) {
+            if (!fetch.more && bm != 0ull && __popcll(bm) <= kCoopRays) {
+                if (item >= 0 && s.pend != kNoLeaf) closest_commit<F64>(r, tris, tri64, s);
+                if (!busy && item >= 0) finish(item, r, s);
+                coop_closest<CULL, F64>(bm, item, r, s, st, nodes, tris, tri64, begin, finish);
+                break;
+            }
+        }
         if (bm == 0ull || (fetch.more && __popcll(bm) <= 64 - RISE_REFILL)) {
             if (!busy && item >= 0) {
                 if (s.pend != kNoLeaf) closest_commit<F64>(r, tris, tri64, s);
@@ -171,13 +408,13 @@ __device__ inline void persist_closest(Stack& st, int64_t n, unsigned long long*
 // the other idle lanes' when the wave refills, or, once no items are left to
 // fetch, when a quarter as many wait as are busy; one that fails goes on.
 template <bool COUNT, bool CULL, bool F64, class R, class Stack, class Begin, class Finish>
-__device__ inline void persist_any(Stack& st, int64_t n, unsigned long long* next, unsigned& nn, unsigned& nt,
+__device__ inline void persist_any(Stack& st, const ItemSource& items, unsigned& nn, unsigned& nt,
                                    const NodeSlot* const& nodes, const Tri48* const& tris, const double* tri64,
                                    Begin begin, Finish finish)
 {
     R r;
     AnyState s;
-    ItemFetch fetch(next, n);
+    ItemFetch fetch(items);
     long long item = -1;
     bool busy = false;
     for (;;) {
@@ -204,6 +441,23 @@ __device__ inline void persist_any(Stack& st, int64_t n, unsigned long long* nex
                     if (busy) item = got;
                 }
             } else if (__ballot(busy) == 0ull) {
+                break;
+            }
+        }
+        if constexpr (CoopStack<Stack>::value && !COUNT) {
+            // Few rays left and none to fetch: first certify what waits.
+            if (!fetch.more && __popcll(__ballot(item >= 0)) <= kCoopRays) {
+                if (!busy && item >= 0) {
+                    if (!s.hit && s.pend != kNoLeaf) any_commit<F64>(r, tris, tri64, s);
+                    if (s.hit || s.over) {
+                        finish(item, s);
+                        item = -1;
+                    } else {
+                        busy = true;
+                    }
+                }
+                const unsigned long long left = __ballot(busy);
+                if (left != 0ull) coop_any<CULL, F64>(left, item, r, s, st, nodes, tris, tri64, begin, finish);
                 break;
             }
         }
