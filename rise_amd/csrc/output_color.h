@@ -53,18 +53,50 @@ RISE_HD inline bool clip_edge(P2 c, P2 a, P2 b, P2 w, P2& out)
     return on_segment(w, c, out);
 }
 
+constexpr P2 kRed{0.640, 0.330}, kGreen{0.300, 0.600}, kBlue{0.150, 0.060}, kWhite{0.3127, 0.3290};
+
+// Where a chromaticity moves to (false: nowhere), by the edges in order.
+RISE_HD inline bool clip_chromaticity(P2 c, P2& hit)
+{
+    return clip_edge(c, kRed, kGreen, kWhite, hit) || clip_edge(c, kRed, kBlue, kWhite, hit) ||
+           clip_edge(c, kBlue, kGreen, kWhite, hit);
+}
+
+// The same with one edge's divisions instead of up to three edges': the sector
+// between two vertices, seen from the white point, holds the only edge that c's
+// ray can meet; the others' lines meet it behind the white point, which
+// clip_edge refuses.  c too near a sector's border, the vertical through the
+// white point or infinity for rounding to be ruled out is left to
+// clip_chromaticity.  The edge's expressions are those of clip_edge, so the
+// result is the same to the bit; no edge takes a NaN.
+RISE_HD inline bool clip_chromaticity_quick(P2 c, P2& hit)
+{
+    if (c.x != c.x || c.y != c.y) return false;
+    const double dx = c.x - kWhite.x, dy = c.y - kWhite.y;
+    const double tr = (kRed.x - kWhite.x) * dy - (kRed.y - kWhite.y) * dx;
+    const double tg = (kGreen.x - kWhite.x) * dy - (kGreen.y - kWhite.y) * dx;
+    const double tb = (kBlue.x - kWhite.x) * dy - (kBlue.y - kWhite.y) * dx;
+    const double eps = 1e-7;
+    const bool clear = fabs(tr) > eps && fabs(tg) > eps && fabs(tb) > eps && fabs(dx) > 1e-6 && fabs(dx) < 4.0 &&
+                       fabs(dy) < 4.0;
+    if (!clear) return clip_chromaticity(c, hit);
+    const bool rg = tr > 0.0 && tg < 0.0, bg = tg > 0.0 && tb < 0.0;  // else red-blue
+    const P2 a{bg ? kBlue.x : kRed.x, bg ? kBlue.y : kRed.y};
+    const P2 b{rg || bg ? kGreen.x : kBlue.x, rg || bg ? kGreen.y : kBlue.y};
+    return clip_edge(c, a, b, kWhite, hit);
+}
+
 // MoveXYZIntoRec709RGBGamut + XYZtoRec709RGB (ColorUtils.cpp:351-363,
 // Color.cpp:214-220): chromaticities outside the Rec.709 triangle move
 // toward the white point onto its edge (red-green, red-blue, blue-green
 // tried in that order), luminance kept; then the XYZ -> Rec.709 matrix.
+template <bool QUICK = false>
 RISE_HD inline void xyz_to_rec709(double X, double Y, double Z, double rgb[3])
 {
-    const P2 red{0.640, 0.330}, green{0.300, 0.600}, blue{0.150, 0.060}, white{0.3127, 0.3290};
     const double ovs = 1.0 / (X + Y + Z);
     const P2 c{X * ovs, Y * ovs};
     P2 hit{0.0, 0.0};
-    if (clip_edge(c, red, green, white, hit) || clip_edge(c, red, blue, white, hit) ||
-        clip_edge(c, blue, green, white, hit)) {
+    if (QUICK ? clip_chromaticity_quick(c, hit) : clip_chromaticity(c, hit)) {
         const double prod = (1.0 / hit.y) * Y;
         X = prod * hit.x;
         Z = prod * (1 - hit.x - hit.y);
@@ -123,17 +155,14 @@ struct Params {
     double exposure;    // 2^EV
 };
 
-// The pixel as the writer sees it before integerizing: RISEPel after the
-// optional DisplayTransformWriter, converted to the output colour space.
-RISE_HD inline void pixel_colour(const Params& p, float fx, float fy, float fz, double out[3])
+// The pixel as the writer sees it before integerizing, RISEPel after the
+// optional DisplayTransformWriter, but for the output colour space's curve.
+template <bool QUICK>
+RISE_HD inline void pixel_linear(const Params& p, float fx, float fy, float fz, double out[3])
 {
-    double c[3];
-    xyz_to_rec709((double)fx, (double)fy, (double)fz, c);
+    xyz_to_rec709<QUICK>((double)fx, (double)fy, (double)fz, out);
     if (p.tone)
-        for (int k = 0; k < 3; ++k) c[k] = display_curve(p.display, c[k] * p.exposure);
-    if (p.color_space == 1)
-        for (int k = 0; k < 3; ++k) c[k] = srgb_oetf(c[k]);
-    for (int k = 0; k < 3; ++k) out[k] = c[k];
+        for (int k = 0; k < 3; ++k) out[k] = display_curve(p.display, out[k] * p.exposure);
 }
 
 // Color_Template::Integerize (Color_Template.h:129-134): clamp to [0, 1],
@@ -144,6 +173,26 @@ RISE_HD inline T integerize(double v, double maxv)
     if (v > 1.0) v = 1.0;
     if (v < 0.0) v = 0.0;
     return (T)(v * maxv);
+}
+
+// integerize(srgb_oetf(x), maxv) without the 64-bit power function, which is
+// 60% of the output stage's instructions: x^(1/2.4) from 32-bit log2 and exp2
+// (relative error e below 1e-6, 7e-7 by their error bounds) and one Newton step
+// of y^12 = x^5 in 64 bits, whose error is 5.5 e^2 < 6e-12.  Where that could
+// change the truncated value (v within 1e-10 of the scale of a whole number)
+// the power function decides.
+template <class T>
+RISE_HD inline T integerize_srgb(double x, double maxv)
+{
+    if (x <= 0.003040247678) return integerize<T>(12.92 * x, maxv);  // 0 at 0
+    if (x == 1.0) return integerize<T>(1.055 * 1.0 - 0.055, maxv);
+    if (x > 1.01) return integerize<T>(1.0, maxv);
+    const double y = (double)exp2f(log2f((float)x) * (float)(1.0 / 2.4));
+    const double x2 = x * x, y2 = y * y, y4 = y2 * y2, y12 = y4 * y4 * y4;
+    const double root = y + y * (double)((float)(x2 * x2 * x - y12) / (12.0f * (float)y12));
+    const double v = (1.055 * root - 0.055) * maxv, g = 1e-10 * maxv;
+    if (floor(v - g) == floor(v + g)) return integerize<T>(1.055 * root - 0.055, maxv);
+    return integerize<T>(srgb_oetf(x), maxv);  // also NaN
 }
 
 // HDRWriter::WriteHDRPixelToBuffer (RasterImages/HDRWriter.h:37-58): shared
