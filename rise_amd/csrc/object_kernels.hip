@@ -1,9 +1,10 @@
 // object_kernels.hip -- batch closest-hit and any-hit kernels over a scene of
 // objects with transforms (object_trace.h).  Persistent waves, one ray per
-// lane at a time: each lane steps its query (the world tree, then the
-// top-level tree over the transformed objects and the trees of the objects it
-// reaches) and takes a new ray when it ends.  The node-group stack is in LDS
-// when the trees are shallow enough, else in a private array.
+// lane at a time: each lane's query is in one of three phases (the world tree,
+// an object's tree, the top-level walk between them), a wave runs the phases of
+// enough lanes in each round, and a lane takes a new ray when its query ends.
+// The node-group stack is in LDS when the trees are shallow enough, else in a
+// private array.
 #include "object_kernels.h"
 
 #include "object_trace.h"
@@ -17,10 +18,11 @@ namespace {
 
 constexpr int kObjBlock = 128;
 
-// Idle lanes at which a wave takes new rays.
-#ifndef RISE_REFILL_OBJ
-#define RISE_REFILL_OBJ 20
-#endif
+// Idle lanes at which a wave takes new rays, and waiting candidates at which it
+// certifies them.  A ray's walk over several trees is long, and 500,000 rays
+// are two or three a lane, so lanes are not left idle: 500,000 rays into 16
+// objects take 2041 us at 20 idle lanes, 2004 at 14, 1980 at 8.
+constexpr int kRefill = 8, kCertify = 2;
 
 __device__ inline void load_ray6(const float* __restrict__ rays, int64_t n, int64_t i, float ray[6])
 {
@@ -28,13 +30,20 @@ __device__ inline void load_ray6(const float* __restrict__ rays, int64_t n, int6
     for (int k = 0; k < 6; ++k) ray[k] = rays[(int64_t)k * n + i];
 }
 
-// The node-group stack: LDS entries per lane when the scene's trees fit
-// (kObjLds), else a private array.
-constexpr int kObjLds = 24;
+// The node-group stack: LDS entries per lane when the scene's trees fit into
+// kObjLds of them, else a private array (0).  Closest hits of more rays than the
+// lanes that are resident so (three waves per SIMD) take kObjLdsSmall entries
+// where those are enough: LDS and, with some spills, registers for four waves.
+// Records of 30,000 / 200,000 / 500,000 / 1,000,000 rays: 484 / 1382 / 4773 /
+// 15,376 us before, 505 / 1270 / 3530 / 11,030 with four waves, 442 us for the
+// 30,000 with three.  Any-hit queries lose by it (200,000 rays 430 -> 484 us) and
+// keep three.
+constexpr int kObjLdsSmall = 16, kObjLds = 24;
+constexpr int obj_waves(int stack) { return stack == kObjLdsSmall ? 4 : 1; }
 
 template <int STACK>
 struct StackOf {
-    using type = ObjLdsStack<kObjLds>;
+    using type = ObjLdsStack<STACK>;
 };
 template <>
 struct StackOf<0> {
@@ -45,7 +54,7 @@ template <int STACK>
 __device__ inline typename StackOf<STACK>::type make_stack(uint2* lds)
 {
     if constexpr (STACK > 0) {
-        return ObjLdsStack<kObjLds>{lds + threadIdx.x, kObjBlock, 0, 0, false};
+        return ObjLdsStack<STACK>{lds + threadIdx.x, kObjBlock, 0, 0, false};
     } else {
         ObjStack st;
         st.sp = st.base = 0;
@@ -53,6 +62,27 @@ __device__ inline typename StackOf<STACK>::type make_stack(uint2* lds)
         return st;
     }
 }
+
+// Which phases a wave runs in this round: those of at least a kVote-th of its
+// busy lanes, so that no phase's code runs for few of them; the others' lanes
+// wait until they are more, or the rest is done.  One of the three always has a
+// third of the lanes.  500,000 rays into 16 objects: 2178 us with every phase
+// of every lane in each round and candidates certified one by one; 2225 / 2076 /
+// 2039 / 2032 at a third / quarter / eighth / sixteenth, the last two with the
+// refill line at 20 and 14.
+constexpr int kVote = 8;
+struct PhaseVote {
+    int n;  // busy lanes
+    bool world, object, next;
+    __device__ inline explicit PhaseVote(int phase)
+    {
+        const int w = __popcll(__ballot(phase == kObjPhaseWorld)), o = __popcll(__ballot(phase == kObjPhaseObject));
+        n = __popcll(__ballot(phase != kObjPhaseDone));
+        world = w * kVote >= n;
+        object = o * kVote >= n;
+        next = (n - w - o) * kVote >= n;
+    }
+};
 
 __global__ void reset_fetch(unsigned long long* c) { *c = 0ull; }
 
@@ -67,43 +97,54 @@ static_assert(sizeof(ObjectHit) <= sizeof(rise_hip_hit) && alignof(ObjectHit) <=
 // lanes finish; a query that has ended is written out when its wave fetches.  REC: stage the ObjectHit in hits[ray] for object_records;
 // else write prim_id and t (float world range).
 template <int A, bool REC, int STACK>
-__global__ __launch_bounds__(kObjBlock) void closest_objects(ObjectSceneView sc, const float* __restrict__ rays,
+__global__ __launch_bounds__(kObjBlock, obj_waves(STACK)) void closest_objects(ObjectSceneView sc, const float* __restrict__ rays,
                                                              int64_t n, unsigned faces, int32_t* __restrict__ prim_id,
                                                              float* __restrict__ t_out,
                                                              rise_hip_hit* __restrict__ hits,
                                                              unsigned long long* next)
 {
-    __shared__ uint2 lds[STACK > 0 ? kObjLds * kObjBlock : 1];
+    __shared__ uint2 lds[STACK > 0 ? STACK * kObjBlock : 1];
     auto st = make_stack<STACK>(lds);
     ObjClosestQuery<A> Q;
     ItemFetch fetch(grid_items(next, n));
     long long ray = -1;
-    bool busy = false;
+    Q.phase = kObjPhaseDone;
+    Q.s.pend = kNoLeaf;
     for (;;) {
-        if (busy) busy = objects_closest_step(sc, st, Q);
+        const bool busy = Q.phase != kObjPhaseDone;
         const unsigned long long bm = __ballot(busy);
-        if (bm != 0ull && !(fetch.more && __popcll(bm) <= 64 - RISE_REFILL_OBJ)) continue;
-        if (!busy && ray >= 0) {
-            if (REC) {
-                *reinterpret_cast<ObjectHit*>(hits + ray) = Q.h;
-            } else {
-                prim_id[ray] = Q.h.prim_id;
-                t_out[ray] = Q.h.prim_id >= 0 ? (float)Q.h.range : INFINITY;
+        if (bm == 0ull || (fetch.more && __popcll(bm) <= 64 - kRefill)) {
+            if (!busy && ray >= 0) {
+                if (REC) {
+                    *reinterpret_cast<ObjectHit*>(hits + ray) = Q.h;
+                } else {
+                    prim_id[ray] = Q.h.prim_id;
+                    t_out[ray] = Q.h.prim_id >= 0 ? (float)Q.h.range : INFINITY;
+                }
+                ray = -1;
             }
-            ray = -1;
-        }
-        if (fetch.more) {
-            const long long got = fetch.take(busy);
-            if (got >= 0) {
-                float r6[6];
-                load_ray6(rays, n, got, r6);
-                objects_closest_begin(sc, r6, faces, st, Q);
-                ray = got;
-                busy = true;
+            if (fetch.more) {
+                const long long got = fetch.take(busy);
+                if (got >= 0) {
+                    float r6[6];
+                    load_ray6(rays, n, got, r6);
+                    objects_closest_begin(sc, r6, faces, st, Q);
+                    ray = got;
+                }
+            } else if (bm == 0ull) {
+                break;
             }
-        } else if (bm == 0ull) {
-            break;
         }
+        const PhaseVote vote(Q.phase);
+        if (vote.world && Q.phase == kObjPhaseWorld) objects_closest_world<true>(sc, st, Q);
+        if (vote.object && Q.phase == kObjPhaseObject) objects_closest_object<true>(st, Q);
+        const bool waits = (Q.phase == kObjPhaseWorld || Q.phase == kObjPhaseObject) && Q.s.pend != kNoLeaf;
+        const int waiting = __popcll(__ballot(waits));
+        if (waiting >= kCertify || waiting * 8 >= vote.n) {
+            if (waits) objects_closest_commit(sc, Q);
+        }
+        if (vote.next && Q.phase != kObjPhaseWorld && Q.phase != kObjPhaseObject && Q.phase != kObjPhaseDone)
+            objects_closest_next(sc, st, Q);
     }
 }
 
@@ -127,32 +168,37 @@ __global__ __launch_bounds__(kObjBlock) void any_objects(ObjectSceneView sc, con
                                                          const float* __restrict__ tmax, int64_t n, unsigned faces,
                                                          uint8_t* __restrict__ occluded, unsigned long long* next)
 {
-    __shared__ uint2 lds[STACK > 0 ? kObjLds * kObjBlock : 1];
+    __shared__ uint2 lds[STACK > 0 ? STACK * kObjBlock : 1];
     auto st = make_stack<STACK>(lds);
     ObjAnyQuery<A> Q;
     ItemFetch fetch(grid_items(next, n));
     long long ray = -1;
-    bool busy = false;
+    Q.phase = kObjPhaseDone;
     for (;;) {
-        if (busy) busy = objects_any_step(sc, st, Q);
+        const bool busy = Q.phase != kObjPhaseDone;
         const unsigned long long bm = __ballot(busy);
-        if (bm != 0ull && !(fetch.more && __popcll(bm) <= 64 - RISE_REFILL_OBJ)) continue;
-        if (!busy && ray >= 0) {
-            occluded[ray] = Q.hit ? 1 : 0;
-            ray = -1;
-        }
-        if (fetch.more) {
-            const long long got = fetch.take(busy);
-            if (got >= 0) {
-                float r6[6];
-                load_ray6(rays, n, got, r6);
-                objects_any_begin(sc, r6, tmax ? (double)tmax[got] : kRiseInfinity, faces, st, Q);
-                ray = got;
-                busy = true;
+        if (bm == 0ull || (fetch.more && __popcll(bm) <= 64 - kRefill)) {
+            if (!busy && ray >= 0) {
+                occluded[ray] = Q.hit ? 1 : 0;
+                ray = -1;
             }
-        } else if (bm == 0ull) {
-            break;
+            if (fetch.more) {
+                const long long got = fetch.take(busy);
+                if (got >= 0) {
+                    float r6[6];
+                    load_ray6(rays, n, got, r6);
+                    objects_any_begin(sc, r6, tmax ? (double)tmax[got] : kRiseInfinity, faces, st, Q);
+                    ray = got;
+                }
+            } else if (bm == 0ull) {
+                break;
+            }
         }
+        const PhaseVote vote(Q.phase);
+        if (vote.world && Q.phase == kObjPhaseWorld) objects_any_world(sc, st, Q);
+        if (vote.object && Q.phase == kObjPhaseObject) objects_any_object(st, Q);
+        if (vote.next && Q.phase != kObjPhaseWorld && Q.phase != kObjPhaseObject && Q.phase != kObjPhaseDone)
+            objects_any_next(sc, st, Q);
     }
 }
 
@@ -193,12 +239,14 @@ hipError_t launch_closest_objects(const ObjectSceneView& sc, int arith, int stac
             RISE_OBJ_CLOSEST_K(A, false, S);                                                     \
         }                                                                                        \
     } while (0)
-    const bool lds = stack_need <= kObjLds;
+    const bool many = n > (int64_t)kObjBlock * resident_grid(closest_objects<kArithIeee, true, kObjLds>, n);
     if (arith == kArithX86Fma) {
-        if (lds) RISE_OBJ_CLOSEST(kArithX86Fma, 1);
+        if (stack_need <= kObjLdsSmall && many) RISE_OBJ_CLOSEST(kArithX86Fma, kObjLdsSmall);
+        else if (stack_need <= kObjLds) RISE_OBJ_CLOSEST(kArithX86Fma, kObjLds);
         else RISE_OBJ_CLOSEST(kArithX86Fma, 0);
     } else {
-        if (lds) RISE_OBJ_CLOSEST(kArithIeee, 1);
+        if (stack_need <= kObjLdsSmall && many) RISE_OBJ_CLOSEST(kArithIeee, kObjLdsSmall);
+        else if (stack_need <= kObjLds) RISE_OBJ_CLOSEST(kArithIeee, kObjLds);
         else RISE_OBJ_CLOSEST(kArithIeee, 0);
     }
 #undef RISE_OBJ_CLOSEST
@@ -215,12 +263,11 @@ hipError_t launch_any_objects(const ObjectSceneView& sc, int arith, int stack_ne
 #define RISE_OBJ_ANY(A, S)                                                                               \
     any_objects<A, S><<<resident_grid(any_objects<A, S>, n), kObjBlock, 0, stream>>>(sc, rays, tmax, n, faces, \
                                                                                       occluded, next)
-    const bool lds = stack_need <= kObjLds;
     if (arith == kArithX86Fma) {
-        if (lds) RISE_OBJ_ANY(kArithX86Fma, 1);
+        if (stack_need <= kObjLds) RISE_OBJ_ANY(kArithX86Fma, kObjLds);
         else RISE_OBJ_ANY(kArithX86Fma, 0);
     } else {
-        if (lds) RISE_OBJ_ANY(kArithIeee, 1);
+        if (stack_need <= kObjLds) RISE_OBJ_ANY(kArithIeee, kObjLds);
         else RISE_OBJ_ANY(kArithIeee, 0);
     }
 #undef RISE_OBJ_ANY

@@ -165,8 +165,17 @@ struct ObjectHit {
     double p_world[3];
 };
 
-// Phases of an object query.
-enum : int { kObjPhaseWorld = 0, kObjPhaseTop = 1, kObjPhaseObject = 2, kObjPhaseDone = 3 };
+// Phases of an object query: a walk of the world's or of an object's tree, the
+// top-level walk that finds the next object (entered at the end of either), the
+// end.
+enum : int {
+    kObjPhaseWorld = 0,
+    kObjPhaseTop = 1,
+    kObjPhaseObject = 2,
+    kObjPhaseDone = 3,
+    kObjPhaseWorldEnd = 4,
+    kObjPhaseObjectEnd = 5
+};
 
 // ObjectManager::IntersectRay over the scene (each object's own closest hit,
 // Object::IntersectRay; the strictly closer world range wins, ties to the
@@ -233,15 +242,42 @@ RISE_HD inline void objects_closest_begin(const ObjectSceneView& sc, const float
     }
 }
 
-// One step; false once the query has ended (the hit is in Q.h).
-template <int A, class Stack>
-RISE_HD inline bool objects_closest_step(const ObjectSceneView& sc, Stack& st, ObjClosestQuery<A>& Q)
+// One step of the world tree's walk, and of an object's.  DEFER: as
+// closest_step's.
+template <bool DEFER, int A, class Stack>
+RISE_HD inline void objects_closest_world(const ObjectSceneView& sc, Stack& st, ObjClosestQuery<A>& Q)
 {
     unsigned nn = 0, nt = 0;
+    if (!closest_step<false, true, true, DEFER>(Q.r, sc.world_nodes, sc.world_tris, st, Q.s, nn, nt, sc.world_tri64))
+        Q.phase = kObjPhaseWorldEnd;
+}
+template <bool DEFER, int A, class Stack>
+RISE_HD inline void objects_closest_object(Stack& st, ObjClosestQuery<A>& Q)
+{
+    unsigned nn = 0, nt = 0;
+    if (!closest_step<false, true, true, DEFER>(Q.q, Q.nodes, Q.tris, st, Q.s, nn, nt, Q.tri64))
+        Q.phase = kObjPhaseObjectEnd;
+}
+
+// Certifies a walk's awaiting candidate.
+template <int A>
+RISE_HD inline void objects_closest_commit(const ObjectSceneView& sc, ObjClosestQuery<A>& Q)
+{
+    if (Q.s.pend == kNoLeaf) return;
+    if (Q.phase == kObjPhaseWorld || Q.phase == kObjPhaseWorldEnd)
+        closest_commit<true>(Q.r, sc.world_tris, sc.world_tri64, Q.s);
+    else closest_commit<true>(Q.q, Q.tris, Q.tri64, Q.s);
+}
+
+// From the end of a tree's walk to the next object's tree or the query's end:
+// keeps the walk's hit if it is the closest so far, then walks the top-level
+// tree on to the next object whose box can hold a closer one.
+template <int A, class Stack>
+RISE_HD inline void objects_closest_next(const ObjectSceneView& sc, Stack& st, ObjClosestQuery<A>& Q)
+{
     const double ow[3] = {Q.r.ox, Q.r.oy, Q.r.oz};
-    if (Q.phase == kObjPhaseWorld) {
-        if (closest_step<false, true, true>(Q.r, sc.world_nodes, sc.world_tris, st, Q.s, nn, nt, sc.world_tri64))
-            return true;
+    if (Q.phase != kObjPhaseTop) objects_closest_commit(sc, Q);
+    if (Q.phase == kObjPhaseWorldEnd) {
         if (Q.s.best_id >= 0) {
             const float4* tp = reinterpret_cast<const float4*>(sc.world_tris + Q.s.best_leaf);
             Q.h.prim_id = Q.s.best_id;
@@ -251,10 +287,8 @@ RISE_HD inline bool objects_closest_step(const ObjectSceneView& sc, Stack& st, O
             Q.h.range = world_range(Q.r, Q.s.best_t);
         }
         obj_closest_to_top(sc, Q);
-        return Q.phase != kObjPhaseDone;
-    }
-    if (Q.phase == kObjPhaseObject) {
-        if (closest_step<false, true, true>(Q.q, Q.nodes, Q.tris, st, Q.s, nn, nt, Q.tri64)) return true;
+        if (Q.phase == kObjPhaseDone) return;
+    } else if (Q.phase == kObjPhaseObjectEnd) {
         st.base = 0;  // back to the top-level walk's entries
         Q.phase = kObjPhaseTop;
         if (Q.s.best_id >= 0) {
@@ -272,18 +306,18 @@ RISE_HD inline bool objects_closest_step(const ObjectSceneView& sc, Stack& st, O
                 Q.w.tlim = obj_closest_limit(Q);
             }
         }
-        return true;
     }
-    if (Q.phase != kObjPhaseTop) return false;
-    const int k = top_step(Q.r, sc.top_nodes, sc.top_leaves, st, Q.w);
-    if (k == -2) {
-        Q.phase = kObjPhaseDone;
-        return false;
-    }
-    if (k < 0) return true;
-    const DevObject& ob = sc.objects[k];
     const double dw[3] = {Q.r.dx, Q.r.dy, Q.r.dz};
-    if (!world_box_reach(ob.lo, ob.hi, ow, dw, Q.r.len_d, Q.h.range)) return true;
+    int k;
+    do {
+        k = top_step(Q.r, sc.top_nodes, sc.top_leaves, st, Q.w);
+        if (k >= 0 && !world_box_reach(sc.objects[k].lo, sc.objects[k].hi, ow, dw, Q.r.len_d, Q.h.range)) k = -1;
+    } while (k == -1);
+    if (k < 0) {
+        Q.phase = kObjPhaseDone;
+        return;
+    }
+    const DevObject& ob = sc.objects[k];
     init_obj_ray(Q.q, ow, dw, ob.to_object);
     const BlasView bl = sc.blas[ob.blas];
     Q.nodes = bl.nodes;
@@ -302,7 +336,6 @@ RISE_HD inline bool objects_closest_step(const ObjectSceneView& sc, Stack& st, O
     st.base = st.sp;  // the object's entries go above the top-level walk's
     Q.k = k;
     Q.phase = kObjPhaseObject;
-    return true;
 }
 
 // The whole closest-hit query for one ray.
@@ -312,7 +345,10 @@ RISE_HD inline void objects_closest(const ObjectSceneView& sc, const float ray[6
 {
     ObjClosestQuery<A> Q;
     objects_closest_begin(sc, ray, faces, st, Q);
-    while (objects_closest_step(sc, st, Q)) {
+    while (Q.phase != kObjPhaseDone) {
+        if (Q.phase == kObjPhaseWorld) objects_closest_world<false>(sc, st, Q);
+        else if (Q.phase == kObjPhaseObject) objects_closest_object<false>(st, Q);
+        else objects_closest_next(sc, st, Q);
     }
     h = Q.h;
 }
@@ -451,53 +487,60 @@ RISE_HD inline void objects_any_begin(const ObjectSceneView& sc, const float ray
     }
 }
 
-// One step; false once the query has ended (the answer is in Q.hit).
+// One step of the world tree's walk, and of an object's.
 template <int A, class Stack>
-RISE_HD inline bool objects_any_step(const ObjectSceneView& sc, Stack& st, ObjAnyQuery<A>& Q)
+RISE_HD inline void objects_any_world(const ObjectSceneView& sc, Stack& st, ObjAnyQuery<A>& Q)
 {
     unsigned nn = 0, nt = 0;
-    if (Q.phase == kObjPhaseWorld) {
-        if (any_step<false, true, true>(Q.r, sc.world_nodes, sc.world_tris, st, Q.s, nn, nt, sc.world_tri64))
-            return true;
-        if (Q.s.hit) {
-            Q.hit = true;
-            Q.phase = kObjPhaseDone;
-            return false;
-        }
+    if (any_step<false, true, true>(Q.r, sc.world_nodes, sc.world_tris, st, Q.s, nn, nt, sc.world_tri64)) return;
+    Q.hit = Q.s.hit;
+    Q.phase = Q.hit ? kObjPhaseDone : kObjPhaseWorldEnd;
+}
+template <int A, class Stack>
+RISE_HD inline void objects_any_object(Stack& st, ObjAnyQuery<A>& Q)
+{
+    unsigned nn = 0, nt = 0;
+    if (any_step<false, true, true>(Q.q, Q.nodes, Q.tris, st, Q.s, nn, nt, Q.tri64)) return;
+    Q.hit = Q.s.hit;
+    Q.phase = Q.hit ? kObjPhaseDone : kObjPhaseObjectEnd;
+}
+
+// From the end of a tree's walk to the next object's tree or the query's end
+// (objects_closest_next).
+template <int A, class Stack>
+RISE_HD inline void objects_any_next(const ObjectSceneView& sc, Stack& st, ObjAnyQuery<A>& Q)
+{
+    if (Q.phase == kObjPhaseWorldEnd) {
         obj_any_to_top(sc, Q);
-        return Q.phase != kObjPhaseDone;
-    }
-    if (Q.phase == kObjPhaseObject) {
-        if (any_step<false, true, true>(Q.q, Q.nodes, Q.tris, st, Q.s, nn, nt, Q.tri64)) return true;
-        if (Q.s.hit) {
-            Q.hit = true;
-            Q.phase = kObjPhaseDone;
-            return false;
-        }
+        if (Q.phase == kObjPhaseDone) return;
+    } else if (Q.phase == kObjPhaseObjectEnd) {
         st.sp = st.base;  // back to the top-level walk's entries
         st.base = 0;
         Q.phase = kObjPhaseTop;
-        return true;
     }
-    if (Q.phase != kObjPhaseTop) return false;
-    const int k = top_step(Q.r, sc.top_nodes, sc.top_leaves, st, Q.w);
-    if (k == -2) {
-        Q.phase = kObjPhaseDone;
-        return false;
-    }
-    if (k < 0) return true;
-    const DevObject& ob = sc.objects[k];
     const double ow[3] = {Q.r.ox, Q.r.oy, Q.r.oz};
     const double dw[3] = {Q.r.dx, Q.r.dy, Q.r.dz};
-    init_obj_ray(Q.q, ow, dw, ob.to_object);
-    const double how_far2 = obj_how_far(Q.q.factor, Q.how_far);
-    // An object-space distance t along dn' is t |d| / |dl| along the world
-    // ray, so the limit reaches |d| how_far2 / |dl| in world space (widened
-    // by 1e-6 for the rounding of the two transforms).
-    const double lim = (how_far2 < kRiseInfinity && Q.q.mag > 0.0) ? how_far2 * Q.r.len_d / Q.q.mag * (1.0 + 1e-6)
-                                                                   : kRiseInfinity;
-    if (!world_box_reach(ob.lo, ob.hi, ow, dw, Q.r.len_d, lim)) return true;
-    const BlasView bl = sc.blas[ob.blas];
+    double how_far2 = kRiseInfinity;
+    int k;
+    do {
+        k = top_step(Q.r, sc.top_nodes, sc.top_leaves, st, Q.w);
+        if (k < 0) continue;
+        const DevObject& ob = sc.objects[k];
+        init_obj_ray(Q.q, ow, dw, ob.to_object);
+        how_far2 = obj_how_far(Q.q.factor, Q.how_far);
+        // An object-space distance t along dn' is t |d| / |dl| along the world
+        // ray, so the limit reaches |d| how_far2 / |dl| in world space (widened
+        // by 1e-6 for the rounding of the two transforms).
+        const double lim = (how_far2 < kRiseInfinity && Q.q.mag > 0.0)
+                               ? how_far2 * Q.r.len_d / Q.q.mag * (1.0 + 1e-6)
+                               : kRiseInfinity;
+        if (!world_box_reach(ob.lo, ob.hi, ow, dw, Q.r.len_d, lim)) k = -1;
+    } while (k == -1);
+    if (k < 0) {
+        Q.phase = kObjPhaseDone;
+        return;
+    }
+    const BlasView bl = sc.blas[sc.objects[k].blas];
     Q.nodes = bl.nodes;
     Q.tris = bl.tris;
     Q.tri64 = bl.tri64;
@@ -505,7 +548,6 @@ RISE_HD inline bool objects_any_step(const ObjectSceneView& sc, Stack& st, ObjAn
     Q.s.faces = Q.faces;
     st.base = st.sp;
     Q.phase = kObjPhaseObject;
-    return true;
 }
 
 // The whole any-hit query for one ray.
@@ -515,7 +557,10 @@ RISE_HD inline bool objects_any(const ObjectSceneView& sc, const float ray[6], d
 {
     ObjAnyQuery<A> Q;
     objects_any_begin(sc, ray, how_far, faces, st, Q);
-    while (objects_any_step(sc, st, Q)) {
+    while (Q.phase != kObjPhaseDone) {
+        if (Q.phase == kObjPhaseWorld) objects_any_world(sc, st, Q);
+        else if (Q.phase == kObjPhaseObject) objects_any_object(st, Q);
+        else objects_any_next(sc, st, Q);
     }
     return Q.hit;
 }
