@@ -179,11 +179,12 @@ enum : int {
 
 // ObjectManager::IntersectRay over the scene (each object's own closest hit,
 // Object::IntersectRay; the strictly closer world range wins, ties to the
-// lower object index, the caller's order) as a state machine advanced one
-// traversal step at a time, so that a persistent kernel can give a lane
-// whose query has ended a new ray while the other lanes of its wave go on.
-// Phases: the world tree, then the top-level walk, which enters the tree of
-// each object it reaches and resumes when that tree is done.
+// lower object index, the caller's order) as a state machine, so that
+// a persistent kernel can give a lane whose query has ended a new ray while the
+// other lanes of its wave go on, and run a phase for the lanes that are in it
+// together.  Phases: a step of the world tree's walk (objects_closest_world), a
+// step of an object's (objects_closest_object), and what lies between two trees
+// (objects_closest_next).
 template <int A>
 struct ObjClosestQuery {
     RayStateT<A> r;  // the world ray (world tree and top-level tree)

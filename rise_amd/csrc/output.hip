@@ -3,8 +3,8 @@
 // One kernel converts every pixel (colour pipeline of output_color.h, FP64)
 // into the bytes or floats the format stores; the host then frames them
 // (headers, row order, PNG's zlib stream, EXR's offset table) and writes the
-// file.  The kernel reads 12 bytes and writes 4-16 bytes per pixel: a
-// bandwidth-bound pass over a film already in HBM.
+// file.  The kernel reads 12 bytes and writes 4-16 bytes per pixel and is
+// bound by its 64-bit arithmetic (k_output).
 #include "rise_hip_output.h"
 
 #include "api_common.h"

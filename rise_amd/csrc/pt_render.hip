@@ -13,6 +13,9 @@
 //                                   (continuation queue)
 //                       connect(d)  any-hit for the shadow queue; adds the
 //                                   unoccluded contributions
+//   finish              all of these for what is left, in one launch: a pass
+//                       of few paths from its first bounce on, a large one
+//                       once few entries are left (k_finish)
 //   film                per-pixel FP32 Kahan sums over the chunk's samples
 // and one resolve per request at the end.  Every path carries its request
 // index, so paths of different scenes and image sizes share the queues.

@@ -2,9 +2,10 @@
 //
 // These replace the per-ray IObjectManager::IntersectRay / IntersectShadowRay
 // calls (Interfaces/IObjectManager.h:38-68, Managers/ObjectManager.cpp:270-373)
-// with one launch over a whole batch.  One lane per ray; the node-group stack
-// lives in LDS (16 entries per lane) when the tree is shallow enough, else in
-// a private array.
+// with one launch over a whole batch.  One lane per ray, eight where few
+// rays are left or given (wave_fetch.h); the node-group stack lives in LDS (8
+// or 16 entries per lane) when the tree is shallow enough, else in a private
+// array.
 #include "rise_hip.h"
 #include "trace_core.h"
 #include "trace_kernels.h"
