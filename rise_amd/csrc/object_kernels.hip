@@ -23,6 +23,7 @@ constexpr int kObjBlock = 128;
 // are two or three a lane, so lanes are not left idle: 500,000 rays into 16
 // objects take 2041 us at 20 idle lanes, 2004 at 14, 1980 at 8.
 constexpr int kRefill = 8, kCertify = 2;
+constexpr int kRefillAny = 20;  // any-hit queries
 
 __device__ inline void load_ray6(const float* __restrict__ rays, int64_t n, int64_t i, float ray[6])
 {
@@ -66,7 +67,8 @@ __device__ inline typename StackOf<STACK>::type make_stack(uint2* lds)
 // Which phases a wave runs in this round: those of at least a kVote-th of its
 // busy lanes, so that no phase's code runs for few of them; the others' lanes
 // wait until they are more, or the rest is done.  One of the three always has a
-// third of the lanes.  500,000 rays into 16 objects: 2178 us with every phase
+// third of the lanes.  (Any-hit queries step every phase in each round: with
+// votes 2,000,000 limited shadow rays take 3279 us instead of 2472.)  500,000 rays into 16 objects: 2178 us with every phase
 // of every lane in each round and candidates certified one by one; 2225 / 2076 /
 // 2039 / 2032 at a third / quarter / eighth / sixteenth, the last two with the
 // refill line at 20 and 14.
@@ -173,32 +175,27 @@ __global__ __launch_bounds__(kObjBlock) void any_objects(ObjectSceneView sc, con
     ObjAnyQuery<A> Q;
     ItemFetch fetch(grid_items(next, n));
     long long ray = -1;
-    Q.phase = kObjPhaseDone;
+    bool busy = false;
     for (;;) {
-        const bool busy = Q.phase != kObjPhaseDone;
+        if (busy) busy = objects_any_step(sc, st, Q);
         const unsigned long long bm = __ballot(busy);
-        if (bm == 0ull || (fetch.more && __popcll(bm) <= 64 - kRefill)) {
-            if (!busy && ray >= 0) {
-                occluded[ray] = Q.hit ? 1 : 0;
-                ray = -1;
-            }
-            if (fetch.more) {
-                const long long got = fetch.take(busy);
-                if (got >= 0) {
-                    float r6[6];
-                    load_ray6(rays, n, got, r6);
-                    objects_any_begin(sc, r6, tmax ? (double)tmax[got] : kRiseInfinity, faces, st, Q);
-                    ray = got;
-                }
-            } else if (bm == 0ull) {
-                break;
-            }
+        if (bm != 0ull && !(fetch.more && __popcll(bm) <= 64 - kRefillAny)) continue;
+        if (!busy && ray >= 0) {
+            occluded[ray] = Q.hit ? 1 : 0;
+            ray = -1;
         }
-        const PhaseVote vote(Q.phase);
-        if (vote.world && Q.phase == kObjPhaseWorld) objects_any_world(sc, st, Q);
-        if (vote.object && Q.phase == kObjPhaseObject) objects_any_object(st, Q);
-        if (vote.next && Q.phase != kObjPhaseWorld && Q.phase != kObjPhaseObject && Q.phase != kObjPhaseDone)
-            objects_any_next(sc, st, Q);
+        if (fetch.more) {
+            const long long got = fetch.take(busy);
+            if (got >= 0) {
+                float r6[6];
+                load_ray6(rays, n, got, r6);
+                objects_any_begin(sc, r6, tmax ? (double)tmax[got] : kRiseInfinity, faces, st, Q);
+                ray = got;
+                busy = true;
+            }
+        } else if (bm == 0ull) {
+            break;
+        }
     }
 }
 

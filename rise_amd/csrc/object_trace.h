@@ -488,60 +488,53 @@ RISE_HD inline void objects_any_begin(const ObjectSceneView& sc, const float ray
     }
 }
 
-// One step of the world tree's walk, and of an object's.
+// One step; false once the query has ended (the answer is in Q.hit).
 template <int A, class Stack>
-RISE_HD inline void objects_any_world(const ObjectSceneView& sc, Stack& st, ObjAnyQuery<A>& Q)
+RISE_HD inline bool objects_any_step(const ObjectSceneView& sc, Stack& st, ObjAnyQuery<A>& Q)
 {
     unsigned nn = 0, nt = 0;
-    if (any_step<false, true, true>(Q.r, sc.world_nodes, sc.world_tris, st, Q.s, nn, nt, sc.world_tri64)) return;
-    Q.hit = Q.s.hit;
-    Q.phase = Q.hit ? kObjPhaseDone : kObjPhaseWorldEnd;
-}
-template <int A, class Stack>
-RISE_HD inline void objects_any_object(Stack& st, ObjAnyQuery<A>& Q)
-{
-    unsigned nn = 0, nt = 0;
-    if (any_step<false, true, true>(Q.q, Q.nodes, Q.tris, st, Q.s, nn, nt, Q.tri64)) return;
-    Q.hit = Q.s.hit;
-    Q.phase = Q.hit ? kObjPhaseDone : kObjPhaseObjectEnd;
-}
-
-// From the end of a tree's walk to the next object's tree or the query's end
-// (objects_closest_next).
-template <int A, class Stack>
-RISE_HD inline void objects_any_next(const ObjectSceneView& sc, Stack& st, ObjAnyQuery<A>& Q)
-{
-    if (Q.phase == kObjPhaseWorldEnd) {
+    if (Q.phase == kObjPhaseWorld) {
+        if (any_step<false, true, true>(Q.r, sc.world_nodes, sc.world_tris, st, Q.s, nn, nt, sc.world_tri64))
+            return true;
+        if (Q.s.hit) {
+            Q.hit = true;
+            Q.phase = kObjPhaseDone;
+            return false;
+        }
         obj_any_to_top(sc, Q);
-        if (Q.phase == kObjPhaseDone) return;
-    } else if (Q.phase == kObjPhaseObjectEnd) {
+        return Q.phase != kObjPhaseDone;
+    }
+    if (Q.phase == kObjPhaseObject) {
+        if (any_step<false, true, true>(Q.q, Q.nodes, Q.tris, st, Q.s, nn, nt, Q.tri64)) return true;
+        if (Q.s.hit) {
+            Q.hit = true;
+            Q.phase = kObjPhaseDone;
+            return false;
+        }
         st.sp = st.base;  // back to the top-level walk's entries
         st.base = 0;
         Q.phase = kObjPhaseTop;
+        return true;
     }
+    if (Q.phase != kObjPhaseTop) return false;
+    const int k = top_step(Q.r, sc.top_nodes, sc.top_leaves, st, Q.w);
+    if (k == -2) {
+        Q.phase = kObjPhaseDone;
+        return false;
+    }
+    if (k < 0) return true;
+    const DevObject& ob = sc.objects[k];
     const double ow[3] = {Q.r.ox, Q.r.oy, Q.r.oz};
     const double dw[3] = {Q.r.dx, Q.r.dy, Q.r.dz};
-    double how_far2 = kRiseInfinity;
-    int k;
-    do {
-        k = top_step(Q.r, sc.top_nodes, sc.top_leaves, st, Q.w);
-        if (k < 0) continue;
-        const DevObject& ob = sc.objects[k];
-        init_obj_ray(Q.q, ow, dw, ob.to_object);
-        how_far2 = obj_how_far(Q.q.factor, Q.how_far);
-        // An object-space distance t along dn' is t |d| / |dl| along the world
-        // ray, so the limit reaches |d| how_far2 / |dl| in world space (widened
-        // by 1e-6 for the rounding of the two transforms).
-        const double lim = (how_far2 < kRiseInfinity && Q.q.mag > 0.0)
-                               ? how_far2 * Q.r.len_d / Q.q.mag * (1.0 + 1e-6)
-                               : kRiseInfinity;
-        if (!world_box_reach(ob.lo, ob.hi, ow, dw, Q.r.len_d, lim)) k = -1;
-    } while (k == -1);
-    if (k < 0) {
-        Q.phase = kObjPhaseDone;
-        return;
-    }
-    const BlasView bl = sc.blas[sc.objects[k].blas];
+    init_obj_ray(Q.q, ow, dw, ob.to_object);
+    const double how_far2 = obj_how_far(Q.q.factor, Q.how_far);
+    // An object-space distance t along dn' is t |d| / |dl| along the world
+    // ray, so the limit reaches |d| how_far2 / |dl| in world space (widened
+    // by 1e-6 for the rounding of the two transforms).
+    const double lim = (how_far2 < kRiseInfinity && Q.q.mag > 0.0) ? how_far2 * Q.r.len_d / Q.q.mag * (1.0 + 1e-6)
+                                                                   : kRiseInfinity;
+    if (!world_box_reach(ob.lo, ob.hi, ow, dw, Q.r.len_d, lim)) return true;
+    const BlasView bl = sc.blas[ob.blas];
     Q.nodes = bl.nodes;
     Q.tris = bl.tris;
     Q.tri64 = bl.tri64;
@@ -549,6 +542,7 @@ RISE_HD inline void objects_any_next(const ObjectSceneView& sc, Stack& st, ObjAn
     Q.s.faces = Q.faces;
     st.base = st.sp;
     Q.phase = kObjPhaseObject;
+    return true;
 }
 
 // The whole any-hit query for one ray.
@@ -558,10 +552,7 @@ RISE_HD inline bool objects_any(const ObjectSceneView& sc, const float ray[6], d
 {
     ObjAnyQuery<A> Q;
     objects_any_begin(sc, ray, how_far, faces, st, Q);
-    while (Q.phase != kObjPhaseDone) {
-        if (Q.phase == kObjPhaseWorld) objects_any_world(sc, st, Q);
-        else if (Q.phase == kObjPhaseObject) objects_any_object(st, Q);
-        else objects_any_next(sc, st, Q);
+    while (objects_any_step(sc, st, Q)) {
     }
     return Q.hit;
 }
