@@ -29,7 +29,14 @@ rise_hip_status rise_hip_debug_trace_host(const float* tris, int64_t n_tris, con
                                           float* t, uint8_t* occluded, uint64_t* counters,
                                           rise_hip_scene_stats* stats);
 
-/* The same over a .risemesh file's triangles (ids = file order), the 8-wide
+/* Closest hits of rise_hip_debug_trace_host (mode bit 1 as there, bit 0 clear)
+ * walked as the kernels' waves walk them: a step's last candidate waits for the
+ * certifier, which runs after a step or not, as a sequence drawn from `seed`
+ * has it.  The results do not depend on it. */
+rise_hip_status rise_hip_debug_trace_waiting_host(const float* tris, int64_t n_tris, const float* rays_soa, int64_t n,
+                                                  int32_t mode, uint32_t seed, int32_t* prim_id, float* t);
+
+/* rise_hip_debug_trace_host over a .risemesh file's triangles (ids = file order), the 8-wide
  * tree collapsed from the file's BVH2 cache when it is valid
  * (stats->bvh_source = 1), else built. */
 rise_hip_status rise_hip_debug_trace_host_risemesh(const rise_hip_risemesh* mesh, const float* rays_soa,

@@ -266,6 +266,67 @@ extern "C" rise_hip_status rise_hip_debug_trace_host(const float* tris, int64_t 
     return trace_host(bvh, n_tris, 0, rays, tmax, n, mode, prim_id, t, occluded, counters, stats);
 }
 
+extern "C" rise_hip_status rise_hip_debug_trace_waiting_host(const float* tris, int64_t n_tris, const float* rays,
+                                                             int64_t n, int32_t mode, uint32_t seed, int32_t* prim_id,
+                                                             float* t)
+{
+    clear_error();
+    if (n_tris < 0) return fail(RISE_HIP_ERR_INVALID_ARGUMENT, "negative count");
+    if (n_tris > 0 && !tris) return fail(RISE_HIP_ERR_INVALID_ARGUMENT, "NULL buffer");
+    if (mode & 1) return fail(RISE_HIP_ERR_INVALID_ARGUMENT, "mode must be 0 or 2");
+    rise_hip_status st = check_trace_args(rays, n, mode, prim_id, t, nullptr);
+    if (st != RISE_HIP_OK) return st;
+    WideBVH bvh;
+    std::string err;
+    try {
+        if (!build_wide_bvh(tris, n_tris, nullptr, BuildParams(), bvh, err))
+            return fail(RISE_HIP_ERR_BUILD, "BVH build failed: " + err);
+    } catch (const std::bad_alloc&) {
+        return fail(RISE_HIP_ERR_OUT_OF_MEMORY, "host allocation failed");
+    }
+    const NodeSlot* nodes = bvh.nodes.data();
+    const Tri48* trs = bvh.tris.data();
+    std::atomic<int64_t> next(0);
+    std::atomic<bool> overflow(false);
+    auto one = [&](auto r, int64_t i) {
+        init_ray(r, rays[i], rays[n + i], rays[2 * n + i], rays[3 * n + i], rays[4 * n + i], rays[5 * n + i]);
+        HostStack st;
+        unsigned nn = 0, nt = 0;
+        uint32_t x = (seed ^ ((uint32_t)i * 0x9e3779b9u)) | 1u;  // xorshift32
+        ClosestState s;
+        closest_begin(r, s);
+        while (closest_step<false, false, false, true>(r, nodes, trs, st, s, nn, nt)) {
+            x ^= x << 13;
+            x ^= x >> 17;
+            x ^= x << 5;
+            if (s.pend != kNoLeaf && (x & 3u) == 0u) closest_commit<false>(r, trs, nullptr, s);
+        }
+        if (s.pend != kNoLeaf) closest_commit<false>(r, trs, nullptr, s);
+        prim_id[i] = s.best_id;
+        t[i] = s.best_id >= 0 ? (float)world_range(r, s.best_t) : INFINITY;
+    };
+    auto worker = [&]() {
+        for (;;) {
+            const int64_t s0 = next.fetch_add(64);
+            if (s0 >= n) break;
+            for (int64_t i = s0; i < std::min<int64_t>(s0 + 64, n); ++i) {
+                try {
+                    if (mode & 2) one(RayStateT<kArithX86Fma>{}, i);
+                    else one(RayStateT<kArithIeee>{}, i);
+                } catch (const std::exception&) {
+                    overflow = true;
+                }
+            }
+        }
+    };
+    std::vector<std::thread> th;
+    for (int k = 1; k < host_threads(); ++k) th.emplace_back(worker);
+    worker();
+    for (auto& x : th) x.join();
+    if (overflow) return fail(RISE_HIP_ERR_BUILD, "traversal stack overflow");
+    return RISE_HIP_OK;
+}
+
 extern "C" rise_hip_status rise_hip_debug_trace_host_risemesh(const rise_hip_risemesh* mesh, const float* rays,
                                                               const float* tmax, int64_t n, int32_t mode,
                                                               int32_t* prim_id, float* t, uint8_t* occluded,

@@ -21,8 +21,9 @@ constexpr int kObjBlock = 128;
 // Idle lanes at which a wave takes new rays, and waiting candidates at which it
 // certifies them.  A ray's walk over several trees is long, and 500,000 rays
 // are two or three a lane, so lanes are not left idle: 500,000 rays into 16
-// objects take 2041 us at 20 idle lanes, 2004 at 14, 1980 at 8.
-constexpr int kRefill = 8, kCertify = 2;
+// objects took 2041 us at 20 idle lanes, 2004 at 14, 1980 at 8; 2137 / 2112 /
+// 2092 / 2080 at 1 / 2 / 4 / 8 waiting candidates.
+constexpr int kRefill = 8, kCertify = 8;
 constexpr int kRefillAny = 20;  // any-hit queries
 
 __device__ inline void load_ray6(const float* __restrict__ rays, int64_t n, int64_t i, float ray[6])

@@ -15,7 +15,10 @@
 // hit found so far, hence on traversal order; it can change the committed
 // hit only when the winner's float distance exceeds its double distance by
 // more than 1e-5 (the oracle flags such rays; none occur on the 1M-triangle
-// workload).
+// workload, many in scenes in units of hundreds).  So that a hit depends on the
+// ray and the tree alone, every form of the walk tests a triangle against the
+// best hit of all triangles before it, in the order of one lane that certifies
+// each candidate at once (closest_step).
 //
 // Stack: node groups (base index, 8-bit hit mask, 8-bit internal mask), at
 // most one per tree level, held in LDS (short stack, STACK entries per lane)
@@ -283,12 +286,18 @@ RISE_HD inline void init_obj_ray(ObjRayT<A>& r, const double ow[3], const double
 // normalized direction (PrepRayFloat, BVH.h:1212-1225).  `best` is the
 // caller's (float) current range.  Every operation is one IEEE float
 // operation in the reference's order (no contraction; 1/det correctly
-// rounded).  A triangle it rejects is never certified.
+// rounded).  A triangle it rejects is never certified.  t: the triangle's float
+// distance, once the tests before the range's have passed.
+constexpr float kFilterEps = 1e-5f;
+
+// The filter's range test.
+RISE_HD inline bool out_of_range(float t, float best) { return t > best + kFilterEps; }
+
 template <class R>
-RISE_HD inline bool filter_float(const R& r, const float4& a, const float4& b, const float4& c, float best)
+RISE_HD inline bool filter_float(const R& r, const float4& a, const float4& b, const float4& c, float best, float& t)
 {
     constexpr int A = R::kArith;
-    constexpr float kEps = 1e-5f;
+    constexpr float kEps = kFilterEps;
     const float e1x = b.x - a.x, e1y = b.y - a.y, e1z = b.z - a.z;
     const float e2x = c.x - a.x, e2y = c.y - a.y, e2z = c.z - a.z;
     const float pv0 = sub_prod<A>(r.fy, e2z, r.fz, e2y);
@@ -305,9 +314,8 @@ RISE_HD inline bool filter_float(const R& r, const float4& a, const float4& b, c
     const float qv2 = sub_prod<A>(tv0, e1y, tv1, e1x);
     const float v = dot3<A>(r.fx, qv0, r.fy, qv1, r.fz, qv2) * inv;
     if (v < -kEps || u + v > 1.0f + kEps) return false;
-    const float t = dot3<A>(e2x, qv0, e2y, qv1, e2z, qv2) * inv;
-    if (t < -kEps || t > best + kEps) return false;
-    return true;
+    t = dot3<A>(e2x, qv0, e2y, qv1, e2z, qv2) * inv;
+    return !(t < -kEps || out_of_range(t, best));
 }
 
 // FP64 Moller-Trumbore, RayTriangleIntersection.cpp:21-68, on v0 and the
@@ -705,22 +713,22 @@ RISE_HD inline bool next_group(Stack& st, NodeGroup& g)
 // CULL: apply the face selection `faces` (face_ok) before the filter.
 // F64: the triangles' double vertices are in tri64 (9 doubles per leaf
 // record, leaf order) and the certifier and face test use them.
+// t: filter_float's.
 template <bool CULL, bool F64, bool ANY, class R>
 RISE_HD inline bool passes_filter(const R& r, const Tri48* __restrict__ tris, const double* __restrict__ tri64,
-                                  unsigned leaf, unsigned faces, float best)
+                                  unsigned leaf, unsigned faces, float best, float& t)
 {
     const float4* tp = reinterpret_cast<const float4*>(tris + leaf);
     const float4 a = tp[0], b = tp[1], c = tp[2];
     if (CULL && faces != 3u && !(float_to_bits(c.w) & kTriDoubleSided) &&
         !(F64 ? face_ok64(r, tri64 + 9 * (size_t)leaf, faces) : face_ok(r, a, b, c, faces)))
         return false;
-    return filter_float(r, a, b, c, best) && !(ANY && (float_to_bits(c.w) & 1));
+    return filter_float(r, a, b, c, best, t) && !(ANY && (float_to_bits(c.w) & 1));
 }
 
-// A candidate that the filter has passed is certified later (below): the
-// certifier is some hundred double operations that one lane in thirty needs
-// per step, so running it at once costs a whole wave those instructions at
-// nearly every step.
+// A candidate that the filter has passed may wait for the certifier (below): that
+// is some hundred double operations that one lane in thirty needs per step, so
+// the candidates of a wave's lanes are certified together.
 constexpr unsigned kNoLeaf = 0xffffffffu;
 
 // Traversal state of one closest-hit query: the current node group, the best
@@ -795,24 +803,30 @@ RISE_HD inline void closest_commit(const R& r, const Tri48* __restrict__ tris, c
 // One traversal step: visit the next node and filter the triangles of its
 // leaf children; when the group is used up, pop the next one.  Returns false
 // once the traversal is over (a candidate may still be awaiting
-// closest_commit).  DEFER: a candidate waits for the caller's closest_commit,
-// or for the next candidate; else it is certified at once.  Waiting leaves the
-// box limit and the filter's range at the hit certified before, which visits
-// a few more nodes and changes no result: the certifier decides every hit.
+// closest_commit).  DEFER: a node's last candidate waits for the caller's
+// closest_commit, so that a wave certifies the candidates of its lanes
+// together; else each is certified at once.  Waiting changes no result: the walk
+// stands still meanwhile (a step does nothing), and a second candidate of the
+// same node has the first certified and takes the filter's range test again.
 template <bool COUNT, bool CULL = false, bool F64 = false, bool DEFER = false, class Stack, class R>
 RISE_HD inline bool closest_step(const R& r, const NodeSlot* __restrict__ nodes, const Tri48* __restrict__ tris,
                                  Stack& st, ClosestState& s, unsigned& n_nodes, unsigned& n_tris,
                                  const double* __restrict__ tri64 = nullptr)
 {
+    if (DEFER && s.pend != kNoLeaf) return true;
     LeafWalk w;
     visit_node<COUNT>(r, nodes, st, s.g, s.tlim, w, n_nodes);
     while (w.slots) {
         unsigned leaf;
+        float t;
         if (!next_triangle(w, leaf)) continue;
         if (COUNT) ++n_tris;
-        if (!passes_filter<CULL, F64, false>(r, tris, tri64, leaf, s.faces, (float)s.best_t)) continue;
+        if (!passes_filter<CULL, F64, false>(r, tris, tri64, leaf, s.faces, (float)s.best_t, t)) continue;
         if (DEFER) {
-            if (s.pend != kNoLeaf) closest_commit<F64>(r, tris, tri64, s);
+            if (s.pend != kNoLeaf) {
+                closest_commit<F64>(r, tris, tri64, s);
+                if (out_of_range(t, (float)s.best_t)) continue;
+            }
             s.pend = leaf;
         } else {
             s.pend = leaf;
@@ -894,9 +908,10 @@ RISE_HD inline bool any_step(const R& r, const NodeSlot* __restrict__ nodes, con
     visit_node<COUNT>(r, nodes, st, s.g, s.tlim, w, n_nodes);
     while (w.slots) {
         unsigned leaf;
+        float t;
         if (!next_triangle(w, leaf)) continue;
         if (COUNT) ++n_tris;
-        if (!passes_filter<CULL, F64, true>(r, tris, tri64, leaf, s.faces, s.fbest)) continue;
+        if (!passes_filter<CULL, F64, true>(r, tris, tri64, leaf, s.faces, s.fbest, t)) continue;
         const bool second = s.pend != kNoLeaf;
         if (!DEFER || second) {
             const unsigned first = s.pend;

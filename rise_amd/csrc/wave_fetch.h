@@ -24,11 +24,10 @@
 #ifndef RISE_CHUNK
 #define RISE_CHUNK 256
 #endif
-// Lanes whose candidate waits when the wave certifies: 2868 us at 1, 2853 at
-// 2, 2880 at 4, 2960 at 8 (the waiting rays visit nodes that the hit would
-// have culled); with vertex records and any-hit shadows alike 1-2%.
+// Lanes whose candidate waits when the wave certifies, the others going on: the
+// ray cast takes 2924 us at 1, 2848 at 2, 2803 at 4, 2790 at 8.
 #ifndef RISE_CERTIFY
-#define RISE_CERTIFY 2
+#define RISE_CERTIFY 8
 #endif
 
 namespace rise_hip {
@@ -156,7 +155,7 @@ struct ItemFetch {
 // Once a wave has at most kCoopRays rays left and none to fetch, each ray gets
 // kCoopLanes lanes: lane j of a group tests slot j ^ oinv of the ray's next
 // node, so one ballot gives every group its hit mask in visiting order, and the
-// lanes of accepted leaves test their triangles side by side.  A step is some
+// lanes of accepted leaves filter their triangles side by side.  A step is some
 // 120 instructions instead of 400, and what bounds the end of a launch (or a
 // launch of few rays) is the longest ray's chain of steps: 7072 rays into 20,000
 // triangles 107 -> 68 us, a million shadow rays into 200,000 574 -> 544 us (and
@@ -248,42 +247,29 @@ __device__ inline void coop_closest(unsigned long long bm, long long item, R& r,
     while (__ballot(on) != 0ull) {
         unsigned leaf, count;
         coop_visit(on, r, nodes, gst, s.g, s.tlim, leaf, count);
-        // This lane's closest certified triangle, compared in the order in which
-        // one lane would walk the slots: closer, then lower id, then lower slot.
-        double ct = kRiseInfinity;
-        int cid = 0;
-        unsigned cleaf = kNoLeaf;
-        for (; count; --count, ++leaf) {
-            if (!passes_filter<CULL, F64, false>(r, tris, tri64, leaf, s.faces, (float)s.best_t)) continue;
-            const float4* tp = reinterpret_cast<const float4*>(tris + leaf);
-            double tt;
-            if (F64 ? certify64(r, tri64 + 9 * (size_t)leaf, tt) : certify(r, tp[0], tp[1], tp[2], tt)) {
-                const int id = float_to_bits(tp[0].w);
-                if (cleaf == kNoLeaf || tt < ct || (tt == ct && id < cid)) {
-                    ct = tt;
-                    cid = id;
-                    cleaf = leaf;
+        // The lane's triangles that pass with the best hit before this node; then
+        // the group's, one after the other in the order of a single lane's walk
+        // (slots, their triangles), each in all lanes of the group alike: the
+        // range test again once another has been certified, and the certifier.
+        unsigned passed = 0;
+        float t;
+        for (unsigned k = 0; k < count; ++k)
+            if (passes_filter<CULL, F64, false>(r, tris, tri64, leaf + k, s.faces, (float)s.best_t, t)) passed |= 1u << k;
+        const unsigned lane0 = __lane_id() & ~(unsigned)(kCoopLanes - 1);
+        bool first = true;
+        for (;;) {
+            const unsigned long long pm = __ballot(passed != 0u);
+            if (pm == 0ull) break;
+            const unsigned gm = (unsigned)(pm >> lane0) & 0xffu;
+            const unsigned at = gm ? lane0 + (__builtin_ctz(xor_permute8(gm, r.oinv)) ^ r.oinv) : __lane_id();
+            const unsigned next = (unsigned)__shfl((int)(leaf + (passed ? __builtin_ctz(passed) : 0u)), (int)at);
+            if (at == __lane_id()) passed &= passed - 1u;
+            if (gm) {
+                if (first || passes_filter<CULL, F64, false>(r, tris, tri64, next, s.faces, (float)s.best_t, t)) {
+                    s.pend = next;
+                    closest_commit<F64>(r, tris, tri64, s);
                 }
-            }
-        }
-        if (__ballot(cleaf != kNoLeaf) != 0ull) {
-            // Leaf triangles of a node lie in slot order, so the lower leaf is the earlier one.
-            for (int d = 1; d < kCoopLanes; d <<= 1) {
-                const int peer = (int)__lane_id() ^ d;
-                const double pt = shfl_f64(ct, peer);
-                const int pid = __shfl(cid, peer);
-                const unsigned pleaf = (unsigned)__shfl((int)cleaf, peer);
-                const bool better = pleaf != kNoLeaf && (cleaf == kNoLeaf || pt < ct || (pt == ct && pid < cid) ||
-                                                         (pt == ct && pid == cid && pleaf < cleaf));
-                ct = better ? pt : ct;
-                cid = better ? pid : cid;
-                cleaf = better ? pleaf : cleaf;
-            }
-            if (cleaf != kNoLeaf && (ct < s.best_t || (ct == s.best_t && cid < s.best_id))) {
-                s.best_t = ct;
-                s.best_id = cid;
-                s.best_leaf = cleaf;
-                s.tlim = box_limit(r, s.best_t);
+                first = false;
             }
         }
         if (on && !next_group(gst, s.g)) {
@@ -316,7 +302,8 @@ __device__ inline void coop_any(unsigned long long bm, long long item, R& r, Any
         coop_visit(on, r, nodes, gst, s.g, s.tlim, leaf, count);
         bool hit = false;
         for (; count && !hit; --count, ++leaf) {
-            if (!passes_filter<CULL, F64, true>(r, tris, tri64, leaf, s.faces, s.fbest)) continue;
+            float t;
+            if (!passes_filter<CULL, F64, true>(r, tris, tri64, leaf, s.faces, s.fbest, t)) continue;
             s.pend = leaf;
             any_commit<F64>(r, tris, tri64, s);
             hit = s.hit;
@@ -347,8 +334,9 @@ struct CoopStack<LdsStack<STACK>> {
 //     idle (or none is busy); then all of them certify what still waits,
 //     finish (world range, stores) and take new items together, the new items
 //     claimed with one atomic per wave;
-//   * candidates that the filter has passed are certified once RISE_CERTIFY
-//     lanes, or an eighth of the busy ones, have one (closest_step's DEFER).
+//   * a candidate that the filter has passed waits, and its query with it, until
+//     RISE_CERTIFY lanes, or an eighth of the busy ones, have one
+//     (closest_step's DEFER).
 // Bound by instruction issue: the kernel's time follows its vector
 // instructions (2.15e9 a launch before, 1.9e9 now at 48 of 64 lanes busy).  On
 // the 1M-triangle, 6.07M-ray cast 3405 -> 2880 us against one claim per refill,

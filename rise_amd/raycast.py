@@ -332,6 +332,20 @@ def host_trace(tris: np.ndarray, rays: np.ndarray, mode: int = 0, tmax: np.ndarr
     return occ, counters, stats.as_dict()
 
 
+def host_trace_waiting(tris: np.ndarray, rays: np.ndarray, seed: int, arith: int = ARITH_IEEE):
+    """rise_hip_debug_trace_waiting_host: host_trace's closest hits with
+    candidates that wait for the certifier as `seed` has it (validation only).
+    Returns (prim_id, t)."""
+    tris = np.ascontiguousarray(tris, dtype=np.float32).reshape(-1, 9)
+    rays = np.ascontiguousarray(rays, dtype=np.float32)
+    n = rays.shape[1]
+    pid, t = np.empty(n, dtype=np.int32), np.empty(n, dtype=np.float32)
+    _lib.check(_lib.lib().rise_hip_debug_trace_waiting_host(
+        tris.ctypes.data, tris.shape[0], rays.ctypes.data, n, 2 if arith == ARITH_X86_FMA else 0, seed,
+        pid.ctypes.data, t.ctypes.data))
+    return pid, t
+
+
 def host_trace_ex(tris: np.ndarray, rays: np.ndarray, mode: int = 0, faces: int = FACES_BOTH,
                   tmax: np.ndarray | None = None, arith: int = ARITH_IEEE):
     """rise_hip_debug_trace_ex_host: the kernels' traversal with a face
