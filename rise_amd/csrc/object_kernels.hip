@@ -21,8 +21,8 @@ constexpr int kObjBlock = 128;
 // Idle lanes at which a wave takes new rays, and waiting candidates at which it
 // certifies them.  A ray's walk over several trees is long, and 500,000 rays
 // are two or three a lane, so lanes are not left idle: 500,000 rays into 16
-// objects took 2041 us at 20 idle lanes, 2004 at 14, 1980 at 8; 2137 / 2112 /
-// 2092 / 2080 at 1 / 2 / 4 / 8 waiting candidates.
+// objects took 2041 us at 20 idle lanes, 2004 at 14, 1980 at 8; 1926 / 1899 /
+// 1867 / 1862 at 1 / 2 / 4 / 8 waiting candidates.
 constexpr int kRefill = 8, kCertify = 8;
 constexpr int kRefillAny = 20;  // any-hit queries
 
@@ -131,7 +131,7 @@ __global__ __launch_bounds__(kObjBlock, obj_waves(STACK)) void closest_objects(O
                 if (got >= 0) {
                     float r6[6];
                     load_ray6(rays, n, got, r6);
-                    objects_closest_begin(sc, r6, faces, st, Q);
+                    objects_closest_begin(sc, r6, st, Q);
                     ray = got;
                 }
             } else if (bm == 0ull) {
@@ -139,8 +139,8 @@ __global__ __launch_bounds__(kObjBlock, obj_waves(STACK)) void closest_objects(O
             }
         }
         const PhaseVote vote(Q.phase);
-        if (vote.world && Q.phase == kObjPhaseWorld) objects_closest_world<true>(sc, st, Q);
-        if (vote.object && Q.phase == kObjPhaseObject) objects_closest_object<true>(st, Q);
+        if (vote.world && Q.phase == kObjPhaseWorld) objects_closest_world<true>(sc, faces, st, Q);
+        if (vote.object && Q.phase == kObjPhaseObject) objects_closest_object<true>(faces, st, Q);
         const bool waits = (Q.phase == kObjPhaseWorld || Q.phase == kObjPhaseObject) && Q.s.pend != kNoLeaf;
         const int waiting = __popcll(__ballot(waits));
         if (waiting >= kCertify || waiting * 8 >= vote.n) {

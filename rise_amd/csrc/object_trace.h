@@ -195,7 +195,6 @@ struct ObjClosestQuery {
     const NodeSlot* nodes;  // the tree of the object being traversed
     const Tri48* tris;
     const double* tri64;
-    unsigned faces;
     int k;  // its object record
     int phase;
 };
@@ -220,7 +219,7 @@ RISE_HD inline void obj_closest_to_top(const ObjectSceneView& sc, ObjClosestQuer
 }
 
 template <int A, class Stack>
-RISE_HD inline void objects_closest_begin(const ObjectSceneView& sc, const float ray[6], unsigned faces, Stack& st,
+RISE_HD inline void objects_closest_begin(const ObjectSceneView& sc, const float ray[6], Stack& st,
                                           ObjClosestQuery<A>& Q)
 {
     Q.h.prim_id = -1;
@@ -233,29 +232,30 @@ RISE_HD inline void objects_closest_begin(const ObjectSceneView& sc, const float
     st.base = 0;
     st.overflow = false;
     init_ray(Q.r, ray[0], ray[1], ray[2], ray[3], ray[4], ray[5]);
-    Q.faces = faces;
     if (sc.world_nodes) {
         closest_begin(Q.r, Q.s);
-        Q.s.faces = faces;
         Q.phase = kObjPhaseWorld;
     } else {
         obj_closest_to_top(sc, Q);
     }
 }
 
-// One step of the world tree's walk, and of an object's.  DEFER: as
+// One step of the world tree's walk, and of an object's, with the query's face
+// selection (an argument, so that it takes no register of a lane).  DEFER: as
 // closest_step's.
 template <bool DEFER, int A, class Stack>
-RISE_HD inline void objects_closest_world(const ObjectSceneView& sc, Stack& st, ObjClosestQuery<A>& Q)
+RISE_HD inline void objects_closest_world(const ObjectSceneView& sc, unsigned faces, Stack& st, ObjClosestQuery<A>& Q)
 {
     unsigned nn = 0, nt = 0;
+    Q.s.faces = faces;
     if (!closest_step<false, true, true, DEFER>(Q.r, sc.world_nodes, sc.world_tris, st, Q.s, nn, nt, sc.world_tri64))
         Q.phase = kObjPhaseWorldEnd;
 }
 template <bool DEFER, int A, class Stack>
-RISE_HD inline void objects_closest_object(Stack& st, ObjClosestQuery<A>& Q)
+RISE_HD inline void objects_closest_object(unsigned faces, Stack& st, ObjClosestQuery<A>& Q)
 {
     unsigned nn = 0, nt = 0;
+    Q.s.faces = faces;
     if (!closest_step<false, true, true, DEFER>(Q.q, Q.nodes, Q.tris, st, Q.s, nn, nt, Q.tri64))
         Q.phase = kObjPhaseObjectEnd;
 }
@@ -325,7 +325,6 @@ RISE_HD inline void objects_closest_next(const ObjectSceneView& sc, Stack& st, O
     Q.tris = bl.tris;
     Q.tri64 = bl.tri64;
     closest_begin(Q.q, Q.s);
-    Q.s.faces = Q.faces;
     if (Q.h.range < kRiseInfinity && Q.r.len_d > 0.0) {
         // A world range w is an object-space distance of about w |dl| / |d|;
         // the rounding of o' and of the point taken back to world space is
@@ -345,10 +344,10 @@ RISE_HD inline void objects_closest(const ObjectSceneView& sc, const float ray[6
                                     ObjectHit& h)
 {
     ObjClosestQuery<A> Q;
-    objects_closest_begin(sc, ray, faces, st, Q);
+    objects_closest_begin(sc, ray, st, Q);
     while (Q.phase != kObjPhaseDone) {
-        if (Q.phase == kObjPhaseWorld) objects_closest_world<false>(sc, st, Q);
-        else if (Q.phase == kObjPhaseObject) objects_closest_object<false>(st, Q);
+        if (Q.phase == kObjPhaseWorld) objects_closest_world<false>(sc, faces, st, Q);
+        else if (Q.phase == kObjPhaseObject) objects_closest_object<false>(faces, st, Q);
         else objects_closest_next(sc, st, Q);
     }
     h = Q.h;

@@ -216,15 +216,15 @@ RISE_HD inline void xform_normal(const double* minv, const double n[3], double o
 // (float)dn' (PrepRayFloat, BVH.h:1212-1225); the certifier sees o' and dn'.
 // The boxes are tested with the FP32 slab test of the float ray ((float)o',
 // (float)dn' scaled as in init_ray); o' is not a float, so each axis's plane
-// distances take the origin's rounding |o' - (float)o'| / d as extra slack
-// (the direction's rounding is relative, covered by RISE_SLAB_PAD).
+// distances take a bound of the origin's rounding |o' - (float)o'| / d as extra
+// slack (slab_axis_rounded; the direction's rounding is relative, covered by
+// RISE_SLAB_PAD).
 template <int A>
 struct ObjRayT {
     static constexpr int kArith = A;
     float ox, oy, oz;  // (float)o'
     float fx, fy, fz;  // (float)dn'
     float ix, iy, iz;  // slab inverses of (float)dn' scaled as in init_ray
-    float ex, ey, ez;  // extra slack per axis: |o' - (float)o'| |inverse| (1 + 2^-20)
     unsigned oinv;     // (~octant of (float)dn') & 7
     double o[3];       // o'
     double dn[3];      // dn'
@@ -275,9 +275,6 @@ RISE_HD inline void init_obj_ray(ObjRayT<A>& r, const double ow[3], const double
     const double f[3] = {r.fx, r.fy, r.fz};
     const double lf = sqrt(f[0] * f[0] + f[1] * f[1] + f[2] * f[2]);
     r.inv_len = lf > 0.0 ? (float)(1.0 / ldexp(lf, sh)) : 1.0f;
-    r.ex = (float)(fabs(r.o[0] - (double)r.ox) * fabs((double)r.ix) * (1.0 + 0x1p-20));
-    r.ey = (float)(fabs(r.o[1] - (double)r.oy) * fabs((double)r.iy) * (1.0 + 0x1p-20));
-    r.ez = (float)(fabs(r.o[2] - (double)r.oz) * fabs((double)r.iz) * (1.0 + 0x1p-20));
 }
 
 // BVH::MollerTrumboreFloat (Acceleration/BVH.h:1111-1167) on the leaf
@@ -473,15 +470,17 @@ RISE_HD inline SlabAxis slab_axis(float p, int e, float o, float inv)
     return SlabAxis{0.0f, 0.0f, -INFINITY, INFINITY};
 }
 
-// slab_axis for an origin known only to within `extra / |inv|` of o: the
-// plane distances widen by `extra` on top of their own slack (the sum, rounded
-// to nearest, is below 2^127 while |b| < 2^126 and extra < 2^125).
-RISE_HD inline SlabAxis slab_axis_widened(float p, int e, float o, float inv, float extra)
+// slab_axis for an origin o rounded to float from a double: the plane distances
+// widen by (2^-24 |o| (1 + 2^-20) + 2^-126) |inv| on top of their own slack.  A
+// float rounded to nearest is off by at most 2^-24 of itself, or by 2^-150 where
+// it is subnormal; the 2^-20 covers the roundings here.
+RISE_HD inline SlabAxis slab_axis_rounded(float p, int e, float o, float inv)
 {
     const float b = (p - o) * inv;
     const float s = ldexpf(inv, e);
-    const float slack = fmaf(fabsf(b), 0x1p-21f, 0x1p-100f) + extra * (1.0f + 0x1p-22f);
-    if (fabsf(b) < 0x1p126f && fabsf(s) < 0x1p119f && extra < 0x1p125f)
+    const float slack =
+        fmaf(fmaf(fabsf(o), 0x1.00001p-24f, 0x1p-126f), fabsf(inv), fmaf(fabsf(b), 0x1p-21f, 0x1p-100f));
+    if (fabsf(b) < 0x1p126f && fabsf(s) < 0x1p119f && slack < 0x1p125f)
         return SlabAxis{s, s * RISE_SLAB_PAD, b - slack, (b + slack) * RISE_SLAB_PAD};
     return SlabAxis{0.0f, 0.0f, -INFINITY, INFINITY};
 }
@@ -536,9 +535,9 @@ RISE_HD inline void slab_axes(const RayStateT<A>& r, const uint4& w0, SlabAxis& 
 template <int A>
 RISE_HD inline void slab_axes(const ObjRayT<A>& r, const uint4& w0, SlabAxis& ax, SlabAxis& ay, SlabAxis& az)
 {
-    ax = slab_axis_widened(bits_to_float(w0.x), (int)(signed char)(w0.w & 0xff), r.ox, r.ix, r.ex);
-    ay = slab_axis_widened(bits_to_float(w0.y), (int)(signed char)((w0.w >> 8) & 0xff), r.oy, r.iy, r.ey);
-    az = slab_axis_widened(bits_to_float(w0.z), (int)(signed char)((w0.w >> 16) & 0xff), r.oz, r.iz, r.ez);
+    ax = slab_axis_rounded(bits_to_float(w0.x), (int)(signed char)(w0.w & 0xff), r.ox, r.ix);
+    ay = slab_axis_rounded(bits_to_float(w0.y), (int)(signed char)((w0.w >> 8) & 0xff), r.oy, r.iy);
+    az = slab_axis_rounded(bits_to_float(w0.z), (int)(signed char)((w0.w >> 16) & 0xff), r.oz, r.iz);
 }
 
 template <class R>
