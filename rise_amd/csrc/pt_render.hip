@@ -70,8 +70,9 @@ constexpr int64_t kChunkPaths = int64_t(1) << 20;   // paths per chunk (at most)
 #endif
 constexpr int64_t kMaxPaths = int64_t(1) << RISE_MAX_PATHS_LOG2;  // paths in flight per pass (at most)
 // Per pass: extension rays, shadow rays and 4 binned-hit counts per depth,
-// then the index-of-refraction pushes dropped for lack of room and the bounce
-// from which k_finish has run the pass, plus one (0: none).
+// then the index-of-refraction pushes dropped for lack of room and the bounces
+// from which k_finish has run the pass (low half) and has run it to its end in
+// one launch (high half), each plus one (0: none).
 constexpr int kCounters = 6 * (kMaxPathDepth + 1) + 2;
 constexpr int kOverflowCounter = 6 * (kMaxPathDepth + 1);
 constexpr int kStopCounter = kOverflowCounter + 1;
@@ -218,7 +219,7 @@ struct Paths {
 // once k_finish has run it.
 __device__ inline bool finished(const Paths& S, int depth)
 {
-    const unsigned stop = *S.stop;
+    const unsigned stop = *S.stop & 0xffffu;
     return stop != 0u && depth >= (int)stop - 1;
 }
 __device__ inline unsigned ext_count(const Paths& S, int depth) { return finished(S, depth) ? 0u : S.cnt_ext[depth]; }
@@ -1851,13 +1852,19 @@ constexpr unsigned kFinishMin = 8;  // entries a workgroup takes at a time, at l
 // us for 64 x 64 paths in fog, this 655.  Bound by the latency of each phase: a
 // workgroup's chains of dependent loads, at one to four busy waves.
 // More than `limit` entries are left to the separate launches, which use the
-// whole device better; the host tries again a few bounces on.  A workgroup
-// takes at most `most` entries at a time.  deep: trees worth the persistent
-// traversal, which ends in eight lanes a ray.
+// whole device better; the host tries again a few bounces on.  first: the
+// bounce of the pass's first launch that takes any number of entries (its own
+// bounce for the others).  With more than `whole` entries a launch runs `span`
+// bounces, an odd number (the entries left go to the other queue), and the
+// next one takes what is left by even shares again: a workgroup's paths end
+// at different bounces, and its waves go empty.  A workgroup takes at most
+// `most` entries at a time.  deep: trees worth the persistent traversal, which
+// ends in eight lanes a ray.
 // SURFACES: conductors or dielectrics among the materials; MEDIA: volumes.
 template <bool SURFACES, bool SKY, bool MEDIA>
 __global__ __launch_bounds__(kFinishBlock, 2) void k_finish(const ReqInfo* __restrict__ reqs, Paths S, int depth0,
-                                                            int bounces, unsigned limit, unsigned most, int deep)
+                                                            int first, int bounces, int span, unsigned limit,
+                                                            unsigned whole, unsigned most, int deep)
 {
     constexpr int B = kFinishBlock, Q = 4 * B;  // an entry becomes at most four lanes
     constexpr int kStackWords = 2 * kFinishStack * B, kShadeWords = shade_lds_words<kMatLambert, B>();
@@ -1868,10 +1875,16 @@ __global__ __launch_bounds__(kFinishBlock, 2) void k_finish(const ReqInfo* __res
     __shared__ unsigned bin_words[kBinWords];
     __shared__ unsigned cnt[2 + kBins];  // next entries, shadow records, binned entries
     __shared__ unsigned long long fetch[2];
+    __shared__ unsigned left_at;
     const unsigned n0 = S.cnt_ext[depth0], stop = *S.stop, tid = threadIdx.x;
-    // The workgroups of this launch write depth0 + 1; an earlier launch less.
-    if (n0 > limit || (stop != 0u && stop < (unsigned)depth0 + 1u)) return;
-    if (tid == 0) *S.stop = (unsigned)depth0 + 1u;
+    // An earlier launch has taken the pass, or what was left of it; the workgroups
+    // of this launch write first + 1 and depth0 + 1.
+    const unsigned from = stop & 0xffffu, ended = stop >> 16;
+    if (n0 > limit || (from != 0u && from < (unsigned)first + 1u) || (ended != 0u && ended < (unsigned)depth0 + 1u))
+        return;
+    const bool to_end = n0 <= whole;
+    const int end = to_end || bounces - depth0 <= span ? bounces : depth0 + span;
+    if (tid == 0) *S.stop = ((unsigned)first + 1u) | (to_end ? ((unsigned)depth0 + 1u) << 16 : 0u);
     const unsigned* q0 = S.queue[depth0 & 1];
     // A share for every workgroup of the grid when the entries are few.
     const unsigned even = (n0 + gridDim.x - 1) / gridDim.x, some = even > kFinishMin ? even : kFinishMin;
@@ -1882,7 +1895,7 @@ __global__ __launch_bounds__(kFinishBlock, 2) void k_finish(const ReqInfo* __res
         unsigned n = n0 - c < chunk ? n0 - c : chunk;
         int cur = 0;
         for (unsigned i = tid; i < n; i += B) queue[0][i] = q0[c + i];
-        for (int d = depth0; d < bounces && n > 0; ++d) {
+        for (int d = depth0; d < end && n > 0; ++d) {
             if (tid < 2 + kBins) cnt[tid] = 0u;
             if (tid < 2) fetch[tid] = 0ull;
             __syncthreads();
@@ -1925,11 +1938,15 @@ __global__ __launch_bounds__(kFinishBlock, 2) void k_finish(const ReqInfo* __res
             }
             if (tid == 0) {  // the pass's counts, as the separate launches leave them
                 if (n_sh) atomicAdd(S.cnt_sh + d, n_sh);
-                if (n) atomicAdd(S.cnt_ext + d + 1, n);
+                if (n) left_at = atomicAdd(S.cnt_ext + d + 1, n);
             }
             cur ^= 1;
         }
         __syncthreads();
+        if (end < bounces) {  // entries left for the next launch
+            for (unsigned i = tid; i < n; i += B) S.queue[end & 1][left_at + i] = queue[cur][i];
+            __syncthreads();
+        }
     }
 }
 
@@ -2532,10 +2549,11 @@ struct PassShape {
     int depth; // deepest tree
 };
 
-// A pass of at most kFinishPaths paths runs as one launch (k_finish), as do the
-// bounces of a larger one from kFinishDepth on; before that the pass is handed
-// over at every second bounce from the fourth, while four or more are left,
-// once at most kFinishLimit entries are.
+// A pass of at most kFinishPaths paths runs as one launch (k_finish).  A larger
+// one is handed over at every second bounce from the fourth, while four or more
+// are left, once at most kFinishLimit entries are; from kFinishDepth on it is
+// handed over whatever is left, kFinishSpan bounces a launch while that is more
+// than kFinishLimit entries.
 // Paths, one launch / one a phase: 131,044 paths take 357 / 493 us in the plain
 // box, 1491 / 1901 in fog, 1640 / 1951 with conductors and glass, 2598 / 3076
 // with 100,000 triangles and 2262 / 2933 under a sky; 262,144 paths 621 / 606,
@@ -2543,15 +2561,27 @@ struct PassShape {
 // Limit 8k / 32k / 128k / 256k / 512k: conductor and glass 333 x 250 x 9 4250 /
 // 3864 / 3468 / 3468 / 4529 us, 48 served previews 20.4 / 19.8 / 19.3 / 20.8 /
 // 25.3 ms, 1080p terrain 19.5 / 19.0 / 18.3 / 19.0 / 19.0 ms (4716 us, 23.3 ms
-// and 20.1 ms without k_finish).
-constexpr int kFinishPaths = 131072, kFinishDepth = 14, kFinishLimit = 131072;
+// and 20.1 ms without k_finish).  Every bounce / second / fourth: 18.8 / 18.9 /
+// 19.4 ms served, conductor and glass 3429 / 3420 / 3779 us; from the second,
+// fourth or sixth the same within 1%.
+// Depth 8 / 14 / 20 / no end to the separate launches: 48 served previews 20.2 /
+// 18.9 / 19.2 / 20.4 ms (66 bounces of empty launches take 1.4 ms), 1080p terrain
+// 17.8 / 17.9 / 18.0 / 18.2, scattering medium, 4.2M paths that live up to 67
+// bounces, 70.3 / 64.4 / 63.6 / 67.3, 100,000 triangles, 2.1M paths without
+// roulette, 51.0 / 46.7 / 42.7 / 41.3.  Span 3 / 5 / 7 / 15 / to the end: the
+// medium 63.9 / 64.6 / 65.3 / 71.1 / 92.1 ms, the triangles 45.5 / 46.7 / 46.9 /
+// 48.2 / 49.9, a furnace of 4.2M paths 23.9 / 23.8 / 23.9 / 24.9 / 30.9 (72.6,
+// 48.0 and 31.1 before k_finish).
+constexpr int kFinishPaths = 131072, kFinishDepth = 14, kFinishLimit = 131072, kFinishSpan = 5;
+static_assert(kFinishPaths <= kFinishLimit, "a whole pass runs to its end in its one launch");
+static_assert(kFinishSpan % 2 == 1, "a span's entries come from one queue and go to the other");
 // Levels from which k_finish traverses with persistent waves.  From 2 / 4 / never:
 // fog 64 x 64 670 / 654 / 657 us, conductor and glass 333 x 250 x 9 3420 / 3410 /
 // 3475 us, 48 served previews 19.0 / 19.0 / 19.1 ms, 1080p terrain 17.9 / 18.0 /
 // 18.3 ms.
 constexpr int kFinishDeep = 4;
 
-using FinishKernel = void (*)(const ReqInfo*, Paths, int, int, unsigned, unsigned, int);
+using FinishKernel = void (*)(const ReqInfo*, Paths, int, int, int, int, unsigned, unsigned, unsigned, int);
 
 FinishKernel pick_finish(const PassShape& sh)
 {
@@ -2573,7 +2603,7 @@ void launch_pass(const ReqInfo* d_info, Paths S, const PassEntry* ent, int n_ent
     hipLaunchKernelGGL(k_generate, dim3(grid_for(paths, 256, 4096)), dim3(256), 0, stream, d_info, ent, n_ent, paths,
                        S);
     const bool can_finish = sh.depth - 1 <= kFinishStack;  // else a tree is too deep for its stack
-    auto finish = [&](int d, unsigned limit, int64_t entries) {
+    auto finish = [&](int d, int first, unsigned limit, int64_t entries) {
         const FinishKernel fn = pick_finish(sh);
         // Resident workgroups, each with room for its records: most * grid <= cap
         // entries, or all entries in one round (then the last workgroup's share
@@ -2583,14 +2613,15 @@ void launch_pass(const ReqInfo* d_info, Paths S, const PassEntry* ent, int n_ent
         const int64_t share = d == 0 ? (entries + grid - 1) / grid : sh.cap / grid;
         unsigned most = (unsigned)std::max<int64_t>(1, std::min<int64_t>(share, kFinishBlock));
         const unsigned blocks = (unsigned)std::min<int64_t>(grid, std::max<int64_t>(1, d == 0 ? grid : sh.cap / most));
-        int bounces = sh.bounces, deep = sh.depth >= kFinishDeep;
-        void* args[] = {(void*)&d_info, &S, &d, &bounces, &limit, &most, &deep};
+        int bounces = sh.bounces, span = kFinishSpan, deep = sh.depth >= kFinishDeep;
+        unsigned all = kFinishLimit;
+        void* args[] = {(void*)&d_info, &S, &d, &first, &bounces, &span, &limit, &all, &most, &deep};
         (void)hipLaunchKernel((const void*)fn, dim3(blocks), dim3(kFinishBlock), args, 0, stream);
     };
     const bool whole = can_finish && paths <= kFinishPaths;
     const int last = whole ? 0 : can_finish ? std::min(sh.bounces, kFinishDepth) : sh.bounces;
     for (int d = 0; d < last; ++d) {
-        if (can_finish && d >= 4 && d % 2 == 0 && sh.bounces - d >= 4) finish(d, kFinishLimit, kFinishLimit);
+        if (can_finish && d >= 4 && d % 2 == 0 && sh.bounces - d >= 4) finish(d, d, kFinishLimit, kFinishLimit);
         void* args[] = {(void*)&d_info, &S, &d};
         (void)hipLaunchKernel((const void*)sh.ext_fn, dim3(sh.ge), dim3(sh.block), args, 0, stream);
 #define RISE_LAUNCH_SHADE(K, KIND)                                                                     \
@@ -2611,7 +2642,9 @@ void launch_pass(const ReqInfo* d_info, Paths S, const PassEntry* ent, int n_ent
         if (sh.mat_mask & (1u << kMatVolume))
             hipLaunchKernelGGL(k_walk, dim3(grid_for(4 * sh.cap, 256, 2048)), dim3(256), 0, stream, d_info, S, d);
     }
-    if (last < sh.bounces) finish(last, 0xffffffffu, whole ? paths : 4 * (int64_t)paths);
+    if (whole) finish(0, 0, 0xffffffffu, paths);
+    else
+        for (int d = last; d < sh.bounces; d += kFinishSpan) finish(d, last, 0xffffffffu, 4 * (int64_t)paths);
     hipLaunchKernelGGL(k_film, dim3(grid_for(film, 256, 4096)), dim3(256), 0, stream, d_info, ent, n_ent, film, S);
 }
 

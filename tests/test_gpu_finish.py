@@ -90,3 +90,38 @@ def test_gpu_finish_deep_tree(cuda):
     b.release()
     deep.release()
     flat.release()
+
+
+LONG = {  # most paths live past the bounce from which k_finish takes any number of entries
+    "furnace": lambda: (pt_scene.furnace_box(0.98), dict(width=700, height=700, spp=1, rr_min_depth=64)),
+    "medium": lambda: (pt_scene.furnace_medium(sigma_s=(8.0, 8.0, 8.0)), dict(width=512, height=512, spp=2)),
+    "cloud": lambda: (pt_scene.cloud_cornell(3, 20000), dict(width=900, height=800, spp=1, rr_min_depth=40,
+                                                              max_diffuse_bounce=30)),
+}
+
+
+@pytest.mark.parametrize("name", sorted(LONG))
+def test_gpu_finish_many_long_paths(cuda, name):
+    """Passes with more entries left at that bounce than one launch takes to the end, against the separate launches
+    (a batch with a tree too deep for k_finish takes none of it)."""
+    (scene, r), k = LONG[name]()
+    q = dataclasses.replace(r, seed=11, **k)
+    rast = PathTracingSpectralRasterizer(scene)
+    log_case(f"{name} alone")
+    film, sq, st = rast.rasterize_scene(q, want_sq=True)
+    deep_s, deep_r = deep_scene()
+    deep = PathTracingSpectralRasterizer(deep_s)
+    dq = dataclasses.replace(deep_r, width=8, height=8, spp=1, seed=5)
+    log_case(f"{name} with a deep tree")
+    dst = deep.rasterize_scene(dq)[2]
+    b = RenderBatch([(rast, q), (deep, dq)], want_sq=True)
+    b.launch()
+    torch.cuda.synchronize()
+    assert np.array_equal(b.films[0].cpu().numpy(), film.cpu().numpy())
+    assert np.array_equal(b.films_sq[0].cpu().numpy(), sq.cpu().numpy())
+    total = b.stats()
+    for key in ("extension_rays", "shadow_rays", "paths"):
+        assert total[key] == st[key] + dst[key], key
+    b.release()
+    rast.release()
+    deep.release()
