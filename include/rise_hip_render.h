@@ -242,9 +242,13 @@ rise_hip_status rise_hip_batch_create(const rise_hip_render_request* requests, s
                                       rise_hip_batch** out_batch);
 
 /* Launch-shape choices of a batch (0 everywhere: defaults).  They change
- * speed only: films are the same under every tuning. */
+ * speed only: films are the same under every tuning.  With trace_block, stack
+ * and persistent all 0, passes of at most 131072 paths and the last bounces of
+ * larger ones run in single launches of a shape of their own; with one of
+ * them chosen, every bounce of every pass has traversal launches of that shape,
+ * which is slower for small passes. */
 typedef struct rise_hip_batch_tuning {
-    int32_t max_paths;    /* paths in flight per pass (0: 4194304); at least one chunk (<= 1048576 paths) */
+    int32_t max_paths;    /* paths in flight per pass (0: 33554432); at least one chunk (<= 1048576 paths) */
     int32_t trace_block;  /* workgroup size of the traversal kernels: 64, 128 or 256 (0: 128) */
     int32_t stack;        /* traversal stack: 0 auto (LDS, sized by tree depth), 8 or 16 LDS entries per
                              lane when the trees fit, -1 private memory */
@@ -257,7 +261,8 @@ typedef struct rise_hip_batch_tuning {
 rise_hip_status rise_hip_batch_create_tuned(const rise_hip_render_request* requests, size_t n_requests,
                                             const rise_hip_batch_tuning* tuning, rise_hip_batch** out_batch);
 
-/* The tuning a batch resolved to (auto choices made concrete). */
+/* The tuning a batch resolved to (auto choices made concrete: the shapes of
+ * its bounces' own launches; passed to another batch they are chosen ones). */
 rise_hip_status rise_hip_batch_get_tuning(const rise_hip_batch* batch, rise_hip_batch_tuning* out_tuning);
 
 /* Enqueues the whole batch on `stream`: kernel launches only (no copies, no

@@ -2171,6 +2171,10 @@ unsigned grid_for(int64_t n, int block, unsigned max_blocks)
     return (unsigned)std::max<int64_t>(1, std::min<int64_t>(g, max_blocks));
 }
 
+// A traversal shape is chosen: every bounce has launches of that shape, and
+// k_finish, which has its own, runs none.
+bool shape_chosen(const rise_hip_batch_tuning& tn) { return tn.trace_block || tn.stack || tn.persistent; }
+
 // Traversal launch shape: the node-group stack holds at most one entry per
 // level below the root, and the smallest LDS stack that fits keeps occupancy
 // highest; persistent waves pay off on deep trees, one ray per thread on
@@ -2363,6 +2367,7 @@ struct rise_hip_batch {
     unsigned mat_mask = 0;                // material kinds present in the batch's scenes
     bool sky = false;                     // some scene has a sky or directional lights
     int depth = 1;                        // deepest tree
+    bool finish = true;                   // k_finish may run passes
     int64_t cap = 0;                   // path pool size
     std::vector<rise_hip_render_request> requests;
     std::vector<PassEntry> entries;    // all passes, concatenated
@@ -2531,6 +2536,7 @@ rise_hip_status plan(rise_hip_batch* b, const rise_hip_render_request* reqs, siz
     b->mat_mask = mat_mask;
     b->sky = has_sky;
     b->depth = depth;
+    b->finish = !shape_chosen(tn);
     b->n_req = (int)n;
     b->requests.assign(reqs, reqs + n);
     b->launched = false;
@@ -2547,6 +2553,7 @@ struct PassShape {
     unsigned mat_mask;
     bool sky;  // some scene has a sky or directional lights
     int depth; // deepest tree
+    bool finish;  // k_finish may run it
 };
 
 // A pass of at most kFinishPaths paths runs as one launch (k_finish).  A larger
@@ -2602,7 +2609,7 @@ void launch_pass(const ReqInfo* d_info, Paths S, const PassEntry* ent, int n_ent
                        4 * (kMaxPathDepth + 1));
     hipLaunchKernelGGL(k_generate, dim3(grid_for(paths, 256, 4096)), dim3(256), 0, stream, d_info, ent, n_ent, paths,
                        S);
-    const bool can_finish = sh.depth - 1 <= kFinishStack;  // else a tree is too deep for its stack
+    const bool can_finish = sh.finish && sh.depth - 1 <= kFinishStack;  // else a tree is too deep for its stack
     auto finish = [&](int d, int first, unsigned limit, int64_t entries) {
         const FinishKernel fn = pick_finish(sh);
         // Resident workgroups, each with room for its records: most * grid <= cap
@@ -2664,7 +2671,7 @@ hipError_t launch(rise_hip_batch* b, hipStream_t stream)
     hipLaunchKernelGGL(k_fill, dim3(grid_for((int64_t)b->film_floats, 256, 4096)), dim3(256), 0, stream, b->d_film,
                        b->film_floats);
     const PassShape sh{b->ext_fn, b->con_fn, b->grid_ext, b->grid_con, (unsigned)b->trace_block,
-                       b->cap,    b->bounces, b->mat_mask, b->sky,   b->depth};
+                       b->cap,    b->bounces, b->mat_mask, b->sky,   b->depth,   b->finish};
     const int passes = (int)b->pass_paths.size();
     for (int p = 0; p < passes; ++p) {
         const Paths S = pass_counters(b->S, b->counters + (size_t)p * kCounters);
@@ -3086,6 +3093,7 @@ rise_hip_status server_launch(rise_hip_server* sv)
         sh.mat_mask = kinds;
         sh.sky = sky;
         sh.depth = depth;
+        sh.finish = !shape_chosen(sv->tuning);
         PassEntry* d_ent = sv->d_ent + (size_t)k * kPassEntries;
         hipError_t e = hipMemcpyAsync(d_ent, ent, (size_t)n_ent * sizeof(PassEntry), hipMemcpyHostToDevice, sv->stream);
         if (e != hipSuccess) return fail_hip(e, "pass table");
