@@ -224,10 +224,15 @@ hipError_t launch_closest_objects(const ObjectSceneView& sc, int arith, int stac
 {
     if (n <= 0) return hipSuccess;
     reset_fetch<<<1, 1, 0, stream>>>(next);
-#define RISE_OBJ_CLOSEST_K(A, R, S)                                                                          \
-    closest_objects<A, R, S><<<resident_grid(closest_objects<A, R, S>, n), kObjBlock, 0, stream>>>(sc, rays, n, \
-                                                                                                  faces, prim_id, \
-                                                                                                  t, hits, next)
+    // The large form's grid serves all its instantiations (each three waves per
+    // SIMD), so that only launches of many rays ask for a second one.
+    unsigned grid = stack_need <= kObjLds ? resident_grid(closest_objects<kArithIeee, true, kObjLds>, n) : 0u;
+    const bool many = stack_need <= kObjLdsSmall && n > (int64_t)kObjBlock * grid;
+#define RISE_OBJ_CLOSEST_K(A, R, S)                                                                         \
+    do {                                                                                                    \
+        if (S != kObjLds) grid = resident_grid(closest_objects<A, R, S>, n);                                \
+        closest_objects<A, R, S><<<grid, kObjBlock, 0, stream>>>(sc, rays, n, faces, prim_id, t, hits, next); \
+    } while (0)
 #define RISE_OBJ_CLOSEST(A, S)                                                                   \
     do {                                                                                         \
         if (hits) {                                                                              \
@@ -237,13 +242,12 @@ hipError_t launch_closest_objects(const ObjectSceneView& sc, int arith, int stac
             RISE_OBJ_CLOSEST_K(A, false, S);                                                     \
         }                                                                                        \
     } while (0)
-    const bool many = n > (int64_t)kObjBlock * resident_grid(closest_objects<kArithIeee, true, kObjLds>, n);
     if (arith == kArithX86Fma) {
-        if (stack_need <= kObjLdsSmall && many) RISE_OBJ_CLOSEST(kArithX86Fma, kObjLdsSmall);
+        if (many) RISE_OBJ_CLOSEST(kArithX86Fma, kObjLdsSmall);
         else if (stack_need <= kObjLds) RISE_OBJ_CLOSEST(kArithX86Fma, kObjLds);
         else RISE_OBJ_CLOSEST(kArithX86Fma, 0);
     } else {
-        if (stack_need <= kObjLdsSmall && many) RISE_OBJ_CLOSEST(kArithIeee, kObjLdsSmall);
+        if (many) RISE_OBJ_CLOSEST(kArithIeee, kObjLdsSmall);
         else if (stack_need <= kObjLds) RISE_OBJ_CLOSEST(kArithIeee, kObjLds);
         else RISE_OBJ_CLOSEST(kArithIeee, 0);
     }
