@@ -64,3 +64,37 @@ def test_gpu_few_rays(cuda, scene, n):
     assert np.array_equal(gt.cpu().numpy(), t[N - n:])
     go = om.intersect_shadow_ray(r, torch.from_numpy(far[N - n:].copy()).to(cuda))
     assert np.array_equal(go.cpu().numpy(), occ[N - n:])
+
+
+@pytest.mark.parametrize("faces", [raycast.FACES_FRONT, raycast.FACES_BACK, raycast.FACES_BOTH])
+@pytest.mark.parametrize("arith", [raycast.ARITH_IEEE, raycast.ARITH_X86_FMA])
+@pytest.mark.parametrize("vertices", [np.float32, np.float64])
+def test_gpu_few_rays_forms(cuda, vertices, arith, faces):
+    """The same ends under a face selection, with records, double vertices (off the float grid) and both arithmetic
+    models, against the per-ray code of a scene with one identity object on host threads."""
+    tris, rays = _grid_of_copies().astype(vertices), _rays()
+    if vertices is np.float64:
+        tris *= 1.0 + np.random.default_rng(25).uniform(-1e-9, 1e-9, tris.shape)
+    far = np.random.default_rng(24).uniform(0.01, 1.0, N).astype(np.float32)
+    objs = raycast.make_objects([(0, *raycast.object_matrices())])
+    want = raycast.host_trace_objects([tris], objs, rays, faces=faces, arith=arith)
+    occ = raycast.host_trace_objects([tris], objs, rays, mode=1, faces=faces, tmax=far, arith=arith)
+    hit = want["prim_id"] >= 0
+    assert 0.1 < hit.mean() < 1.0
+    om = raycast.ObjectManager(arith)
+    om.add_mesh(tris)
+    om.prepare_for_rendering()
+    for n in (1, 7, 8, 9, 15, 16, 17, 33, 1000, 40_959, 40_961, N):
+        log_case(f"{vertices.__name__} {arith} faces {faces} n={n}")
+        r = torch.from_numpy(np.ascontiguousarray(rays[:, N - n:])).to(cuda)
+        g, h = raycast.hit_fields(om.intersect_ray_ex(r, faces)), hit[N - n:]
+        assert np.array_equal(g["prim_id"], want["prim_id"][N - n:])
+        for field in ("range", "alpha", "beta", "point", "geom_normal"):
+            assert np.array_equal(g[field][h], want[field][N - n:][h]), field
+        go = om.intersect_shadow_ray_ex(r, faces, torch.from_numpy(far[N - n:].copy()).to(cuda))
+        assert np.array_equal(go.cpu().numpy(), occ[N - n:])
+        if faces == raycast.FACES_BOTH:
+            gp, gt = om.intersect_ray(r)
+            assert np.array_equal(gp.cpu().numpy(), want["prim_id"][N - n:])
+            assert np.array_equal(gt.cpu().numpy()[h], want["range"][N - n:][h].astype(np.float32))
+    om.release()
