@@ -22,8 +22,10 @@ constexpr int kObjBlock = 128;
 // certifies them.  A ray's walk over several trees is long, and 500,000 rays
 // are two or three a lane, so lanes are not left idle: 500,000 rays into 16
 // objects took 2041 us at 20 idle lanes, 2004 at 14, 1980 at 8; 1926 / 1899 /
-// 1867 / 1862 at 1 / 2 / 4 / 8 waiting candidates.
-constexpr int kRefill = 8, kCertify = 8;
+// 1867 / 1862 at 1 / 2 / 4 / 8 waiting candidates.  Few rays are bound by the
+// longest ray's chain and take the large stack's form: 2000 rays 1174 us at 8,
+// 1157 at 2 (obj_certify).
+constexpr int kRefill = 8;
 constexpr int kRefillAny = 20;  // any-hit queries
 
 __device__ inline void load_ray6(const float* __restrict__ rays, int64_t n, int64_t i, float ray[6])
@@ -41,6 +43,7 @@ __device__ inline void load_ray6(const float* __restrict__ rays, int64_t n, int6
 // 30,000 with three.  Any-hit queries lose by it (200,000 rays 430 -> 484 us) and
 // keep three.
 constexpr int kObjLdsSmall = 16, kObjLds = 24;
+constexpr int obj_certify(int stack) { return stack == kObjLdsSmall ? 8 : 2; }
 constexpr int obj_waves(int stack) { return stack == kObjLdsSmall ? 4 : 1; }
 
 template <int STACK>
@@ -143,7 +146,7 @@ __global__ __launch_bounds__(kObjBlock, obj_waves(STACK)) void closest_objects(O
         if (vote.object && Q.phase == kObjPhaseObject) objects_closest_object<true>(faces, st, Q);
         const bool waits = (Q.phase == kObjPhaseWorld || Q.phase == kObjPhaseObject) && Q.s.pend != kNoLeaf;
         const int waiting = __popcll(__ballot(waits));
-        if (waiting >= kCertify || waiting * 8 >= vote.n) {
+        if (waiting >= obj_certify(STACK) || waiting * 8 >= vote.n) {
             if (waits) objects_closest_commit(sc, Q);
         }
         if (vote.next && Q.phase != kObjPhaseWorld && Q.phase != kObjPhaseObject && Q.phase != kObjPhaseDone)
