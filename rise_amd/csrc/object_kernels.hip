@@ -71,11 +71,11 @@ __device__ inline typename StackOf<STACK>::type make_stack(uint2* lds)
 // Which phases a wave runs in this round: those of at least a kVote-th of its
 // busy lanes, so that no phase's code runs for few of them; the others' lanes
 // wait until they are more, or the rest is done.  One of the three always has a
-// third of the lanes.  (Any-hit queries step every phase in each round: with
-// votes 2,000,000 limited shadow rays take 3279 us instead of 2472.)  500,000 rays into 16 objects: 2178 us with every phase
-// of every lane in each round and candidates certified one by one; 2225 / 2076 /
+// third of the lanes.  500,000 rays into 16 objects: 2178 us with every phase of
+// every lane in each round and candidates certified one by one; 2225 / 2076 /
 // 2039 / 2032 at a third / quarter / eighth / sixteenth, the last two with the
-// refill line at 20 and 14.
+// refill line at 20 and 14.  (Any-hit queries step every phase in each round:
+// with votes 2,000,000 limited shadow rays take 3279 us instead of 2472.)
 constexpr int kVote = 8;
 struct PhaseVote {
     int n;  // busy lanes
@@ -100,14 +100,13 @@ static_assert(sizeof(ObjectHit) <= sizeof(rise_hip_hit) && alignof(ObjectHit) <=
 
 // Persistent: the grid is sized to the resident waves, each lane's first ray
 // is assigned statically and later ones are fetched wave-wide (ItemFetch) as
-// lanes finish; a query that has ended is written out when its wave fetches.  REC: stage the ObjectHit in hits[ray] for object_records;
-// else write prim_id and t (float world range).
+// lanes finish; a query that has ended is written out when its wave fetches.
+// REC: stage the ObjectHit in hits[ray] for object_records; else write prim_id
+// and t (float world range).
 template <int A, bool REC, int STACK>
-__global__ __launch_bounds__(kObjBlock, obj_waves(STACK)) void closest_objects(ObjectSceneView sc, const float* __restrict__ rays,
-                                                             int64_t n, unsigned faces, int32_t* __restrict__ prim_id,
-                                                             float* __restrict__ t_out,
-                                                             rise_hip_hit* __restrict__ hits,
-                                                             unsigned long long* next)
+__global__ __launch_bounds__(kObjBlock, obj_waves(STACK)) void closest_objects(
+    ObjectSceneView sc, const float* __restrict__ rays, int64_t n, unsigned faces, int32_t* __restrict__ prim_id,
+    float* __restrict__ t_out, rise_hip_hit* __restrict__ hits, unsigned long long* next)
 {
     __shared__ uint2 lds[STACK > 0 ? STACK * kObjBlock : 1];
     auto st = make_stack<STACK>(lds);

@@ -95,7 +95,8 @@ RISE_HD inline void encode_pixel(const out::Params& p, int mode, const float* px
     if (mode == kRgba8) {
         uint8_t o[4];
         encode_ldr<uint8_t, QUICK>(p, c, o);
-        if (QUICK && (uintptr_t)out % 4 == 0) ((uint32_t*)out)[i] = o[0] | o[1] << 8 | o[2] << 16 | (uint32_t)o[3] << 24;
+        if (QUICK && (uintptr_t)out % 4 == 0)
+            ((uint32_t*)out)[i] = o[0] | o[1] << 8 | o[2] << 16 | (uint32_t)o[3] << 24;
         else
             for (int k = 0; k < 4; ++k) ((uint8_t*)out)[4 * i + k] = o[k];
         return;

@@ -463,7 +463,8 @@ constexpr int kExtendWaves = 5;
 // finish early are refilled; otherwise one thread traces one ray to the end
 // (grid-stride), which costs less per ray when trees are shallow.
 template <int STACK, int BLOCK, bool PERSIST>
-__global__ __launch_bounds__(BLOCK, PERSIST ? kExtendWaves : 1) void k_extend(const ReqInfo* __restrict__ reqs, Paths S, int depth)
+__global__ __launch_bounds__(BLOCK, PERSIST ? kExtendWaves : 1) void k_extend(const ReqInfo* __restrict__ reqs,
+                                                                              Paths S, int depth)
 {
     __shared__ uint2 lds[STACK > 0 ? STACK * BLOCK : 1];
     const unsigned n = ext_count(S, depth);
@@ -538,7 +539,8 @@ __device__ inline GgxParams ggx_params(const PtSceneView& sc, const DevMaterial&
 __device__ inline float ggx_favg(const PtSceneView& sc, const DevMaterial& m, float nm, const GgxParams& g)
 {
     if (m.favg >= 0 && g.amb == 1.0f) {
-        int row = 0, col = 0;  // an absent spectrum has the one default value; outside its range a spectrum is 0, the last entry
+        // An absent spectrum has the one default value; outside its range a spectrum is 0, the last entry.
+        int row = 0, col = 0;
         if (m.ior_spd >= 0) {
             const DevSpd d = sc.spds[m.ior_spd];
             row = (nm < d.begin || nm > d.end) ? d.n : spd_bin(d, nm);
@@ -999,8 +1001,8 @@ __device__ inline void write_lane(const Paths& S, f3 no, unsigned lw, f3 dir, fl
 }
 
 // The same for lane w of a path, appended to the next extension queue at `at`.
-__device__ inline void write_continuation(const Paths& S, f3 no, unsigned slot, unsigned w, unsigned* at, f3 dir, float pdf,
-                                          float imp, unsigned bounces, const IorStack& st, unsigned vbn)
+__device__ inline void write_continuation(const Paths& S, f3 no, unsigned slot, unsigned w, unsigned* at, f3 dir,
+                                          float pdf, float imp, unsigned bounces, const IorStack& st, unsigned vbn)
 {
     *at = slot * 4u + w;
     write_lane(S, no, w * (unsigned)S.cap + slot, dir, pdf, imp, bounces, st, vbn);
@@ -1155,20 +1157,21 @@ __device__ inline void shade_entries(const ReqInfo* __restrict__ reqs, const Pat
         const int trips = __ballot(surface && !nm) != 0ull ? kHwss : 1;
         if constexpr (MAT != kMatDielectric) {
             // The record's stage slot of trip k: direction, distance, value.
+            auto slot_of = [&](int k, int word) -> float& { return stage[(k * 5 + word) * BLOCK + threadIdx.x]; };
             auto put = [&](int k, f3 to, float dist, float val) {
-                stage[(k * 5 + 0) * BLOCK + threadIdx.x] = to.x;
-                stage[(k * 5 + 1) * BLOCK + threadIdx.x] = to.y;
-                stage[(k * 5 + 2) * BLOCK + threadIdx.x] = to.z;
-                stage[(k * 5 + 3) * BLOCK + threadIdx.x] = dist;
-                stage[(k * 5 + 4) * BLOCK + threadIdx.x] = val;
+                slot_of(k, 0) = to.x;
+                slot_of(k, 1) = to.y;
+                slot_of(k, 2) = to.z;
+                slot_of(k, 3) = dist;
+                slot_of(k, 4) = val;
             };
             auto flush = [&](unsigned mask, unsigned kind) {
                 push4.reserve(v.n_sh, mask);
                 for (int k = 0; k < kHwss; ++k) {
                     if (!((mask >> k) & 1u)) continue;
-                    const f3 to = mk3(stage[(k * 5 + 0) * BLOCK + threadIdx.x], stage[(k * 5 + 1) * BLOCK + threadIdx.x], stage[(k * 5 + 2) * BLOCK + threadIdx.x]);
+                    const f3 to = mk3(slot_of(k, 0), slot_of(k, 1), slot_of(k, 2));
                     const f3 so = offset_ray(h.p, dot3(to, h.ng) > 0.0f ? h.ng : -h.ng);
-                    write_shadow(S, v.sh0 + push4.pos(k), so, to, stage[(k * 5 + 3) * BLOCK + threadIdx.x], stage[(k * 5 + 4) * BLOCK + threadIdx.x],
+                    write_shadow(S, v.sh0 + push4.pos(k), so, to, slot_of(k, 3), slot_of(k, 4),
                                  (slot * 4u + (nm ? lane : (unsigned)k)) | kind, (unsigned)(mobj + 1));
                 }
             };
@@ -1273,7 +1276,8 @@ __device__ inline void shade_entries(const ReqInfo* __restrict__ reqs, const Pat
                     if (cosd > 0.0f) {
                         const BsdfDir<MAT> bd = bsdf_dir<false>(h, bv, dd);
                         if (nm) {
-                            vd = S.thr0[li] * (S.thr[li] * (L.le * bsdf_value(sc, mat, bv, bd, lam_of(lane), amb) * cosd));
+                            vd = S.thr0[li] *
+                                 (S.thr[li] * (L.le * bsdf_value(sc, mat, bv, bd, lam_of(lane), amb) * cosd));
                             has_d = vd > 0.0f;
                         } else {
 #pragma unroll 1
@@ -1389,7 +1393,8 @@ __device__ inline void shade_entries(const ReqInfo* __restrict__ reqs, const Pat
                 }
             }
             const unsigned qi = push(v.n_out, cont);
-            if (cont) write_continuation(S, surface_origin(h, cdir), slot, cw, v.out + qi, cdir, cpdf, cimp, cst, ist, vbn);
+            if (cont)
+                write_continuation(S, surface_origin(h, cdir), slot, cw, v.out + qi, cdir, cpdf, cimp, cst, ist, vbn);
         } else {
             // A dielectric: for a lane already on its own, and for each wavelength of
             // a shared ray that branches here (:2634-2760; no NEE or RR at this vertex).
@@ -1632,7 +1637,8 @@ __device__ inline void volume_entries(const ReqInfo* __restrict__ reqs, const Pa
             }
             const unsigned sd = push(v.n_sh, has_d);
             if (has_d)
-                write_shadow(S, v.sh0 + sd, p, dd, INFINITY, vd, (slot * 4u + lane) | ((kRecDir + (unsigned)l) << kRecKindShift),
+                write_shadow(S, v.sh0 + sd, p, dd, INFINITY, vd,
+                             (slot * 4u + lane) | ((kRecDir + (unsigned)l) << kRecKindShift),
                              kShadowNoWalk | (unsigned)(mobj + 1));
         }
 
@@ -2644,7 +2650,8 @@ void launch_pass(const ReqInfo* d_info, Paths S, const PassEntry* ent, int n_ent
             hipLaunchKernelGGL((k_shade<kMatDielectric, false>), dim3(gs), dim3(kShadeBlock), 0, stream, d_info, S, d);
 #undef RISE_LAUNCH_SHADE
         if (sh.mat_mask & (1u << kMatVolume))
-            hipLaunchKernelGGL(sh.sky ? k_volume<true> : k_volume<false>, dim3(gs), dim3(kShadeBlock), 0, stream, d_info, S, d);
+            hipLaunchKernelGGL(sh.sky ? k_volume<true> : k_volume<false>, dim3(gs), dim3(kShadeBlock), 0, stream,
+                               d_info, S, d);
         (void)hipLaunchKernel((const void*)sh.con_fn, dim3(sh.gc), dim3(sh.block), args, 0, stream);
         if (sh.mat_mask & (1u << kMatVolume))
             hipLaunchKernelGGL(k_walk, dim3(grid_for(4 * sh.cap, 256, 2048)), dim3(256), 0, stream, d_info, S, d);

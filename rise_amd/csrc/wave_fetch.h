@@ -131,7 +131,8 @@ struct ItemFetch {
             i = cur + rank;
             cur += want;
             if (want > left) {
-                const float share = (float)(total - end) * 16.0f / (float)src.first;  // a quarter of this wave's even share
+                // A quarter of this wave's even share.
+                const float share = (float)(total - end) * 16.0f / (float)src.first;
                 const unsigned size = (unsigned)fminf(fmaxf(share, 32.0f), (float)RISE_CHUNK);
                 const unsigned need = want - left, take = size > need ? size : need;
                 unsigned long long base = 0;
@@ -197,7 +198,8 @@ __device__ inline void coop_visit(bool on, const R& r, const NodeSlot* __restric
         g.hits &= g.hits - 1u;
         const unsigned at = k ^ r.oinv;
         const unsigned ni = g.base + __builtin_popcount(g.imask & ((1u << at) - 1u));
-        if (g.hits) st.push(make_uint2(g.base, g.hits | (g.imask << 8)));  // every lane of the group writes the same entry
+        // Every lane of the group writes the same entry.
+        if (g.hits) st.push(make_uint2(g.base, g.hits | (g.imask << 8)));
         const unsigned char* node = reinterpret_cast<const unsigned char*>(nodes + ni);
         const unsigned slot = (__lane_id() & (kCoopLanes - 1)) ^ r.oinv;
         const uint4 w0 = *reinterpret_cast<const uint4*>(node);
@@ -254,7 +256,8 @@ __device__ inline void coop_closest(unsigned long long bm, long long item, R& r,
         unsigned passed = 0;
         float t;
         for (unsigned k = 0; k < count; ++k)
-            if (passes_filter<CULL, F64, false>(r, tris, tri64, leaf + k, s.faces, (float)s.best_t, t)) passed |= 1u << k;
+            if (passes_filter<CULL, F64, false>(r, tris, tri64, leaf + k, s.faces, (float)s.best_t, t))
+                passed |= 1u << k;
         const unsigned lane0 = __lane_id() & ~(unsigned)(kCoopLanes - 1);
         bool first = true;
         for (;;) {
@@ -341,8 +344,7 @@ struct CoopStack<LdsStack<STACK>> {
 // instructions (2.15e9 a launch before, 1.9e9 now at 48 of 64 lanes busy).  On
 // the 1M-triangle, 6.07M-ray cast 3405 -> 2880 us against one claim per refill,
 // certifying and finishing at once, and a node test that branched per child.
-// Counted queries (COUNT) certify at once, so that their counts are those of
-// the traversal alone, whatever else its wave holds.
+// Counted queries (COUNT) certify at once; their counts and hits are the same.
 // begin(item, r, s) starts a query, or returns false to skip the item;
 // finish(item, r, s) takes its result.
 template <bool COUNT, bool CULL, bool F64, class R, class Stack, class Begin, class Finish>
