@@ -260,13 +260,14 @@ __device__ inline void coop_closest(unsigned long long bm, long long item, R& r,
                 passed |= 1u << k;
         const unsigned lane0 = __lane_id() & ~(unsigned)(kCoopLanes - 1);
         bool first = true;
-        for (;;) {
-            const unsigned long long pm = __ballot(passed != 0u);
-            if (pm == 0ull) break;
+        unsigned long long pm = __ballot(passed != 0u);
+        while (pm != 0ull) {
             const unsigned gm = (unsigned)(pm >> lane0) & 0xffu;
             const unsigned at = gm ? lane0 + (__builtin_ctz(xor_permute8(gm, r.oinv)) ^ r.oinv) : __lane_id();
-            const unsigned next = (unsigned)__shfl((int)(leaf + (passed ? __builtin_ctz(passed) : 0u)), (int)at);
+            // A leaf holds at most seven, so bit 7 stands for none.
+            const unsigned next = (unsigned)__shfl((int)(leaf + __builtin_ctz(passed | 0x80u)), (int)at);
             if (at == __lane_id()) passed &= passed - 1u;
+            pm = __ballot(passed != 0u);
             if (gm) {
                 if (first || passes_filter<CULL, F64, false>(r, tris, tri64, next, s.faces, (float)s.best_t, t)) {
                     s.pend = next;
