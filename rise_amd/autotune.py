@@ -55,7 +55,9 @@ def time_batch(items, tuning: dict, repeats: int = 2) -> float:
 def tune(items, proxy_spp: int | None = 1, space=None, repeats: int = 2, budget_s: float = 60.0):
     """Returns (best tuning, [(tuning, ms), ...]) for a list of
     (rasterizer, RenderSettings) items.  proxy_spp: sample count of the proxy
-    (None: the items as given)."""
+    (None: the items as given).  Automatic shapes within a hundredth of the
+    fastest are taken before a chosen one: the proxy's passes may be larger or
+    smaller than the real ones."""
     import dataclasses
 
     proxy = []
@@ -71,5 +73,10 @@ def tune(items, proxy_spp: int | None = 1, space=None, repeats: int = 2, budget_
         results.append((tn, ms))
         if time.perf_counter() - t0 > budget_s:
             break
-    best = min(results, key=lambda r: r[1])[0]
+    best, ms = min(results, key=lambda r: r[1])
+    automatic = [r for r in results if not any(r[0].get(k) for k in ("persistent", "trace_block", "stack"))]
+    if automatic:
+        tn, t = min(automatic, key=lambda r: r[1])
+        if t <= 1.01 * ms:
+            best = tn
     return best, results

@@ -40,8 +40,9 @@ __device__ inline void load_ray6(const float* __restrict__ rays, int64_t n, int6
 // where those are enough: LDS and, with some spills, registers for four waves.
 // Records of 30,000 / 200,000 / 500,000 / 1,000,000 rays: 484 / 1382 / 4773 /
 // 15,376 us before, 505 / 1270 / 3530 / 11,030 with four waves, 442 us for the
-// 30,000 with three.  Any-hit queries lose by it (200,000 rays 430 -> 484 us) and
-// keep three.
+// 30,000 with three (by the rule and with waiting candidates' walks standing
+// still 461 / 1183 / 3246 / 10,202).  Any-hit queries lose by it (200,000 rays 430
+// -> 484 us) and keep three.
 constexpr int kObjLdsSmall = 16, kObjLds = 24;
 constexpr int obj_certify(int stack) { return stack == kObjLdsSmall ? 8 : 2; }
 constexpr int obj_waves(int stack) { return stack == kObjLdsSmall ? 4 : 1; }

@@ -342,9 +342,9 @@ struct CoopStack<LdsStack<STACK>> {
 //     RISE_CERTIFY lanes, or an eighth of the busy ones, have one
 //     (closest_step's DEFER).
 // Bound by instruction issue: the kernel's time follows its vector
-// instructions (2.15e9 a launch before, 1.9e9 now at 48 of 64 lanes busy).  On
-// the 1M-triangle, 6.07M-ray cast 3405 -> 2880 us against one claim per refill,
-// certifying and finishing at once, and a node test that branched per child.
+// instructions, 2.03e9 a launch of the 1M-triangle, 6.07M-ray cast with 35 of 64
+// lanes active in one (2.31e9 with one claim per refill, certifying and finishing
+// at once, and a node test that branched per child: 3405 us, 2790 now).
 // Counted queries (COUNT) certify at once; their counts and hits are the same.
 // begin(item, r, s) starts a query, or returns false to skip the item;
 // finish(item, r, s) takes its result.
